@@ -43,7 +43,7 @@ PEAK_FP32_MFMA = 157.3e12     # MI355X dense FP32 matrix, FLOP/s
 PEAK_HBM = 8.0e12             # MI355X HBM3E, B/s
 PEAK_FP32_VALU_UNPACKED = 78.6e12   # FP32 vector FMAs without packed FP32 (half the 157.3 figure)
 PEAK_FP64 = 78.6e12           # MI355X FP64 (vector and matrix), FLOP/s
-KERNEL_KIND = {0: "k_prune_mfma", 1: "k_prune_lane", 2: "k_prune_plain"}
+KERNEL_KIND = {0: "k_prune_mfma", 1: "k_prune_lane", 2: "k_prune_f64"}
 
 
 def log(msg: str):

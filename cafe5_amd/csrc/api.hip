@@ -30,9 +30,9 @@ hipError_t launch_reconstruct(const ReconNode* nodes, int n_nodes, const int* ki
 hipError_t launch_fold(const double* mt64, const float* lf32, double* out64, float* out32, const double* err64,
                        const float* err32, int n_dev, int n_rows, int N, int Np, long long slot_elems,
                        int first_slot, int n, hipStream_t stream);
-hipError_t launch_prune_plain(int nq, int grid, const PruneParams& p, hipStream_t st);
-hipError_t launch_prune_mfma(bool fp64, const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st);
-hipError_t mfma_occupancy(bool fp64, const MfmaShape& s, int* per_cu);
+hipError_t f64_dispatch(const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st, int* per_cu);
+hipError_t launch_prune_mfma(const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st);
+hipError_t mfma_occupancy(const MfmaShape& s, int* per_cu);
 hipError_t f16_dispatch(const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st, int* per_cu);
 hipError_t launch_split_f16(const float* mt32, _Float16* hi, _Float16* lo, int Np, long long slot_elems, int n_slots,
                             hipStream_t st);
@@ -118,11 +118,11 @@ struct BucketHost {
 
 // Device buffers of one evaluation (eager calls or a plan).
 struct EvalBufs {
-    DevBuf node_slot, prior64, prior32, catp, buckets, tiles, ntiles, counters, fb_tiles, fb_count, val,
+    DevBuf node_slot, prior64, prior32, catp, buckets, tiles, ntiles, fb_tiles, fb_count, val,
         flag, lnl, cat, post, fail, total, scratch, root, segs, class_off, fam_list;
     void release_all()
     {
-        DevBuf* all[] = {&node_slot, &prior64, &prior32, &catp, &buckets, &tiles, &ntiles, &counters, &fb_tiles,
+        DevBuf* all[] = {&node_slot, &prior64, &prior32, &catp, &buckets, &tiles, &ntiles, &fb_tiles,
                          &fb_count, &val, &flag, &lnl, &cat, &post, &fail, &total, &scratch, &root, &segs,
                          &class_off, &fam_list};
         for (DevBuf* b : all) b->release();
@@ -366,7 +366,7 @@ int cafe_gpu_create(int device, cafe_gpu_ctx** out)
         cafe_gpu_destroy(ctx);
         return fail(rc, "%s", msg.c_str());
     }
-    ctx->join_ev.assign(3 * (kSideStreams + 1), nullptr);
+    ctx->join_ev.assign(2 * (kSideStreams + 1), nullptr);
     for (auto& e : ctx->join_ev) (void)hipEventCreateWithFlags(&e, hipEventDisableTiming);
     // log-gamma of integers from the host libm: the reference's
     // lgamma cache (probability.cpp:69-75)
@@ -687,29 +687,30 @@ int cafe_gpu_set_error_model(cafe_gpu_ctx* ctx, int n_dev, int n_rows, const dou
 namespace {
 
 // Kernel size class: buckets whose vectors have the same number of 16-row
-// tiles (MFMA paths) or the same PLAIN64 rows per lane (PLAIN64 path).
+// tiles.
 struct KernelClass {
     int nt;              // 16-row tiles of the class's largest vector
-    int nq;              // PLAIN64 rows per lane (row s = lane + 64 q)
     int slot_tiles;      // 16-row tiles of its largest stored (non-root) vector
     MfmaShape s32, s64;  // launch shapes of the FP32 and FP64 MFMA kernels
     MfmaShape s16;       // launch shape of the split-FP16 kernel (BATCHED16)
     MfmaShape r64;       // FP64 recompute of the FP32 pass (a few tiles: latency)
     int lane_rows = 0;   // > 0: the FP32 main pass runs k_prune_lane with this many rows (64-family tiles)
-    bool plain = false;  // PLAIN64, or vectors over 64 tiles (1,024 rows): the main pass is k_prune_plain's (final FP64)
+    bool f64 = false;    // the main pass is k_prune_f64's (final values)
+    long long fams = 0;  // its family-likelihoods
+    bool plain = false;  // PLAIN64, or vectors over 64 tiles (1,024 rows): f64 on every path
     int lane_slots = 0;  // its slot instance
     int lane_per_cu = 0; // its workgroups resident per CU
     int lane_grid_mult = 0;   // workgroups per resident slot (0: default)
-    int fb32 = 1;        // FP32 matrix-core main pass: blocks of 16 families per tile (2: 32-family tiles)
+    int fb = 1;          // matrix-core main pass: blocks of 16 families per tile
     bool tuned = false;  // its shape came from the context's tuning table
     int r16 = 0;         // 16-family tiles its families fill (the recompute lists' capacity)
     int r_begin = 0;     // offset of its FP64 recompute list
     int begin, end;      // its main tiles
     int seg_begin = 0, seg_end = 0;   // its (bucket, point) segments
-    // byte offsets of its global scratch in the main pass, the FP64 and the
-    // PLAIN64 recompute: disjoint, since one class's recompute can run
-    // beside another class's main pass
-    size_t off_main = 0, off_r64 = 0, off_rp = 0;
+    // byte offsets of its global scratch in the main pass and the FP64
+    // recompute: disjoint, since one class's recompute can run beside another
+    // class's main pass
+    size_t off_main = 0, off_r64 = 0;
     int stream = 0;      // side stream of its launches
 };
 
@@ -718,29 +719,18 @@ struct PrunePlan {
     int path = 0, model = 0;
     std::vector<KernelClass> classes;
     std::vector<int> class_counts;   // main tiles per class (+ padding)
-    std::vector<int> plain_off;      // offsets of the one-family PLAIN64 recompute lists
     std::vector<int> main_order;     // main-pass launch order (longest first)
     int light_stream = 0;            // the side stream expected to finish its main-pass work first
-    bool has_plain = false;          // a class runs its main pass on PLAIN64 (reads the FP64 pool)
-    int plain_list_size = 0;
+    bool has_f64 = false;            // a class's main pass reads the FP64 pool
     int n_split = 0;                 // BATCHED16: pool slots converted to FP16 halves before pruning
     int n_tiles = 0, n_segs = 0, maxLR = 0;
     int r16_total = 0;               // capacity of the FP64 recompute lists (16-family tiles)
     int waves_per_cu = 16;           // persistent grid: resident waves per CU
     int n_cu = 256;
-    long long per_wg_plain = 0;
     PruneParams base{};
-    // fb_count layout: [0, n) FP64 recompute tiles per class, [n, 2n) PLAIN64
-    // tiles per class, [2n] / [2n+1] families recomputed in each pass
-    int fam_count_off() const { return 2 * (int)classes.size(); }
-    // workgroups of a launch: resident waves per CU over the machine, no more
-    // than the tiles, and a multiple of 8 (the MFMA kernels give each XCD a
-    // contiguous share of the tiles) when there are at least 8
-    int grid(int w, int max_tiles) const
-    {
-        const int g = std::max(1, std::min(n_cu * waves_per_cu / std::max(1, w), max_tiles));
-        return g >= 8 ? g / 8 * 8 : g;
-    }
+    // fb_count layout: [0, n) FP64 recompute tiles per class, [n] families
+    // recomputed in FP64, [n + 1] those with FP64 values near the subnormal range
+    int fam_count_off() const { return (int)classes.size(); }
     // a lane-kernel launch: as an MFMA launch with partials in LDS
     int grid_lane(int per_cu, int max_tiles, int mult = 0) const
     {
@@ -767,7 +757,7 @@ struct PrunePlan {
 // split the output tiles, NTW per wave, so that W NTW >= nt (one pass; the
 // scaled FP32 kernel needs the whole vector in one pass).  Small vectors run
 // one wave per family tile (throughput), large ones several (latency).
-MfmaShape mfma_shape(int nt, bool fp64)
+MfmaShape mfma_shape(int nt)
 {
     MfmaShape s{1, 1, false, 0};
     if (nt <= 4) s = {std::max(1, nt), 1, false, 0};
@@ -806,38 +796,72 @@ int builtin_fb32(int path, int nt, bool only_mfma_class, long long fam_points, i
     return nt > 16 || (only_mfma_class && fam_points >= 32LL * n_cu) ? 2 : 1;
 }
 
-// FP64 recompute shape: its lists hold a few tiles, so the time is one tile's
-// chain of steps; one or two output tiles per wave (four above 32 tiles) over
-// up to 8 waves (16 above 16 tiles) keep each step's k-loop short, with room
-// for four k-tiles of loads in flight.
-MfmaShape mfma_shape_chain(int nt)
+// Partials of the FP64 kernel: 2 KB per stored tile and family block.
+size_t f64_frag_bytes(const MfmaShape& s, int n_slots, int nt) { return (size_t)n_slots * nt * s.fb * 64 * 32; }
+
+size_t f64_shm(const MfmaShape& s, int n_slots, int nt, int n_leaves)
 {
-    if (nt <= 2) return {std::max(1, nt), 1, false, 0};
-    if (nt <= 4) return {1, 4, false, 0};
-    if (nt <= 8) return {1, 8, false, 0};
-    if (nt <= 16) return {1, 16, false, 0};
-    if (nt <= 32) return {2, 16, false, 0};
-    return {4, 16, false, 0};
+    return (size_t)f64_meta_bytes(s.w, s.fb, n_leaves, s.staged) + (s.lds ? f64_frag_bytes(s, n_slots, nt) : 0);
+}
+
+// FP64 shape (k_prune_f64) for vectors of nt tiles and a list of `tiles`
+// 16-family tiles.  One wave per row tile and 16 families per workgroup, with
+// the partials in LDS, wherever they fit a CU (150 KB): against global partials
+// 3.51 to 4.93 ms per step (160,000 family-likelihoods, 101 rows, 34 taxa) and
+// 9.8 to 13.0 (80,000, 201 rows, 60 taxa).  Two differences, where the list
+// fills the chip:
+//  - up to 5 tiles per vector 32 families, as one wave's matrix loads are then
+//    most of its step: 3.08 -> 2.56 ms (320,000, 61 rows);
+//  - vectors past LDS stream matrices and partials from L2: 2 x 2 blocks per
+//    wave use every load twice, 8.2 -> 6.0 ms (24,000, 401 rows).
+// Short lists of such vectors (the recompute) are one tile's chain of steps:
+// two row tiles in each of 16 waves take all 32 tiles of 501 rows in one pass
+// (search at B = 500: 45.0 -> 43.6 ms).
+MfmaShape f64_shape(int nt, long long tiles, int n_slots, int n_leaves, int n_cu)
+{
+    MfmaShape s{1, 1, true, 0};
+    s.staged = n_leaves <= 512;   // their counts take 32 KB; more stay in memory
+    s.w = std::min(16, nt);
+    s.lds = s.staged && f64_shm(s, n_slots, nt, n_leaves) <= 150 * 1024;
+    if (s.lds && nt <= 5 && tiles >= 16LL * n_cu) {
+        MfmaShape two = s;
+        two.fb = 2;
+        if (f64_shm(two, n_slots, nt, n_leaves) <= 75 * 1024) s = two;
+    } else if (!s.lds && s.staged) {
+        s.ntw = 2;
+        s.fb = tiles >= 4LL * n_cu ? 2 : 1;
+        s.w = std::min(s.fb == 2 ? 8 : 16, (nt + 1) / 2);
+    }
+    s.shm = f64_shm(s, n_slots, nt, n_leaves);
+    return s;
+}
+
+int f64_occupancy(MfmaShape& s)
+{
+    const PruneParams none{};
+    HIP_OR_FAIL(f64_dispatch(s, 0, none, nullptr, &s.per_cu));
+    return CAFE_GPU_OK;
+}
+
+size_t f64_scratch_bytes(const MfmaShape& s, int n_slots, int nt, int grid)
+{
+    return s.lds ? 0 : (size_t)grid * f64_frag_bytes(s, n_slots, nt);
 }
 
 // Dynamic LDS of an MFMA launch without its partials: the bookkeeping and the
 // tile's leaf counts.
-size_t mfma_meta_only(const MfmaShape& s, bool fp64, int n_slots, int n_leaves)
+size_t mfma_meta_only(const MfmaShape& s, int n_slots, int n_leaves)
 {
-    return (size_t)mfma_meta_bytes(n_slots, s.w, !fp64, s.fb) + (size_t)mfma_count_bytes(n_leaves, s.fb);
+    return (size_t)mfma_meta_bytes(n_slots, s.w, s.fb) + (size_t)mfma_count_bytes(n_leaves, s.fb);
 }
 
 // Partial vectors go to LDS when the workgroup's share stays small enough for
-// several workgroups per CU; the rest use the global scratch.  A latency
-// shape (one workgroup per CU is enough: few tiles) may take up to 144 KB of
-// the CU's 160 KB.
-void place_partials(MfmaShape& s, bool fp64, int n_slots, int slot_tiles, int n_leaves, bool latency = false)
+// several workgroups per CU; the rest use the global scratch.
+void place_partials(MfmaShape& s, int n_slots, int slot_tiles, int n_leaves)
 {
-    const size_t meta = mfma_meta_only(s, fp64, n_slots, n_leaves);
-    const size_t frag = (size_t)n_slots * slot_tiles * s.fb * 64 * 4 * (fp64 ? 8 : 4);
-    if (latency)
-        s.lds = (s.w <= 8 || (s.w == 16 && s.ntw == 1)) && meta + frag + 4096 <= 144 * 1024;
-    else if (s.fb > 1)   // two workgroups per CU, or one of 8 waves
+    const size_t meta = mfma_meta_only(s, n_slots, n_leaves);
+    const size_t frag = (size_t)n_slots * slot_tiles * s.fb * 64 * 4 * 4;
+    if (s.fb > 1)   // two workgroups per CU, or one of 8 waves
         s.lds = s.w <= 8 && meta + frag + 4096 <= (s.w >= 8 ? 144 : 76) * 1024;
     else
         s.lds = s.w <= 4 && meta + frag + 4096 <= 64 * 1024 && (meta + frag) / s.w <= 20 * 1024;
@@ -849,7 +873,7 @@ void place_partials(MfmaShape& s, bool fp64, int n_slots, int slot_tiles, int n_
 // matrix-core kernel.
 constexpr int kF16MaxTiles = 32;
 constexpr int kMfmaMaxTiles = 64;     // the matrix-core shapes' largest vectors (1,024 rows)
-constexpr int kPlainMaxRows = 2048;   // k_prune_plain's largest instance: 32 rows per lane
+constexpr int kMaxRows = 2048;        // the largest vectors of any path
 
 // The split-FP16 kernel's partials: per 32-row block and lane three 16-byte
 // B operands (hi, lo, bound).
@@ -873,10 +897,10 @@ size_t f16_scratch_bytes(const MfmaShape& s, int n_slots, int slot_tiles, int gr
 size_t lane_shm(int n_leaves) { return (size_t)n_leaves * 64 * sizeof(int); }
 
 // Global scratch of an MFMA launch (partials not in LDS), bytes.
-size_t mfma_scratch_bytes(const MfmaShape& s, bool fp64, int n_slots, int slot_tiles, int grid)
+size_t mfma_scratch_bytes(const MfmaShape& s, int n_slots, int slot_tiles, int grid)
 {
     if (s.lds) return 0;
-    return (size_t)grid * n_slots * slot_tiles * s.fb * 64 * 4 * (fp64 ? 8 : 4);
+    return (size_t)grid * n_slots * slot_tiles * s.fb * 64 * 4 * 4;
 }
 
 // The tuning entry for a class of a plan whose size classes are plan_classes
@@ -906,22 +930,29 @@ bool tuned_mfma_shape(cafe_gpu_ctx* ctx, int path, const cafe_gpu_ctx::TuneEntry
     const bool f16 = path == CAFE_GPU_PATH_BATCHED16 && e.kernel == 0;
     if (f16 && nt > kF16MaxTiles) return false;
     const bool fp64 = path == CAFE_GPU_PATH_BATCHED64;
-    // 32-family tiles: the FP32 kernel's main pass (BATCHED32, or BATCHED16
-    // classes past the split-FP16 kernel's sizes)
-    if (e.kernel == 2 && (fp64 || nt > kMaxTilesFb2 || (path == CAFE_GPU_PATH_BATCHED16 && nt <= kF16MaxTiles)))
+    // 32-family tiles: the FP64 kernel, and the FP32 kernel's main pass
+    // (BATCHED32, or BATCHED16 classes past the split-FP16 kernel's sizes)
+    if (e.kernel == 2 && !fp64 && (nt > kMaxTilesFb2 || (path == CAFE_GPU_PATH_BATCHED16 && nt <= kF16MaxTiles)))
         return false;
     s = MfmaShape{e.ntw, e.w, e.lds != 0, 0, 0};
     s.fb = e.kernel == 2 ? 2 : 1;
-    if (f16) place_partials16(s, ctx->n_slots_lane, slot_tiles, ctx->n_leaves);
-    else place_partials(s, fp64, ctx->n_slots, slot_tiles, ctx->n_leaves);
-    if (e.lds && !s.lds) return false;   // LDS partials that do not fit
-    if (!e.lds && s.lds) {               // global scratch asked for
-        s.lds = false;
-        s.shm = f16 ? (size_t)f16_meta_bytes(ctx->n_slots_lane, s.w) + (size_t)mfma_count_bytes(ctx->n_leaves)
-                    : mfma_meta_only(s, fp64, ctx->n_slots, ctx->n_leaves);
-    }
+    hipError_t q = hipSuccess;
     const PruneParams none{};
-    const hipError_t q = f16 ? f16_dispatch(s, 0, none, nullptr, &s.per_cu) : mfma_occupancy(fp64, s, &s.per_cu);
+    if (fp64) {
+        s.shm = f64_shm(s, ctx->n_slots, nt, ctx->n_leaves);
+        if (s.shm > 150 * 1024 || ctx->n_leaves > 512) return false;   // LDS partials that do not fit
+        q = f64_dispatch(s, 0, none, nullptr, &s.per_cu);
+    } else {
+        if (f16) place_partials16(s, ctx->n_slots_lane, slot_tiles, ctx->n_leaves);
+        else place_partials(s, ctx->n_slots, slot_tiles, ctx->n_leaves);
+        if (e.lds && !s.lds) return false;   // LDS partials that do not fit
+        if (!e.lds && s.lds) {               // global scratch asked for
+            s.lds = false;
+            s.shm = f16 ? (size_t)f16_meta_bytes(ctx->n_slots_lane, s.w) + (size_t)mfma_count_bytes(ctx->n_leaves)
+                        : mfma_meta_only(s, ctx->n_slots, ctx->n_leaves);
+        }
+        q = f16 ? f16_dispatch(s, 0, none, nullptr, &s.per_cu) : mfma_occupancy(s, &s.per_cu);
+    }
     if (q != hipSuccess || s.per_cu < 1) {
         (void)hipGetLastError();
         return false;   // no such instance, or it does not fit a CU
@@ -946,7 +977,7 @@ int apply_tuning(cafe_gpu_ctx* ctx, int path, KernelClass& kc, unsigned long lon
     }
     MfmaShape s;
     if (!tuned_mfma_shape(ctx, path, *e, kc.nt, kc.slot_tiles, s)) return CAFE_GPU_OK;
-    if ((e->kernel == 2) != (kc.fb32 == 2)) return CAFE_GPU_OK;   // the tiles were cut for the other width
+    if (s.fb != kc.fb) return CAFE_GPU_OK;   // the tiles were cut for another width
     if (path == CAFE_GPU_PATH_BATCHED16 && e->kernel == 0) kc.s16 = s;
     else if (path == CAFE_GPU_PATH_BATCHED64) kc.s64 = s;
     else kc.s32 = s;
@@ -1058,11 +1089,6 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     for (auto& bk : ctx->buckets)
         maxLR = std::max(maxLR, std::max(round_up(bk.B + 1, kTile), round_up(bk.R + 1, kTile)));
     pp.maxLR = maxLR;
-    auto nq_of = [](const BucketHost& bk) {
-        int c = 1;
-        while (c * 64 < std::max(bk.B + 1, bk.R)) c <<= 1;
-        return c;
-    };
     auto nt_of = [](const BucketHost& bk) {   // root rows run 0..R
         return std::max(round_up(bk.B + 1, kTile), round_up(bk.R + 1, kTile)) / kTile;
     };
@@ -1070,11 +1096,19 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     for (int bi = 0; bi < (int)ctx->buckets.size(); ++bi) {
         const BucketHost& bk = ctx->buckets[bi];
         // vectors (sizes 0..B) and root rows (sizes 0..R) up to 2,048 rows:
-        // PLAIN64 covers 32 x 64; the MFMA shapes take up to 64 tiles of 16
-        // and larger vectors run on PLAIN64 in every path
-        if (std::max(bk.B + 1, bk.R + 1) > kPlainMaxRows)
+        // the FP32 and FP16 shapes take up to 64 tiles of 16, larger vectors
+        // run on the FP64 kernel in every path
+        if (std::max(bk.B + 1, bk.R + 1) > kMaxRows)
             return fail(CAFE_GPU_EINVAL, "bucket B=%d R=%d exceeds the sizes this path supports", bk.B, bk.R);
-        bucket_class.push_back({path == CAFE_GPU_PATH_PLAIN64 ? nq_of(bk) : nt_of(bk), bi});
+        // PLAIN64: one class per power of two of 4-tile blocks (the FP64
+        // kernel takes vectors of any length)
+        int key = nt_of(bk);
+        if (path == CAFE_GPU_PATH_PLAIN64) {
+            int pow2 = 4;
+            while (pow2 < key) pow2 <<= 1;
+            key = pow2;
+        }
+        bucket_class.push_back({key, bi});
     }
     // heavy classes (and, within a class, larger buckets) first
     std::stable_sort(bucket_class.begin(), bucket_class.end(), [&](const std::pair<int, int>& x,
@@ -1101,33 +1135,40 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     for (const auto& kr : key_rows)
         if (lane_rows_of(kr.first) == 0) ++n_mfma_keys;
     std::map<int, long long> key_fams;
-    for (auto& bc : bucket_class) key_fams[bc.first] += (long long)ctx->buckets[bc.second].count * n_points;
+    std::map<int, int> key_nt;   // and the tiles of its largest vector
+    for (auto& bc : bucket_class) {
+        key_fams[bc.first] += (long long)ctx->buckets[bc.second].count * n_points;
+        key_nt[bc.first] = std::max(key_nt[bc.first], nt_of(ctx->buckets[bc.second]));
+    }
     // the plan's size classes, for the tuning entries measured in a plan
     unsigned long long plan_classes = 0;
     for (const auto& kr : key_rows)
         if (kr.first >= 1 && kr.first <= 64) plan_classes |= 1ull << (kr.first - 1);
     std::vector<TileDesc> tiles;
     std::vector<SegDesc> segs;
-    std::vector<int> cls_fams;
     int prev_key = -1;
     for (auto& bc : bucket_class) {
         const BucketHost& bk = ctx->buckets[bc.second];
         if (pp.classes.empty() || bc.first != prev_key) {
             KernelClass kc{};
             kc.begin = kc.end = (int)tiles.size();
+            kc.fams = key_fams[bc.first];
             kc.seg_begin = kc.seg_end = (int)segs.size();
             // the kernel is chosen here: its tiles carry 64 families (per
             // lane) or 16 (matrix cores)
             kc.plain = path == CAFE_GPU_PATH_PLAIN64 || bc.first > kMfmaMaxTiles;
+            kc.f64 = kc.plain || path == CAFE_GPU_PATH_BATCHED64;
             kc.lane_rows = kc.plain ? 0 : lane_rows_of(bc.first);
-            kc.fb32 = kc.lane_rows > 0 || kc.plain
-                          ? 1
-                          : builtin_fb32(path, bc.first, n_mfma_keys == 1, key_fams[bc.first], ctx->n_cu);
+            if (kc.f64)
+                kc.fb = f64_shape(key_nt[bc.first], kc.fams / kTile, ctx->n_slots, ctx->n_leaves, ctx->n_cu).fb;
+            kc.fb = kc.lane_rows > 0 ? 1
+                  : kc.f64           ? kc.fb
+                                     : builtin_fb32(path, bc.first, n_mfma_keys == 1, key_fams[bc.first], ctx->n_cu);
             if (const cafe_gpu_ctx::TuneEntry* te = kc.plain ? nullptr : find_tuning(ctx, path, bc.first, plan_classes)) {
                 MfmaShape probe;
                 if (tuned_mfma_shape(ctx, path, *te, bc.first, bc.first, probe)) {
                     kc.lane_rows = 0;
-                    kc.fb32 = probe.fb;
+                    kc.fb = probe.fb;
                 }
             }
             if (kc.lane_rows > 0) {
@@ -1138,15 +1179,13 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
                 if (kc.lane_per_cu == 0) kc.lane_rows = 0;   // no instance fits: matrix-core kernel
             }
             pp.classes.push_back(kc);
-            cls_fams.push_back(0);
             prev_key = bc.first;
         }
         KernelClass& kc = pp.classes.back();
         const int ci = (int)pp.classes.size() - 1;
         kc.nt = std::max(kc.nt, nt_of(bk));
-        kc.nq = std::max(kc.nq, nq_of(bk));
         kc.slot_tiles = std::max(kc.slot_tiles, round_up(bk.B + 1, kTile) / kTile);
-        const int tw = kc.lane_rows > 0 ? 64 : kTile * kc.fb32;   // families per tile
+        const int tw = kc.lane_rows > 0 ? 64 : kTile * kc.fb;   // families per tile
         for (int pi = 0; pi < n_points; ++pi) {
             for (int f0 = 0; f0 < bk.count; f0 += tw)
                 tiles.push_back(TileDesc{bc.second, point_ids[pi], f0, std::min(tw, bk.count - f0)});
@@ -1154,29 +1193,26 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
                 segs.push_back(SegDesc{bc.second, point_ids[pi], ci, f0});
         }
         kc.r16 += n_points * ((bk.count + kTile - 1) / kTile);
-        cls_fams[ci] += bk.count * n_points;
         kc.end = (int)tiles.size();
         kc.seg_end = (int)segs.size();
     }
     const int n_cls = (int)pp.classes.size();
     for (auto& kc : pp.classes) {
-        if (kc.plain) {
-            pp.has_plain = true;
+        if (kc.f64) {
+            pp.has_f64 = true;
+            kc.s64 = f64_shape(kc.nt, kc.fams / kTile, ctx->n_slots, ctx->n_leaves, ctx->n_cu);
+            if (int rc = f64_occupancy(kc.s64)) return rc;
             continue;
         }
-        kc.s32 = kc.fb32 == 2 ? mfma_shape_fb2(kc.nt) : mfma_shape(kc.nt, false);
-        kc.s64 = mfma_shape(kc.nt, true);
-        kc.r64 = mfma_shape_chain(kc.nt);
-        place_partials(kc.s32, false, ctx->n_slots, kc.slot_tiles, ctx->n_leaves);
-        place_partials(kc.s64, true, ctx->n_slots, kc.slot_tiles, ctx->n_leaves);
-        place_partials(kc.r64, true, ctx->n_slots, kc.slot_tiles, ctx->n_leaves, true);
-        HIP_OR_FAIL(mfma_occupancy(false, kc.s32, &kc.s32.per_cu));
-        HIP_OR_FAIL(mfma_occupancy(true, kc.s64, &kc.s64.per_cu));
-        HIP_OR_FAIL(mfma_occupancy(true, kc.r64, &kc.r64.per_cu));
+        kc.s32 = kc.fb == 2 ? mfma_shape_fb2(kc.nt) : mfma_shape(kc.nt);
+        kc.r64 = f64_shape(kc.nt, 1, ctx->n_slots, ctx->n_leaves, ctx->n_cu);
+        place_partials(kc.s32, ctx->n_slots, kc.slot_tiles, ctx->n_leaves);
+        HIP_OR_FAIL(mfma_occupancy(kc.s32, &kc.s32.per_cu));
+        if (int rc = f64_occupancy(kc.r64)) return rc;
         if (path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles) {
             // the program whose outputs reuse a child's slot (the store's
             // maxima exchange orders all reads before the writes)
-            kc.s16 = mfma_shape(kc.nt, false);
+            kc.s16 = mfma_shape(kc.nt);
             place_partials16(kc.s16, ctx->n_slots_lane, kc.slot_tiles, ctx->n_leaves);
             const PruneParams none{};
             HIP_OR_FAIL(f16_dispatch(kc.s16, 0, none, nullptr, &kc.s16.per_cu));
@@ -1185,11 +1221,6 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
                 kc.s16.shm = (size_t)f16_meta_bytes(ctx->n_slots_lane, kc.s16.w) + (size_t)mfma_count_bytes(ctx->n_leaves);
                 HIP_OR_FAIL(f16_dispatch(kc.s16, 0, none, nullptr, &kc.s16.per_cu));
             }
-        }
-        if (kc.r64.per_cu == 0 && kc.r64.lds) {   // the device does not fit that much LDS: global scratch
-            kc.r64.lds = false;
-            kc.r64.shm = mfma_meta_only(kc.r64, true, ctx->n_slots, ctx->n_leaves);
-            HIP_OR_FAIL(mfma_occupancy(true, kc.r64, &kc.r64.per_cu));
         }
     }
     // Measured shapes from the context's tuning table replace the built-in
@@ -1235,26 +1266,21 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     pp.class_counts.assign(n_cls + 4, 0);
     for (int i = 0; i < n_cls; ++i) pp.class_counts[i] = pp.classes[i].end - pp.classes[i].begin;
     // [0, n_cls] offsets of the 16-family recompute lists (room for all of a
-    // class's families in 16-family tiles), [n_cls + 1, 2 n_cls + 1] of the
-    // one-family PLAIN64 lists
-    std::vector<int> class_off(2 * (n_cls + 1), 0);
+    // class's families in 16-family tiles)
+    std::vector<int> class_off(n_cls + 1, 0);
     for (int i = 0; i < n_cls; ++i) {
         pp.classes[i].r_begin = class_off[i];
         class_off[i + 1] = class_off[i] + pp.classes[i].r16;
     }
     pp.r16_total = class_off[n_cls];
-    for (int i = 0; i < n_cls; ++i) class_off[n_cls + 1 + i + 1] = class_off[n_cls + 1 + i] + cls_fams[i];
-    pp.plain_list_size = class_off[2 * n_cls + 1];
-    pp.plain_off.assign(class_off.begin() + n_cls + 1, class_off.end());
     pp.n_segs = (int)segs.size();
 
     HIP_OR_FAIL(b.tiles.ensure(sizeof(TileDesc) * std::max(1, pp.n_tiles)));
-    HIP_OR_FAIL(b.fb_tiles.ensure(sizeof(TileDesc) * ((size_t)std::max(1, pp.r16_total) + std::max(1, pp.plain_list_size))));
+    HIP_OR_FAIL(b.fb_tiles.ensure(sizeof(TileDesc) * (size_t)std::max(1, pp.r16_total)));
     HIP_OR_FAIL(b.ntiles.ensure(sizeof(int) * (n_cls + 4)));
-    HIP_OR_FAIL(b.counters.ensure(sizeof(int) * (3 * n_cls + 8)));
-    HIP_OR_FAIL(b.fb_count.ensure(sizeof(int) * (2 * n_cls + 4)));
+    HIP_OR_FAIL(b.fb_count.ensure(sizeof(int) * (n_cls + 2)));
     HIP_OR_FAIL(b.segs.ensure(sizeof(SegDesc) * std::max(1, pp.n_segs)));
-    HIP_OR_FAIL(b.class_off.ensure(sizeof(int) * 2 * (n_cls + 1)));
+    HIP_OR_FAIL(b.class_off.ensure(sizeof(int) * (n_cls + 1)));
     {
         size_t maxp = 0;
         for (int i = 0; i < n_points; ++i) maxp = std::max(maxp, (size_t)point_ids[i] + 1);
@@ -1264,44 +1290,28 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     HIP_OR_FAIL(hipMemcpy(b.ntiles.p, pp.class_counts.data(), sizeof(int) * pp.class_counts.size(),
                           hipMemcpyHostToDevice));
     HIP_OR_FAIL(hipMemcpy(b.segs.p, segs.data(), sizeof(SegDesc) * pp.n_segs, hipMemcpyHostToDevice));
-    HIP_OR_FAIL(hipMemcpy(b.class_off.p, class_off.data(), sizeof(int) * 2 * (n_cls + 1), hipMemcpyHostToDevice));
+    HIP_OR_FAIL(hipMemcpy(b.class_off.p, class_off.data(), sizeof(int) * (n_cls + 1), hipMemcpyHostToDevice));
 
     // Global scratch: per class and pass (classes of one pass run
-    // concurrently, passes one after another).  PLAIN64 partials take one
-    // region of n_slots x ldv doubles per workgroup unless they fit in LDS.
-    const int ldv = round_up(maxLR, 4) + 4;
-    pp.per_wg_plain = (long long)ctx->n_slots * ldv;
-    const bool plain_in_lds = sizeof(double) * (size_t)ctx->n_slots * ldv <= 48 * 1024;
-    auto plain_bytes = [&](int n) {
-        return plain_in_lds || n <= 0 ? (size_t)0 : (size_t)pp.grid(1, n) * 8 * (size_t)pp.per_wg_plain;
-    };
-    size_t main_sz = 0, r64_sz = 0, rp_sz = 0;
+    // concurrently, passes one after another).
+    size_t main_sz = 0, r64_sz = 0;
     for (int ci = 0; ci < n_cls; ++ci) {
         KernelClass& kc = pp.classes[ci];
         const int n = pp.class_counts[ci];
         size_t mb = 0;
-        if (kc.plain) mb = plain_bytes(n);
-        else if (path == CAFE_GPU_PATH_BATCHED64)
-            mb = mfma_scratch_bytes(kc.s64, true, ctx->n_slots, kc.slot_tiles, pp.grid(kc.s64, n));
+        if (kc.f64) mb = f64_scratch_bytes(kc.s64, ctx->n_slots, kc.nt, pp.grid(kc.s64, n));
         else if (kc.lane_rows > 0) mb = 0;
         else if (path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles) mb = f16_scratch_bytes(kc.s16, ctx->n_slots_lane, kc.slot_tiles, pp.grid(kc.s16, n));
-        else mb = mfma_scratch_bytes(kc.s32, false, ctx->n_slots, kc.slot_tiles, pp.grid(kc.s32, n));
+        else mb = mfma_scratch_bytes(kc.s32, ctx->n_slots, kc.slot_tiles, pp.grid(kc.s32, n));
         kc.off_main = main_sz;
         main_sz += align256(mb);
-        if ((path == CAFE_GPU_PATH_BATCHED32 || path == CAFE_GPU_PATH_BATCHED16) && !kc.plain) {
+        if (!kc.f64) {
             kc.off_r64 = r64_sz;
-            r64_sz += align256(mfma_scratch_bytes(kc.r64, true, ctx->n_slots, kc.slot_tiles, pp.grid(kc.r64, kc.r16)));
-        }
-        if (path != CAFE_GPU_PATH_PLAIN64 && !kc.plain) {
-            kc.off_rp = rp_sz;
-            rp_sz += align256(plain_bytes(pp.plain_off[ci + 1] - pp.plain_off[ci]));
+            r64_sz += align256(f64_scratch_bytes(kc.r64, ctx->n_slots, kc.nt, pp.grid(kc.r64, kc.r16)));
         }
     }
-    for (auto& kc : pp.classes) {
-        kc.off_r64 += main_sz;
-        kc.off_rp += main_sz + r64_sz;
-    }
-    HIP_OR_FAIL(b.scratch.ensure(std::max<size_t>(main_sz + r64_sz + rp_sz, 256)));
+    for (auto& kc : pp.classes) kc.off_r64 += main_sz;
+    HIP_OR_FAIL(b.scratch.ensure(std::max<size_t>(main_sz + r64_sz, 256)));
 
     PruneParams& p = pp.base;
     p.buckets = b.buckets.as<BucketDev>();
@@ -1347,16 +1357,14 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     p.mt16h = ctx->mt16h.as<_Float16>();
     p.mt16l = ctx->mt16l.as<_Float16>();
     p.scratch = b.scratch.p;
-    p.ldv = ldv;
     p.n_slots = ctx->n_slots;
     p.zero = 0;
     return CAFE_GPU_OK;
 }
 
 // Enqueues the pruning sequence: the main path per size class, then
-// (device-side lists, no host round trip) the FP64 recompute of the FP32
-// families the flush bound did not certify and the PLAIN64 recompute of
-// families near the subnormal range.  late_build (when set) enqueues the
+// (device-side lists, no host round trip) the FP64 recompute of the families
+// a reduced path's bound did not certify.  late_build (when set) enqueues the
 // FP64 pool, which only the recompute stages read: it runs on the side stream
 // expected to finish its main-pass work first, after that work.
 int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream_t st, hipEvent_t ev_main,
@@ -1365,23 +1373,18 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
 {
     const int n_cls = (int)pp.classes.size();
     int* d_cnt = b.ntiles.as<int>();
-    int* d_ctr = b.counters.as<int>();
     int* fbc = b.fb_count.as<int>();
     char* scratch = (char*)pp.base.scratch;
-    HIP_OR_FAIL(launch_fill_zero(b.counters.p, sizeof(int) * (3 * n_cls + 8), st));
-    HIP_OR_FAIL(launch_fill_zero(b.fb_count.p, sizeof(int) * (2 * n_cls + 4), st));
+    HIP_OR_FAIL(launch_fill_zero(b.fb_count.p, sizeof(int) * (n_cls + 2), st));
     // BATCHED16 reads the FP16 halves of the FP32 matrices
     if (pp.path == CAFE_GPU_PATH_BATCHED16)
         HIP_OR_FAIL(launch_split_f16(ctx->mt32.as<float>(), ctx->mt16h.as<_Float16>(), ctx->mt16l.as<_Float16>(),
                                      ctx->Np, ctx->slot_elems, pp.n_split, st));
 
-    // Three stages per size class: the main pass, then (BATCHED32) the FP64
-    // recompute of the families the FP32 bound did not certify, then
-    // (BATCHED32/64) the PLAIN64 recompute of those near the subnormal range.
-    // Each recompute stage packs its class's flagged families into a list
-    // sized on the device and prunes it.
+    // Two stages per size class: the main pass, then (reduced paths) the FP64
+    // recompute of the families the bound did not certify, which packs its
+    // class's flagged families into a list sized on the device and prunes it.
     TileDesc* fb64 = b.fb_tiles.as<TileDesc>();
-    TileDesc* fbplain = fb64 + std::max(1, pp.r16_total);
     const int* coff = b.class_off.as<int>();
     const int fam_off = pp.fam_count_off();
     const SegDesc* segs = b.segs.as<SegDesc>();
@@ -1391,14 +1394,12 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
         PruneParams q = pp.base;
         q.tiles = b.tiles.as<TileDesc>() + kc.begin;
         q.n_tiles_dev = d_cnt + ci;
-        q.tile_counter = d_ctr + ci;
         q.slot_tiles = kc.slot_tiles;
         q.scratch = scratch + kc.off_main;
-        if (kc.plain) {   // final FP64 values: nothing to recompute
-            q.scratch_per_wg = pp.per_wg_plain;
-            HIP_OR_FAIL(launch_prune_plain(kc.nq, pp.grid(1, n), q, s));
-        } else if (pp.path == CAFE_GPU_PATH_BATCHED64) {
-            HIP_OR_FAIL(launch_prune_mfma(true, kc.s64, pp.grid(kc.s64, n), q, s));
+        if (kc.f64) {   // final FP64 values: nothing to recompute
+            q.slot_tiles = kc.nt;
+            if (!kc.plain) q.near_floor = fbc + fam_off + 1;
+            HIP_OR_FAIL(f64_dispatch(kc.s64, pp.grid(kc.s64, n), q, s, nullptr));
         } else if (kc.lane_rows > 0) {   // BATCHED32 / BATCHED16: small vectors, one family per lane
             q.steps = ctx->d_steps_hot.as<StepDev>();
             q.n_slots = ctx->n_slots_hot;
@@ -1409,46 +1410,28 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
             q.n_slots = ctx->n_slots_lane;
             HIP_OR_FAIL(f16_dispatch(kc.s16, pp.grid(kc.s16, n), q, s, nullptr));
         } else {
-            HIP_OR_FAIL(launch_prune_mfma(false, kc.s32, pp.grid(kc.s32, n), q, s));
+            HIP_OR_FAIL(launch_prune_mfma(kc.s32, pp.grid(kc.s32, n), q, s));
         }
         return CAFE_GPU_OK;
     };
     auto stage_r64 = [&](int ci, hipStream_t s) -> int {
-        if (pp.path != CAFE_GPU_PATH_BATCHED32 && pp.path != CAFE_GPU_PATH_BATCHED16) return CAFE_GPU_OK;
         const KernelClass& kc = pp.classes[ci];
-        if (kc.plain) return CAFE_GPU_OK;
+        if (kc.f64) return CAFE_GPU_OK;
         HIP_OR_FAIL(launch_pack(segs + kc.seg_begin, kc.seg_end - kc.seg_begin, b.buckets.as<BucketDev>(),
                                 pp.base.perm, b.flag.as<int>(), pp.base.F, kFlagRecompute64, b.fam_list.as<int>(),
                                 fb64, coff, fbc, fbc + fam_off, kTile, s));
         PruneParams q = pp.base;
         q.tiles = fb64 + kc.r_begin;
         q.n_tiles_dev = fbc + ci;
-        q.tile_counter = d_ctr + n_cls + ci;
-        q.slot_tiles = kc.slot_tiles;
+        q.slot_tiles = kc.nt;
         q.scratch = scratch + kc.off_r64;
-        HIP_OR_FAIL(launch_prune_mfma(true, kc.r64, pp.grid(kc.r64, kc.r16), q, s));
-        return CAFE_GPU_OK;
-    };
-    auto stage_plain = [&](int ci, hipStream_t s) -> int {
-        if (pp.path == CAFE_GPU_PATH_PLAIN64) return CAFE_GPU_OK;
-        const KernelClass& kc = pp.classes[ci];
-        if (kc.plain) return CAFE_GPU_OK;
-        HIP_OR_FAIL(launch_pack(segs + kc.seg_begin, kc.seg_end - kc.seg_begin, b.buckets.as<BucketDev>(),
-                                pp.base.perm, b.flag.as<int>(), pp.base.F, kFlagRecomputePlain,
-                                b.fam_list.as<int>(), fbplain, coff + n_cls + 1, fbc + n_cls, fbc + fam_off + 1, 1,
-                                s));
-        PruneParams q = pp.base;
-        q.tiles = fbplain + pp.plain_off[ci];
-        q.n_tiles_dev = fbc + n_cls + ci;
-        q.tile_counter = d_ctr + 2 * n_cls + ci;
-        q.scratch = scratch + kc.off_rp;
-        q.scratch_per_wg = pp.per_wg_plain;
-        HIP_OR_FAIL(launch_prune_plain(kc.nq, pp.grid(1, pp.plain_off[ci + 1] - pp.plain_off[ci]), q, s));
+        q.near_floor = fbc + fam_off + 1;
+        HIP_OR_FAIL(f64_dispatch(kc.r64, pp.grid(kc.r64, kc.r16), q, s, nullptr));
         return CAFE_GPU_OK;
     };
 
     // Stage by stage over the classes: every main pass, then every FP64
-    // recompute followed on the same stream by the class's PLAIN64 recompute.
+    // recompute.
     // When concurrent, the classes of one stage run on the side streams (the
     // main passes on their longest-first assignment, the recomputes round
     // robin in that order: measured 1.5% faster per step than placing the
@@ -1458,20 +1441,14 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
     const int S = concurrent ? std::min((int)ctx->side.size(), n_cls) : 0;
     if (late_build && S <= 1)
         if (int rc = (*late_build)(st)) return rc;
-    // launch2 (may be null) follows every launch of the stage on the same
-    // streams, before the join: the PLAIN64 pass of a class reads only the
-    // flags its own main pass and FP64 pass wrote, on the same stream
     using Launch = std::function<int(int, hipStream_t)>;
-    auto stage = [&](int idx, const Launch& launch, const Launch* launch2 = nullptr) -> int {
+    auto stage = [&](int idx, const Launch& launch) -> int {
         if (S <= 1) {
             for (int ci = 0; ci < n_cls; ++ci) {
                 if (cls_ev && idx == 0) HIP_OR_FAIL(hipEventRecord((*cls_ev)[ci], st));
                 if (int rc = launch(ci, st)) return rc;
             }
             if (cls_ev && idx == 0) HIP_OR_FAIL(hipEventRecord((*cls_ev)[n_cls], st));
-            if (launch2)
-                for (int ci = 0; ci < n_cls; ++ci)
-                    if (int rc = (*launch2)(ci, st)) return rc;
             return CAFE_GPU_OK;
         }
         hipEvent_t* ev = ctx->join_ev.data() + idx * (kSideStreams + 1);
@@ -1482,9 +1459,6 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
             const int k = idx == 0 ? pp.classes[ci].stream % S : i % S;
             if (int rc = launch(ci, ctx->side[k])) return rc;
         }
-        if (launch2)
-            for (int i = 0; i < n_cls; ++i)
-                if (int rc = (*launch2)(pp.main_order[i], ctx->side[i % S])) return rc;
         if (idx == 0 && late_build)
             if (int rc = (*late_build)(ctx->side[pp.light_stream % S])) return rc;
         for (int k = 0; k < S; ++k) {
@@ -1495,12 +1469,8 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
     };
     if (int rc = stage(0, stage_main)) return rc;
     if (ev_main) HIP_OR_FAIL(hipEventRecord(ev_main, st));
-    const Launch plain = stage_plain;
-    if (pp.path == CAFE_GPU_PATH_BATCHED32 || pp.path == CAFE_GPU_PATH_BATCHED16) {
-        if (int rc = stage(1, stage_r64, &plain)) return rc;
-    } else if (pp.path != CAFE_GPU_PATH_PLAIN64) {
-        if (int rc = stage(2, stage_plain)) return rc;
-    }
+    if (pp.path == CAFE_GPU_PATH_BATCHED32 || pp.path == CAFE_GPU_PATH_BATCHED16)
+        if (int rc = stage(1, stage_r64)) return rc;
     if (ev_fb) HIP_OR_FAIL(hipEventRecord(ev_fb, st));
     return CAFE_GPU_OK;
 }
@@ -1701,7 +1671,7 @@ int plan_enqueue(cafe_gpu_plan* pl, bool timed)
     // BATCHED32 reads the FP64 pool only in its recompute stages: concurrent
     // runs with the recurrence build make the FP32 pools first and the FP64
     // one beside the main pass
-    const bool split = !timed && pl->algo != 0 && !pl->pp.has_plain &&
+    const bool split = !timed && pl->algo != 0 && !pl->pp.has_f64 &&
                        (pl->pp.path == CAFE_GPU_PATH_BATCHED32 || pl->pp.path == CAFE_GPU_PATH_BATCHED16);
     if (timed) HIP_OR_FAIL(hipEventRecord(pl->ev[0], st));
     HIP_OR_FAIL(launch_build(pl->algo, pl->d_lam.as<double>(), pl->d_t.as<double>(), ctx->lg.as<double>(), pl->n_keys,
@@ -2084,13 +2054,13 @@ int cafe_gpu_plan_class_times(cafe_gpu_plan* pl, int cap, int* n_classes, int* c
             const KernelClass& kc = pl->pp.classes[i];
             const int n = pl->pp.class_counts[i];
             int* l = launch + 6 * i;
-            if (kc.plain) {
-                l[0] = 2;
-                l[1] = kc.nq;
-                l[2] = 1;
-                l[3] = 0;
-                l[4] = pl->pp.grid(1, n);
-                l[5] = 1;
+            if (kc.f64) {
+                l[0] = kc.plain ? 2 : 0;
+                l[1] = kc.s64.ntw;
+                l[2] = kc.s64.w;
+                l[3] = kc.s64.lds ? 1 : 0;
+                l[4] = pl->pp.grid(kc.s64, n);
+                l[5] = kTile * kc.s64.fb;
             } else if ((pl->path == CAFE_GPU_PATH_BATCHED32 || pl->path == CAFE_GPU_PATH_BATCHED16) &&
                        kc.lane_rows > 0) {
                 l[0] = 1;
@@ -2101,7 +2071,7 @@ int cafe_gpu_plan_class_times(cafe_gpu_plan* pl, int cap, int* n_classes, int* c
                 l[5] = 64;
             } else {
                 const bool f16 = pl->path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles;
-                const MfmaShape& sh = pl->path == CAFE_GPU_PATH_BATCHED64 ? kc.s64 : f16 ? kc.s16 : kc.s32;
+                const MfmaShape& sh = f16 ? kc.s16 : kc.s32;
                 l[0] = f16 ? 3 : 0;
                 l[1] = sh.ntw;
                 l[2] = sh.w;

@@ -104,15 +104,13 @@ enum : int {
 // Output flags per (point, family).
 enum : int {
     kFlagZeroSum = 1,     // root vector sums to 0 (gamma_core.cpp:151-152)
-    kFlagRecompute64 = 2, // FP32 result not certified: recompute on BATCHED64
-    kFlagRecomputePlain = 4  // FP64 value near the subnormal range: recompute on PLAIN64
+    kFlagRecompute64 = 2  // reduced-precision result not certified: recompute in FP64
 };
 
 struct PruneParams {
     // work list
     const TileDesc* tiles;
     const int* n_tiles_dev;   // number of tiles (device-resident count)
-    int* tile_counter;        // persistent-kernel work counter (zeroed before launch)
     // model
     const BucketDev* buckets;
     const OpDev* ops;
@@ -156,14 +154,12 @@ struct PruneParams {
     const _Float16* mt16h;
     const _Float16* mt16l;
     int vec_exp16;
-    // partial-vector scratch: per workgroup n_slots x 16 x ldv values
+    // partial-vector scratch, a region of n_slots vectors per workgroup
     void* scratch;
-    long long scratch_per_wg;  // elements
-    int ldv;
     int n_slots;
     int slot_tiles;           // MFMA: 16-row tiles per stored partial vector
     int zero;                 // always 0 (an offset the compiler cannot fold)
-    int plain_lds;            // PLAIN64: partial vectors in dynamic LDS
+    int* near_floor;          // FP64: counts the families with values below kFp64Floor (null: not counted)
     // nonzero band of the FP32 row-major pool: per slot and 16-row tile t,
     // band[slot * band_stride + t] = lo | hi << 16, the k-tiles [lo, hi)
     // outside of which the tile's entries are exactly 0 (null: no band)
@@ -190,16 +186,16 @@ struct MfmaShape {
     size_t shm;
     int per_cu;          // workgroups resident on one CU (registers and LDS)
     int grid_mult = 0;   // workgroups per resident slot (0: the planner's default)
-    int fb = 1;          // blocks of 16 families per tile (2: FP32 only)
+    int fb = 1;          // blocks of 16 families per tile (4: FP64 only)
+    bool staged = true;      // FP64: a tile's leaf counts in LDS
 };
 
 // Dynamic-LDS bookkeeping of the scaled FP32 kernel for n_slots partial
 // vectors, w waves and fb blocks of 16 families: per slot a flush bound
 // (double), an exponent and a renormalisation shift (int) per family, per-wave
 // maxima (float) per family, and one nominal-scale exponent.
-__host__ __device__ inline int mfma_meta_bytes(int n_slots, int w, bool scaled, int fb = 1)
+__host__ __device__ inline int mfma_meta_bytes(int n_slots, int w, int fb = 1)
 {
-    if (!scaled) return 0;
     const int fw = 16 * fb;
     const int b = n_slots * fw * 8 + n_slots * w * fw * 4 + 2 * n_slots * fw * 4 + n_slots * 4;
     return (b + 31) & ~31;
@@ -210,6 +206,14 @@ __host__ __device__ inline int mfma_meta_bytes(int n_slots, int w, bool scaled, 
 __host__ __device__ inline int f16_meta_bytes(int n_slots, int w)
 {
     const int b = w * 16 * 4 + n_slots * 16 * 4;
+    return (b + 31) & ~31;
+}
+
+// Dynamic LDS of the FP64 kernel besides its partials: two maxima (double) per
+// wave and family, and the tile's leaf counts where they are staged.
+__host__ __device__ inline int f64_meta_bytes(int w, int fb, int n_leaves, bool staged)
+{
+    const int b = w * 16 * fb * 16 + (staged ? n_leaves * 16 * fb * 4 : 0);
     return (b + 31) & ~31;
 }
 

@@ -1,0 +1,423 @@
+// prune_f64.hip -- FP64 pruning on the matrix cores, in the reference's
+// summation order (inference_prune / compute_node_probability,
+// src/core.cpp:134-145, src/probability.cpp:175-330): the PLAIN64 and BATCHED64
+// paths and the FP64 recompute of the reduced paths.
+//
+// v_mfma_f64_16x16x4f64 adds its four products to the accumulator one after
+// another, each as a fused multiply-add, in ascending k (checked bit for bit
+// against a chain of fma() on the device, subnormal values included).  MFMA j
+// of k-tile kt contracts the sizes x = 16 kt + 4 j + g of lane group g, so
+// every sum runs over x = 0, 1, 2, ... as matrix::multiply's does
+// (matrix_cache.cpp:50-56), and a node's factors multiply in the children's
+// order (probability.cpp:208-217, 222-231).
+//
+// Lane l = 16 g + f of a wave holds, for 16-row tile t of a vector, the sizes
+// 16 t + 4 r + g (r = 0..3) of family f: the D layout of the instruction, and
+// the B layout of the next contraction, so a node's output is its parent's
+// input as stored.  A workgroup of W waves carries FB blocks of 16 families of
+// one bucket at one parameter point through the tree; a wave takes chunks of
+// NTW row tiles (chunk = wave, wave + W, ...), and each matrix fragment it loads
+// feeds the MFMAs of all FB blocks.
+//
+// What bounds it: an FP64 MFMA takes a SIMD's FP64 unit for 64 cycles, so the
+// steps' address arithmetic is kept on the scalar side; at 201 rows a step is
+// 13,300 cycles of MFMAs on the SIMD with four of the thirteen waves and about
+// 7,000 of barrier and step start.  10,000 families of 34 taxa at bound 200
+// take 0.96 ms (27 TF/s of 71 the library's products reach), against 37.2 ms
+// one family per wave with the lanes over rows; 250 families of 12 taxa 0.06
+// against 2.2 ms.
+#include "prune_common.h"
+
+namespace cafe {
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+// A key this far (relatively) below the best product cannot be the best key:
+// the logarithms' rounding is 1e-13 at most over FP64's range.
+constexpr double kNearBest = 1.0 - 1e-9;
+
+// Most waves of a workgroup: sixteen leave 128 VGPRs per wave, eight 256.
+template <int NTW, int FB> struct F64Waves { static constexpr int v = NTW * FB > 2 || FB > 1 ? 8 : 16; };
+
+// q, kept as a scalar base: the compiler would otherwise fold the lane offset
+// into per-lane 64-bit addresses, and an FP64 matrix instruction holds the
+// SIMD's vector unit for its 64 cycles, so every vector instruction beside
+// the matrix ones waits for one of another wave.
+typedef const __attribute__((address_space(1))) double* Gptr;
+__device__ __forceinline__ Gptr uniform(const double* q)
+{
+    Gptr r = (Gptr)q;
+    asm("" : "+s"(r));
+    return r;
+}
+
+// *(q + byte offset): one 32-bit lane offset serves all loads (hidden here, or
+// its 64-bit form would be kept across the loop).
+__device__ __forceinline__ double at(Gptr q, unsigned off)
+{
+    asm volatile("" : "+v"(off));
+    return *(Gptr)((const __attribute__((address_space(1))) char*)q + off);
+}
+
+// Partial vectors in LDS or in global scratch (typed by address space: a
+// generic pointer would make their accesses flat ones).
+template <bool LDSP> struct Partials { typedef __attribute__((address_space(1))) d4* ptr; };
+template <> struct Partials<true> { typedef __attribute__((address_space(3))) d4* ptr; };
+
+template <int NTW, int FB, bool LDSP, bool STAGED>
+__global__ __launch_bounds__((64 * F64Waves<NTW, FB>::v)) void k_prune_f64(PruneParams p)
+{
+    constexpr int FW = 16 * FB;   // families per tile
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int W = __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6));
+    const int fl = lane & 15;
+    const int g = lane >> 4;
+    const int Np = p.Np;
+    const int slot_tiles = p.slot_tiles;
+    extern __shared__ __align__(32) unsigned char s_dyn[];
+    typedef __attribute__((address_space(3))) unsigned char* Lds;
+    const Lds lds = (Lds)s_dyn;
+    __attribute__((address_space(3))) double* s_a = (__attribute__((address_space(3))) double*)lds;   // [W][FW] per-wave maxima
+    __attribute__((address_space(3))) double* s_b = s_a + W * FW;                                     // [W][FW]
+    // [leaf][FW] byte offsets of the tile's leaf columns (where they fit)
+    __attribute__((address_space(3))) unsigned* s_cnt = (__attribute__((address_space(3))) unsigned*)(s_b + W * FW);
+    typedef typename Partials<LDSP>::ptr Frag;
+    Frag frag;
+    if constexpr (LDSP) frag = (Frag)(lds + f64_meta_bytes(W, FB, p.n_leaves, STAGED));
+    else frag = (Frag)p.scratch + (long long)blockIdx.x * p.n_slots * slot_tiles * FB * 64;
+    unsigned a_lane[4];   // byte offsets of the lane's entries (fl, 4 j + g) of a 16 x 16 block
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a_lane[j] = 8u * ((4 * j + g) * Np + fl);
+    // a block past the matrix's last column: zeros (Np >= N + 16)
+    const int zero_col = Np - kTile;
+
+    // each XCD (workgroup b runs on b % 8) takes one contiguous range of the
+    // list, whose neighbours share their matrices in its L2
+    const int n_tiles = *as_const(p.n_tiles_dev);
+    const int groups = (gridDim.x % 8 == 0) ? 8 : 1;
+    const int per_group = gridDim.x / groups;
+    const int grp = blockIdx.x % groups;
+    const int t_lo = (int)((long long)n_tiles * grp / groups);
+    const int t_hi = (int)((long long)n_tiles * (grp + 1) / groups);
+    for (int tile = t_lo + (int)blockIdx.x / groups; tile < t_hi; tile += per_group) {
+        const TileDesc td = ld_const(p.tiles, tile);
+        const BucketDev bk = ld_const(p.buckets, td.bucket);
+        const int nf = td.nf < 0 ? -td.nf : td.nf;
+        for (int i = threadIdx.x; STAGED && i < p.n_leaves * FW; i += 64 * W) {
+            const int f = i & (FW - 1);
+            const int ff = td.fam0 + (f < nf ? f : 0);
+            const int fam = td.nf < 0 ? p.fam_list[ff] : bk.fam_begin + ff;
+            s_cnt[i] = 8u * Np * p.counts_T[(long long)(i / FW) * p.F + fam];
+        }
+        int fam[FB], dst[FB];   // this lane's families, and their places in the caller's order
+#pragma unroll
+        for (int f = 0; f < FB; ++f) {
+            const int ff = td.fam0 + (16 * f + fl < nf ? 16 * f + fl : 0);
+            fam[f] = td.nf < 0 ? p.fam_list[ff] : bk.fam_begin + ff;
+            dst[f] = p.perm[fam[f]];
+        }
+        const __attribute__((address_space(4))) int* nslot = as_const(p.node_slot + (long long)td.point * p.n_nodes);
+        const int nkt = bk.Lp / kTile;   // k-tiles of a child vector
+        __syncthreads();
+
+        // The wave's work is a list of steps: for every op and each of the wave's
+        // chunks of it, the op's children.  While a step is computed, the next
+        // one's first loads -- its leaf columns, or the first FB k-tiles of its
+        // A operand (the same loads from a selected base, stride and lane
+        // offset) -- are in flight, also across the barrier between ops: they
+        // read nothing the kernel writes.
+        struct Step {
+            StepDev sd;
+            int st;      // its index in the program
+            int first;   // the op's first step
+            int c;       // chunk
+        };
+        auto root_of = [&](const Step& s) { return (s.sd.ctl & kStepRoot) != 0; };
+        auto tiles_of = [&](bool root) { return ((root ? bk.R : bk.L) + kTile - 1) / kTile; };
+        auto base_of = [&](const Step& s) {   // root rows are sizes 1..R
+            return (long long)nslot[s.sd.node] * p.slot_elems + (root_of(s) ? 1 : 0);
+        };
+        auto row_tile = [&](const Step& s, int i) {   // clamped: a chunk's tiles past the end are dropped
+            const int n = tiles_of(root_of(s));
+            return s.c * NTW + i < n ? s.c * NTW + i : n - 1;
+        };
+        auto issue = [&](d4 (&pf)[FB][NTW], const Step& s) {
+            const bool leaf = s.sd.leaf_col >= 0;
+            const double* M = (leaf ? p.leaf64 : p.mt64) + base_of(s);
+#pragma unroll
+            for (int f = 0; f < FB; ++f) {
+                const int col = leaf ? s.sd.leaf_col : 0;
+                const unsigned cnt = STAGED ? s_cnt[col * FW + 16 * f + fl] : 8u * Np * p.counts_T[(long long)col * p.F + fam[f]];
+                const unsigned cn = cnt + 8u * g;
+                const int kt = leaf ? 0 : Np * (f < nkt ? kTile * f : zero_col);
+                const unsigned off = leaf ? cn : a_lane[0];
+                const int step = leaf ? 4 : 4 * Np;
+#pragma unroll
+                for (int i = 0; i < NTW; ++i) {
+                    const double* C = M + (kt + kTile * row_tile(s, i));
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) pf[f][i][r] = at(uniform(C + r * step), off);
+                }
+            }
+        };
+        d4 acc[FB][NTW];
+        auto compute = [&](const d4 (&pf)[FB][NTW], const Step& s) {
+            const bool root = root_of(s);
+            d4 x[FB][NTW];
+            if (s.sd.leaf_col >= 0) {   // column `count` (the error model is folded into it)
+#pragma unroll
+                for (int f = 0; f < FB; ++f)
+#pragma unroll
+                    for (int i = 0; i < NTW; ++i) x[f][i] = pf[f][i];
+            } else {
+                const Frag V = frag + s.sd.in_slot * slot_tiles * FB * 64 + lane;
+                const double* M = p.mt64 + base_of(s);
+                auto mma = [&](const d4 (&a)[NTW], const d4 (&b)[FB]) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int f = 0; f < FB; ++f)
+#pragma unroll
+                            for (int i = 0; i < NTW; ++i)
+                                x[f][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][j], b[f][j], x[f][i], 0, 0, 0);
+                };
+                // k-tiles FB .. nkt - 1: D in flight while one is multiplied.  The
+                // loop has no other branch, so that every wait covers only the
+                // oldest k-tile: past the end it multiplies the zero block,
+                // which adds exactly 0.
+                constexpr int D = 2;
+                d4 a[D][NTW], b[D][FB];
+                auto load = [&](d4 (&a)[NTW], d4 (&b)[FB], int kt) {
+                    const int kb = kt < nkt ? kt : nkt - 1;
+                    const int c = Np * (kt < nkt ? kTile * kt : zero_col);
+#pragma unroll
+                    for (int i = 0; i < NTW; ++i) {
+                        const Gptr C = uniform(M + (c + kTile * row_tile(s, i)));
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) a[i][j] = at(C, a_lane[j]);
+                    }
+#pragma unroll
+                    for (int f = 0; f < FB; ++f) b[f] = V[(kb * FB + f) * 64];
+                };
+#pragma unroll
+                for (int f = 0; f < FB; ++f)
+#pragma unroll
+                    for (int i = 0; i < NTW; ++i) x[f][i] = d4{0, 0, 0, 0};
+                d4 b0[FB][FB];
+#pragma unroll
+                for (int k = 0; k < FB; ++k)
+#pragma unroll
+                    for (int f = 0; f < FB; ++f) b0[k][f] = V[((k < nkt ? k : 0) * FB + f) * 64];
+                if (nkt > FB) {
+#pragma unroll
+                    for (int d = 0; d < D; ++d) load(a[d], b[d], FB + d);
+#pragma unroll
+                    for (int k = 0; k < FB; ++k) mma(pf[k], b0[k]);
+                    for (int kt = FB; kt < nkt; kt += D)
+#pragma unroll
+                        for (int d = 0; d < D; ++d) {
+                            mma(a[d], b[d]);
+                            load(a[d], b[d], kt + d + D);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < FB; ++k) mma(pf[k], b0[k]);
+                }
+            }
+            if (s.sd.ctl & kStepFirst) {
+#pragma unroll
+                for (int f = 0; f < FB; ++f)
+#pragma unroll
+                    for (int i = 0; i < NTW; ++i) acc[f][i] = x[f][i];
+                asm volatile("");   // (a branch: the vector unit is the scarce one)
+            } else {
+#pragma unroll
+                for (int f = 0; f < FB; ++f)
+#pragma unroll
+                    for (int i = 0; i < NTW; ++i) acc[f][i] *= x[f][i];
+            }
+            if (!(s.sd.ctl & kStepLast)) return;
+            const int len = root ? bk.R : bk.L, nrt = tiles_of(root);
+            const Frag out = frag + (s.sd.ctl & kStepSlotMask) * slot_tiles * FB * 64 + lane;
+#pragma unroll
+            for (int i = 0; i < NTW; ++i) {
+                const int t = s.c * NTW + i;
+                if (t >= nrt) break;
+#pragma unroll
+                for (int f = 0; f < FB; ++f) {
+                    d4 v = acc[f][i];
+                    if (kTile * t + kTile > len) {   // rows past the bound
+                        asm volatile("");
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) v[r] = kTile * t + 4 * r + g < len ? v[r] : 0.0;
+                    }
+                    out[(t * FB + f) * 64] = v;
+                    if (root && p.root_out && 16 * f + fl < nf)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int j = kTile * t + 4 * r + g;
+                            if (j < len) p.root_out[(long long)dst[f] * p.root_stride + j] = v[r];
+                        }
+                }
+            }
+        };
+        // the step after s: the next child, the op's next chunk, or the next op
+        auto advance = [&](Step& s) {
+            if (!(s.sd.ctl & kStepLast)) {
+                ++s.st;
+            } else if ((s.c + W) * NTW < tiles_of(root_of(s))) {
+                s.c += W;
+                s.st = s.first;
+            } else {
+                s.c = wv;
+                s.first = ++s.st;
+            }
+            s.sd = ld_const(p.steps, s.st < p.n_steps ? s.st : p.n_steps - 1);
+        };
+        d4 pfa[FB][NTW], pfb[FB][NTW];
+        Step sa{ld_const(p.steps, 0), 0, 0, wv}, sb;
+        issue(pfa, sa);
+        // an op ends where the following step is another op's
+        for (;;) {
+            sb = sa;
+            advance(sb);
+            issue(pfb, sb);
+            compute(pfa, sa);
+            if (sb.first != sa.first) __syncthreads();
+            if (sb.st >= p.n_steps) break;
+            sa = sb;
+            advance(sa);
+            issue(pfa, sa);
+            compute(pfb, sb);
+            if (sa.first != sb.first) __syncthreads();
+            if (sa.st >= p.n_steps) break;
+        }
+        const int root_slot = ld_const(p.steps, p.n_steps - 1).ctl & kStepSlotMask;
+
+        // max_j log x_j + log prior_j (base_model.cpp:84-90) or x_j prior_j
+        // (gamma_core.cpp:156-161): the largest product first, then the
+        // logarithms of the rows near it only (of all rows where the product
+        // leaves FP64's normal range), so the maximum is over the same values
+        const Frag x = frag + root_slot * slot_tiles * FB * 64 + lane;
+        const double* __restrict__ pr = p.prior64 + bk.prior_off;
+        const double inf = __builtin_huge_val();
+        const int nrt = (bk.R + kTile - 1) / kTile;
+        double best[FB], xmax[FB];
+#pragma unroll
+        for (int f = 0; f < FB; ++f) {
+            best[f] = -inf;
+            xmax[f] = 0.0;
+        }
+        for (int t = wv; t < nrt; t += W)
+#pragma unroll
+            for (int f = 0; f < FB; ++f) {
+                const d4 v = x[(t * FB + f) * 64];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int j = kTile * t + 4 * r + g;
+                    if (j >= bk.R) continue;
+                    const double q = v[r] * pr[j];
+                    best[f] = q > best[f] ? q : best[f];
+                    xmax[f] = v[r] > xmax[f] ? v[r] : xmax[f];
+                }
+            }
+        // a family's maxima over its lanes, then over the waves
+        auto over_lanes = [&](double v) {
+            for (int d = 16; d <= 32; d <<= 1) {
+                const double o = __shfl_xor(v, d);
+                v = o > v ? o : v;
+            }
+            return v;
+        };
+#pragma unroll
+        for (int f = 0; f < FB; ++f) {
+            best[f] = over_lanes(best[f]);
+            xmax[f] = over_lanes(xmax[f]);
+            if (g == 0) {
+                s_a[wv * FW + 16 * f + fl] = best[f];
+                s_b[wv * FW + 16 * f + fl] = xmax[f];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < FB; ++f)
+            for (int w = 0; w < W; ++w) {
+                const double b = s_a[w * FW + 16 * f + fl], m = s_b[w * FW + 16 * f + fl];
+                best[f] = b > best[f] ? b : best[f];
+                xmax[f] = m > xmax[f] ? m : xmax[f];
+            }
+        double val[FB];
+#pragma unroll
+        for (int f = 0; f < FB; ++f) val[f] = best[f];
+        if (p.model == 0) {
+#pragma unroll
+            for (int f = 0; f < FB; ++f) val[f] = -inf;
+            for (int t = wv; t < nrt; t += W)
+#pragma unroll
+                for (int f = 0; f < FB; ++f) {
+                    const d4 v = x[(t * FB + f) * 64];
+                    const bool every = !(best[f] >= kFp64Floor && best[f] < inf);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int j = kTile * t + 4 * r + g;
+                        if (j < bk.R && (every || v[r] * pr[j] >= best[f] * kNearBest)) {
+                            const double k = log(v[r]) + log(pr[j]);
+                            val[f] = k > val[f] ? k : val[f];
+                        }
+                    }
+                }
+            __syncthreads();   // the waves have read the first maxima
+#pragma unroll
+            for (int f = 0; f < FB; ++f) {
+                val[f] = over_lanes(val[f]);
+                if (g == 0) s_a[wv * FW + 16 * f + fl] = val[f];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int f = 0; f < FB; ++f)
+                for (int w = 0; w < W; ++w) {
+                    const double b = s_a[w * FW + 16 * f + fl];
+                    val[f] = b > val[f] ? b : val[f];
+                }
+        }
+        if (wv == 0 && g == 0) {
+#pragma unroll
+            for (int f = 0; f < FB; ++f) {
+                if (16 * f + fl >= nf) continue;
+                // a first key that is not a number stays (std::max_element
+                // keeps it): row 0 of the vector is this lane's
+                const double x0 = x[f * 64][0];
+                const double k0 = p.model == 0 ? log(x0) + log(pr[0]) : x0 * pr[0];
+                p.out_val[(long long)td.point * p.F + dst[f]] = k0 != k0 ? k0 : val[f];
+                p.out_flag[(long long)td.point * p.F + dst[f]] = xmax[f] == 0.0 ? kFlagZeroSum : 0;
+                // values near the subnormal range are counted
+                if (p.near_floor && (xmax[f] < kFp64Floor || best[f] < kFp64Floor)) atomicAdd(p.near_floor, 1);
+            }
+        }
+        __syncthreads();   // every wave is done with this tile's LDS and vectors
+    }
+}
+
+// One instance per shape; with per_cu set, reports how many workgroups of it
+// fit on one CU (0: no such shape or it does not fit) instead of launching.
+hipError_t f64_dispatch(const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st, int* per_cu)
+{
+    if (per_cu) *per_cu = 0;
+#define CAFE_F64_CASE(NTW, FB, LDSP, STAGED)                                                                      \
+    if (s.ntw == NTW && s.fb == FB && s.lds == LDSP && s.staged == STAGED && s.w >= 1 && s.w <= F64Waves<NTW, FB>::v) { \
+        if (per_cu)                                                                                               \
+            return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, k_prune_f64<NTW, FB, LDSP, STAGED>, 64 * s.w, \
+                                                                s.shm);                                           \
+        hipLaunchKernelGGL((k_prune_f64<NTW, FB, LDSP, STAGED>), dim3(grid < 1 ? 1 : grid), dim3(64 * s.w), s.shm, st, \
+                           p);                                                                                    \
+        return hipGetLastError();                                                                                 \
+    }
+    CAFE_F64_CASE(1, 1, true, true) CAFE_F64_CASE(1, 1, false, true) CAFE_F64_CASE(1, 1, false, false)
+    CAFE_F64_CASE(2, 1, false, true) CAFE_F64_CASE(1, 2, true, true) CAFE_F64_CASE(2, 2, false, true)
+#undef CAFE_F64_CASE
+    return hipErrorInvalidValue;
+}
+
+}  // namespace cafe

@@ -1,4 +1,4 @@
-// prune_mfma.hip -- batched Felsenstein pruning on the matrix cores
+// prune_mfma.hip -- batched FP32 Felsenstein pruning on the matrix cores
 // (replaces inference_prune / compute_node_probability, src/core.cpp:134-145,
 // src/probability.cpp:175-330, and the root reductions of base_model.cpp:77-95
 // and gamma_core.cpp:143-165, for many families at once).
@@ -17,9 +17,7 @@
 // This is the D layout of v_mfma_f32_16x16x4f32, and it is also the B operand
 // layout of the next contraction when the contraction index of MFMA j of
 // k-tile kt in lane group g is x = 16 kt + 4 g + j: a node's output is the next
-// node's input without any data movement.  v_mfma_f64_16x16x4f64 returns D row
-// g + 4 r in register r; the FP64 kernel feeds A row m from size
-// 4 (m % 4) + m / 4, which lands size 4 g + r in that register as well.
+// node's input without any data movement.
 //
 // Persistent kernels: a fixed grid walks the class's tile list (its length is
 // device-resident, so recompute lists built on the device need no host round
@@ -28,26 +26,12 @@
 
 namespace cafe {
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef double doublex4 __attribute__((ext_vector_type(4)));
+typedef float V4 __attribute__((ext_vector_type(4)));
 
-template <typename T> struct Vec4;
-template <> struct Vec4<float> { typedef floatx4 type; };
-template <> struct Vec4<double> { typedef doublex4 type; };
-
-__device__ __forceinline__ floatx4 mfma16(float a, float b, floatx4 c)
+__device__ __forceinline__ V4 mfma16(float a, float b, V4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ doublex4 mfma16(double a, double b, doublex4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ const float* pool_of(const PruneParams& p, float*) { return p.mt32; }
-__device__ __forceinline__ const double* pool_of(const PruneParams& p, double*) { return p.mt64; }
-__device__ __forceinline__ const float* leaf_of(const PruneParams& p, float*) { return p.leaf32; }
-__device__ __forceinline__ const double* leaf_of(const PruneParams& p, double*) { return p.leaf64; }
 
 // Waits for this wave's LDS traffic and meets the workgroup at a barrier,
 // leaving global loads in flight (the next step's prefetched operands).
@@ -56,28 +40,13 @@ __device__ __forceinline__ void lds_barrier()
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// Size that A row m of a 16-row tile carries (see the fragment layout above).
-__device__ __forceinline__ int a_row(float*, int m) { return m; }
-__device__ __forceinline__ int a_row(double*, int m) { return 4 * (m & 3) + (m >> 2); }
-
-// Matrix element (s, c): the FP32 pool is row-major, the FP64 pool c-major.
-// Offsets within one matrix fit in 32 bits (Np <= 1040), so addresses are a
-// uniform base plus a 32-bit lane offset.
-__device__ __forceinline__ float mat(const float* M, int Np, int s, int c) { return M[s * Np + c]; }
-__device__ __forceinline__ double mat(const double* M, int Np, int s, int c) { return M[c * Np + s]; }
-
-// A operand of k-tile kt for a lane whose A row is size s: the four entries
-// (s, 16 kt + 4 g + j), j = 0..3.  FP32: one 16-byte load from the row.
-__device__ __forceinline__ int a_off(float*, int Np, int s, int g) { return s * Np + 4 * g; }
-__device__ __forceinline__ floatx4 load_a(const float* M, int off, int kt, int)
+// A operand of k-tile kt for a lane whose A row starts at `off` (row s * Np +
+// 4 g): the four entries (s, 16 kt + 4 g + j), j = 0..3, one 16-byte load from
+// the row-major pool.  Offsets within one matrix fit in 32 bits (Np <= 1040),
+// so addresses are a uniform base plus a 32-bit lane offset.
+__device__ __forceinline__ V4 load_a(const float* M, int off, int kt)
 {
-    return *(const floatx4*)(M + off + kTile * kt);
-}
-__device__ __forceinline__ int a_off(double*, int Np, int s, int g) { return 4 * g * Np + s; }
-__device__ __forceinline__ doublex4 load_a(const double* M, int off, int kt, int Np)
-{
-    const int o = off + kTile * kt * Np;
-    return doublex4{M[o], M[o + Np], M[o + 2 * Np], M[o + 3 * Np]};
+    return *(const V4*)(M + off + kTile * kt);
 }
 
 // ds_swizzle pattern: lane l reads lane l ^ 16 (within each 32-lane half).
@@ -101,9 +70,9 @@ __device__ __forceinline__ void await_loaded(const V& v)
     for (int j = 0; j < 4; ++j) asm volatile("" ::"v"(v[j]));
 }
 
-// Operand prefetch depth: FP32 prefetches k-tiles 0 and 1 of an internal
-// step (two 16-byte loads per output tile), FP64 k-tile 0 (four 8-byte loads).
-template <typename T> struct Prefetch { static constexpr int PK = sizeof(T) == 4 ? 2 : 1; };
+// Operand prefetch depth: k-tiles 0 and 1 of an internal step (two 16-byte
+// loads per output tile).
+constexpr int PK = 2;
 
 __device__ __forceinline__ RootBest root_combine(RootBest b)
 {
@@ -119,18 +88,16 @@ __device__ __forceinline__ RootBest root_combine(RootBest b)
 
 // One k-tile of MFMAs: x[f][i] += A_i(kt) B_f(kt) for the wave's NTW output
 // tiles and the tile's FB blocks of 16 families (each A operand feeds FB
-// MFMAs).  SCALED: the stored child fragment of block f is renormalised on the
-// fly by 2^bsh[f].
-template <typename T, int NTW, bool SCALED, int FB>
-__device__ __forceinline__ void mma_step(typename Vec4<T>::type (&x)[FB][NTW], const typename Vec4<T>::type (&a)[NTW],
-                                         const typename Vec4<T>::type (&b)[FB], const int (&bsh)[FB])
+// MFMAs).  The stored child fragment of block f is renormalised on the fly by
+// 2^bsh[f].
+template <int NTW, int FB>
+__device__ __forceinline__ void mma_step(V4 (&x)[FB][NTW], const V4 (&a)[NTW], const V4 (&b)[FB], const int (&bsh)[FB])
 {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
 #pragma unroll
         for (int f = 0; f < FB; ++f) {
-            T bj = b[f][j];
-            if constexpr (SCALED) bj = ldexpf(bj, bsh[f]);
+            const float bj = ldexpf(b[f][j], bsh[f]);
 #pragma unroll
             for (int i = 0; i < NTW; ++i) x[f][i] = mfma16(a[i][j], bj, x[f][i]);
         }
@@ -146,40 +113,33 @@ __device__ __forceinline__ void mma_step(typename Vec4<T>::type (&x)[FB][NTW], c
 // fragment zeroed, which adds exactly 0, so each wait covers only the oldest
 // buffer.  A one-wave kernel holds whole vectors (nts <= NTW), so its ring
 // only needs the NTW - PK k-tiles past the prefetched ones (none for NTW <= PK).
-template <typename T, int NTW, int W, int FB> struct Ring {
-    // two k-tiles in flight; a deeper ring costs registers (the 4-tile FP32
-    // shapes would drop to one wave per SIMD) without shortening their step
-    // time, which other waves' work covers.  The FP64 recompute shapes with
-    // one or two tiles per wave run a few workgroups whose step time is the
-    // k-loop's memory latency: four in flight.  W = 16 leaves 128 VGPRs per
-    // wave: two with one output tile of one family block per wave (the FP64
-    // recompute of the largest vectors is such a chain), else one.
-    static constexpr int deep = W >= 16 ? (NTW == 1 && FB == 1 ? 2 : 1) : (sizeof(T) == 8 && NTW <= 2 ? 4 : 2);
-    static constexpr int tail = NTW > Prefetch<T>::PK ? NTW - Prefetch<T>::PK : 0;
+template <int NTW, int W, int FB> struct Ring {
+    // two k-tiles in flight; a deeper ring costs registers (the 4-tile shapes
+    // would drop to one wave per SIMD) without shortening their step time,
+    // which other waves' work covers.  W = 16 leaves 128 VGPRs per wave: two
+    // with one output tile of one family block per wave, else one.
+    static constexpr int deep = W >= 16 ? (NTW == 1 && FB == 1 ? 2 : 1) : 2;
+    static constexpr int tail = NTW > PK ? NTW - PK : 0;
     static constexpr int D = W == 1 ? tail : deep;
 };
 
 // Child fragments of k-tile kt, family block f: stored at (kt FB + f) 64 + lane
 // from the slot's base (both blocks of a k-tile side by side).
-template <typename T, int NTW, int D, bool SCALED, int FB>
-__device__ __forceinline__ void child_gemm(typename Vec4<T>::type (&x)[FB][NTW], const T* __restrict__ M, int Np,
-                                           const int (&ao)[NTW],
-                                           const typename Vec4<T>::type (&pf)[Prefetch<T>::PK][NTW],
-                                           const typename Vec4<T>::type* bsrc, int nts, const int (&bsh)[FB])
+template <int NTW, int D, int FB>
+__device__ __forceinline__ void child_gemm(V4 (&x)[FB][NTW], const float* __restrict__ M, const int (&ao)[NTW],
+                                           const V4 (&pf)[PK][NTW], const V4* bsrc, int nts, const int (&bsh)[FB])
 {
-    typedef typename Vec4<T>::type V4;
-    constexpr int PK = Prefetch<T>::PK;
     {
         V4 b0[FB];
 #pragma unroll
         for (int f = 0; f < FB; ++f) b0[f] = bsrc[f * 64];
-        mma_step<T, NTW, SCALED, FB>(x, pf[0], b0, bsh);
-        if (PK > 1 && nts > 1) {
+        mma_step<NTW, FB>(x, pf[0], b0, bsh);
+        if (nts > 1) {
             V4 b1[FB];
 #pragma unroll
             for (int f = 0; f < FB; ++f) b1[f] = bsrc[(FB + f) * 64];
-            mma_step<T, NTW, SCALED, FB>(x, pf[PK - 1], b1, bsh);
-        } else if (PK > 1) {
+            mma_step<NTW, FB>(x, pf[PK - 1], b1, bsh);
+        } else {
             // unused second k-tile: still wait for it (see the leaf step)
 #pragma unroll
             for (int i = 0; i < NTW; ++i) await_loaded(pf[PK - 1][i]);
@@ -192,18 +152,18 @@ __device__ __forceinline__ void child_gemm(typename Vec4<T>::type (&x)[FB][NTW],
     for (int d = 0; d < D; ++d) {
         const int k = PK + d < nts ? PK + d : nts - 1;
 #pragma unroll
-        for (int i = 0; i < NTW; ++i) a[d][i] = load_a(M, ao[i], k, Np);
+        for (int i = 0; i < NTW; ++i) a[d][i] = load_a(M, ao[i], k);
 #pragma unroll
         for (int f = 0; f < FB; ++f) bb[d][f] = PK + d < nts ? bsrc[(k * FB + f) * 64] : V4{0, 0, 0, 0};
     }
     for (int kt = PK; kt < nts; kt += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            mma_step<T, NTW, SCALED, FB>(x, a[d], bb[d], bsh);
+            mma_step<NTW, FB>(x, a[d], bb[d], bsh);
             const int kn = kt + D + d;   // the k-tile this buffer holds next
             const int k = kn < nts ? kn : nts - 1;
 #pragma unroll
-            for (int i = 0; i < NTW; ++i) a[d][i] = load_a(M, ao[i], k, Np);
+            for (int i = 0; i < NTW; ++i) a[d][i] = load_a(M, ao[i], k);
 #pragma unroll
             for (int f = 0; f < FB; ++f) bb[d][f] = kn < nts ? bsrc[(k * FB + f) * 64] : V4{0, 0, 0, 0};
         }
@@ -218,8 +178,7 @@ __device__ __forceinline__ void child_gemm(typename Vec4<T>::type (&x)[FB][NTW],
 // the same loads from per-lane offsets computed once per tile, so the waits
 // count the younger loads exactly).  Wave wv computes NTW output tiles (W NTW
 // covers the largest vector of the size class; tiles past a vector's end are
-// computed on a clamped, in-bounds tile and dropped): FP64 tiles wv + W i;
-// FP32 the contiguous run [wv n / W, (wv + 1) n / W) of the n row tiles, so
+// computed on a clamped, in-bounds tile and dropped): the contiguous run [wv n / W, (wv + 1) n / W) of the n row tiles, so
 // that an interior step multiplies only the k-tiles inside the union of its
 // rows' bands (the FP32 pool's nonzero k-tiles per row tile, recorded by the
 // build): the A blocks it skips are exactly 0, so each sum is unchanged.
@@ -227,7 +186,7 @@ __device__ __forceinline__ void child_gemm(typename Vec4<T>::type (&x)[FB][NTW],
 // workgroup's region of the global scratch; the leaf counts of the tile's
 // families are staged in LDS.
 //
-// T = float, SCALED: FP32 matrices are stored times 2^kMatExp; a node's raw
+// FP32 matrices are stored times 2^kMatExp; a node's raw
 // product is stored as computed, and its per-family maximum m renormalises it
 // when it is read: v' = raw 2^(a - e), e = exponent of m, so max v' is just
 // below 2^a (a = vec_exp).  The exponent is carried as an integer, and a
@@ -235,12 +194,11 @@ __device__ __forceinline__ void child_gemm(typename Vec4<T>::type (&x)[FB][NTW],
 // root whether the family is kept or recomputed in FP64.  A single-wave
 // workgroup finishes a node's exponent, shift and bound when it stores the
 // node; with several waves the reader combines the per-wave maxima.
-// T = double: unscaled, so values (and underflow) follow the reference.
 // ---------------------------------------------------------------------------
 // Single-wave kernels with small per-wave tiles ask for 4 waves per SIMD (the
 // register budget that still holds both prefetch buffers without spilling).
-template <int NTW, int W, int BYTES> struct WavesHint {
-    static constexpr int v = (W == 1 && NTW * BYTES <= 8) ? 4 : 1;
+template <int NTW, int W, int FB> struct WavesHint {
+    static constexpr int v = (W == 1 && NTW * FB <= 2) ? 4 : 1;
 };
 
 // FB = 2: a tile carries 32 families, two blocks of 16 (block f holds
@@ -248,22 +206,18 @@ template <int NTW, int W, int BYTES> struct WavesHint {
 // (matrix fragment) feeds both blocks' MFMAs, so a tile reads its matrices
 // once for twice the families, and a k-tile's loads in flight cover twice the
 // matrix-core work.  The per-family bookkeeping is kept per block.
-template <typename T, int NTW, int W, bool SCALED, bool LDSP, int FB>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(WavesHint<NTW, W, (int)sizeof(T) * FB>::v)))
+template <int NTW, int W, bool LDSP, int FB>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(WavesHint<NTW, W, FB>::v)))
 void k_prune_mfma(PruneParams p)
 {
-    typedef typename Vec4<T>::type V4;
-    constexpr int PK = Prefetch<T>::PK;
-    constexpr bool kF64 = sizeof(T) == 8;
     constexpr int FW = 16 * FB;   // families per tile
     static_assert(FB == 1 || PK >= FB, "a leaf step loads one column per family block into the prefetch buffers");
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int fl = lane & 15;
     const int g = lane >> 4;
-    const int my_arow = a_row((T*)nullptr, fl);
-    const T* __restrict__ pool = pool_of(p, (T*)nullptr);
-    const T* __restrict__ lpool = leaf_of(p, (T*)nullptr);
+    const float* __restrict__ pool = p.mt32;
+    const float* __restrict__ lpool = p.leaf32;
     const int Np = p.Np;
     const int n_slots = p.n_slots;
     const int slot_tiles = p.slot_tiles;
@@ -286,7 +240,7 @@ void k_prune_mfma(PruneParams p)
     int* m_esum = (int*)(m_wmax + n_slots * W * FW);
     int* m_bsh = m_esum + n_slots * FW;
     int* m_l2s = m_bsh + n_slots * FW;
-    const int meta = mfma_meta_bytes(n_slots, W, SCALED, FB);
+    const int meta = mfma_meta_bytes(n_slots, W, FB);
     int* s_cnt = (int*)(s_dyn + meta);                // [leaf][FW]
     V4* frag = LDSP ? (V4*)(s_dyn + meta + mfma_count_bytes(p.n_leaves, FB))
                     : (V4*)p.scratch + (long long)blockIdx.x * n_slots * slot_tiles * FB * 64;
@@ -330,37 +284,34 @@ void k_prune_mfma(PruneParams p)
         const int rows_root = bk.Rp / kTile;  // root rows are sizes 0..R
         // flush-bound terms of an interior factor (FP32 matrix entries, MFMA
         // products and stored vector entries that may flush)
-        const double cint = SCALED ? kTau32 * (bk.Lp * kTwoPowMinusMatExp * (1.0 + two_m_a) + two_m_a) : 0.0;
+        const double cint = kTau32 * (bk.Lp * kTwoPowMinusMatExp * (1.0 + two_m_a) + two_m_a);
 
         // per-lane offsets of this wave's output tiles, non-root [0] / root [1]:
-        // A operand row (FP32 row-major) or column block (FP64 c-major), and
-        // leaf rows within a c-major column
+        // A operand row (row-major), and leaf rows within a c-major column
         // (separate arrays, chosen with selects: an array indexed by the
         // root flag would be placed in scratch memory)
         int offA0[NTW], offA1[NTW], offL0[NTW], offL1[NTW];
-        // FP32: this wave's run of row tiles, non-root [c0, c1) / root [r0, r1)
-        const int c0 = kF64 ? 0 : wv * nts / W, c1 = kF64 ? 0 : (wv + 1) * nts / W;
-        const int r0 = kF64 ? 0 : wv * rows_root / W, r1 = kF64 ? 0 : (wv + 1) * rows_root / W;
+        // this wave's run of row tiles, non-root [c0, c1) / root [r0, r1)
+        const int c0 = wv * nts / W, c1 = (wv + 1) * nts / W;
+        const int r0 = wv * rows_root / W, r1 = (wv + 1) * rows_root / W;
 #pragma unroll
         for (int i = 0; i < NTW; ++i) {
-            const int u0 = kF64 ? wv + W * i : c0 + i, e0 = kF64 ? nts : c1;
-            const int u1 = kF64 ? wv + W * i : r0 + i, e1 = kF64 ? rows_root : r1;
-            const int t0 = u0 < e0 ? u0 : nts - 1;
-            const int t1 = u1 < e1 ? u1 : rows_root - 1;
-            offA0[i] = kF64 ? 4 * g * Np + kTile * t0 + my_arow : (kTile * t0 + my_arow) * Np + 4 * g;
-            offA1[i] = kF64 ? 4 * g * Np + kTile * t1 + my_arow : (kTile * t1 + my_arow) * Np + 4 * g;
+            const int t0 = c0 + i < c1 ? c0 + i : nts - 1;
+            const int t1 = r0 + i < r1 ? r0 + i : rows_root - 1;
+            offA0[i] = (kTile * t0 + fl) * Np + 4 * g;
+            offA1[i] = (kTile * t1 + fl) * Np + 4 * g;
             offL0[i] = kTile * t0 + 4 * g;
             offL1[i] = kTile * t1 + 4 * g;
         }
-        // one-wave FP32 kernels start a non-root product from a 0/1 row mask
+        // one-wave kernels start a non-root product from a 0/1 row mask
         // (rows past the bound are 0 and stay 0), so the node's store needs no
         // masking; the others mask when they store
-        constexpr bool kMaskFirst = SCALED && W == 1 && NTW == 2 && FB == 1;   // registers to spare: the 2-tile class
+        constexpr bool kMaskFirst = W == 1 && NTW == 2 && FB == 1;   // registers to spare: the 2-tile class
         V4 keep[kMaskFirst ? NTW : 1];
 #pragma unroll
         for (int i = 0; i < (kMaskFirst ? NTW : 1); ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) keep[i][r] = kTile * (wv + W * i) + 4 * g + r < bk.L ? T(1) : T(0);
+            for (int r = 0; r < 4; ++r) keep[i][r] = kTile * (wv + W * i) + 4 * g + r < bk.L ? 1.f : 0.f;
 
         // loads of step st (clamped to the last step) into pf; its descriptor
         // into sd.  A leaf step loads its column for family block k into
@@ -373,7 +324,7 @@ void k_prune_mfma(PruneParams p)
         auto kband = [&](int slot, bool root, int& klo, int& kn) {
             klo = 0;
             kn = nts;
-            if constexpr (!kF64 && W > 1) {
+            if constexpr (W > 1) {
                 if (!band) return;
                 const int a = root ? r0 : c0, b = root ? r1 : c1;
                 int lo = nts, hi = 0;
@@ -401,7 +352,7 @@ void k_prune_mfma(PruneParams p)
             const bool root = (sd.ctl & kStepRoot) != 0;
             const bool leaf = sd.leaf_col >= 0;
             const int slot = nslot[sd.node];
-            const T* __restrict__ M = (leaf ? lpool : pool) + (long long)slot * p.slot_elems;
+            const float* __restrict__ M = (leaf ? lpool : pool) + (long long)slot * p.slot_elems;
             klo = 0;
             kn = nts;
             if (!leaf) kband(slot, root, klo, kn);
@@ -413,19 +364,13 @@ void k_prune_mfma(PruneParams p)
                     const int oa = root ? offA1[i] : offA0[i];
                     const int ol = cn + (root ? offL1[i] : offL0[i]);
                     const int kk = klo + (k < kn ? k : kn - 1);
-                    if constexpr (!kF64) {
-                        const int off = leaf ? ol + (FB > 1 ? 0 : 4 * k * zero) : oa + kTile * kk;
-                        pf[k][i] = *(const floatx4*)(M + off);
-                    } else {
-                        const int base = leaf ? ol : oa + kTile * kk * Np;
-                        const int step = leaf ? 1 + zero : Np;
-                        pf[k][i] = V4{M[base], M[base + step], M[base + 2 * step], M[base + 3 * step]};
-                    }
+                    const int off = leaf ? ol + (FB > 1 ? 0 : 4 * k * zero) : oa + kTile * kk;
+                    pf[k][i] = *(const V4*)(M + off);
                 }
             }
         };
 
-        // per-op state (SCALED bookkeeping: a renormalised child v' holds
+        // per-op state (a renormalised child v' holds
         // v_c = v' 2^E_c with max v' < 2^a; its factor X' = M' v'
         // (M' = 2^kMatExp M) holds X_c = X' 2^(E_c - kMatExp) and is at most
         // 2^(kMatExp + a), leaf factors 2^kMatExp.
@@ -451,8 +396,8 @@ void k_prune_mfma(PruneParams p)
             bool live[NTW];
 #pragma unroll
             for (int i = 0; i < NTW; ++i) {
-                const int u = kF64 ? wv + W * i : (root ? r0 : c0) + i;
-                live[i] = u < (kF64 ? rows : root ? r1 : c1);
+                const int u = (root ? r0 : c0) + i;
+                live[i] = u < (root ? r1 : c1);
                 tt[i] = live[i] ? u : rows - 1;
             }
             if (sd.ctl & kStepFirst) {
@@ -470,14 +415,12 @@ void k_prune_mfma(PruneParams p)
             }
             V4 x[FB][NTW];
             if (sd.leaf_col >= 0) {
-                if (SCALED) {
 #pragma unroll
-                    for (int f = 0; f < FB; ++f) {
-                        e_sum[f] -= kMatExp;
-                        cert[f] += leaf_cert;
-                    }
-                    log2S += kMatExp;
+                for (int f = 0; f < FB; ++f) {
+                    e_sum[f] -= kMatExp;
+                    cert[f] += leaf_cert;
                 }
+                log2S += kMatExp;
 #pragma unroll
                 for (int f = 0; f < FB; ++f)
 #pragma unroll
@@ -493,33 +436,31 @@ void k_prune_mfma(PruneParams p)
                 int bsh[FB];
 #pragma unroll
                 for (int f = 0; f < FB; ++f) bsh[f] = 0;
-                if (SCALED) {
-                    log2S += kMatExp + a_exp;
+                log2S += kMatExp + a_exp;
 #pragma unroll
-                    for (int f = 0; f < FB; ++f) {
-                        const int q = sd.in_slot * FW + 16 * f + fl;
-                        if (W == 1) {
-                            bsh[f] = m_bsh[q];
-                            e_sum[f] += m_esum[q] - kMatExp;
-                            cert[f] += m_cert[q] + cint;
-                        } else {
-                            float m = 0.f;
-                            for (int w2 = 0; w2 < W; ++w2)
-                                m = fmaxf(m, m_wmax[(sd.in_slot * W + w2) * FW + 16 * f + fl]);
-                            int e = 0;
-                            const float mant = m > 0.f ? frexpf(m, &e) : 1.f;
-                            bsh[f] = a_exp - e;
-                            e_sum[f] += m_esum[q] + e - a_exp - kMatExp;
-                            cert[f] += (m > 0.f ? (ldexp(m_cert[q] * 1.01, m_l2s[sd.in_slot] - e) + ldexp(kTau32, -e)) *
-                                                      rcp_up(mant)
-                                                : 1e300) +
-                                       cint;
-                        }
+                for (int f = 0; f < FB; ++f) {
+                    const int q = sd.in_slot * FW + 16 * f + fl;
+                    if (W == 1) {
+                        bsh[f] = m_bsh[q];
+                        e_sum[f] += m_esum[q] - kMatExp;
+                        cert[f] += m_cert[q] + cint;
+                    } else {
+                        float m = 0.f;
+                        for (int w2 = 0; w2 < W; ++w2)
+                            m = fmaxf(m, m_wmax[(sd.in_slot * W + w2) * FW + 16 * f + fl]);
+                        int e = 0;
+                        const float mant = m > 0.f ? frexpf(m, &e) : 1.f;
+                        bsh[f] = a_exp - e;
+                        e_sum[f] += m_esum[q] + e - a_exp - kMatExp;
+                        cert[f] += (m > 0.f ? (ldexp(m_cert[q] * 1.01, m_l2s[sd.in_slot] - e) + ldexp(kTau32, -e)) *
+                                                  rcp_up(mant)
+                                            : 1e300) +
+                                   cint;
                     }
                 }
-                // FP32: the step's k-tiles start at klo (column 16 klo of the
+                // the step's k-tiles start at klo (column 16 klo of the
                 // row-major rows, fragment klo of the child)
-                const T* __restrict__ M = pool + (long long)nslot[sd.node] * p.slot_elems + (kF64 ? 0 : kTile * klo);
+                const float* __restrict__ M = pool + (long long)nslot[sd.node] * p.slot_elems + kTile * klo;
                 int ao[NTW];
 #pragma unroll
                 for (int i = 0; i < NTW; ++i) {
@@ -528,7 +469,7 @@ void k_prune_mfma(PruneParams p)
                     ao[i] = root ? offA1[i] : offA0[i];
                 }
                 const V4* bsrc = frag + ((long long)sd.in_slot * slot_tiles + klo) * FB * 64 + lane;
-                child_gemm<T, NTW, Ring<T, NTW, W, FB>::D, SCALED, FB>(x, M, Np, ao, pf, bsrc, kn, bsh);
+                child_gemm<NTW, Ring<NTW, W, FB>::D, FB>(x, M, ao, pf, bsrc, kn, bsh);
             }
 #pragma unroll
             for (int f = 0; f < FB; ++f)
@@ -537,7 +478,7 @@ void k_prune_mfma(PruneParams p)
             if (!(sd.ctl & kStepLast)) return;
 
             if (!root) {
-                T wmax[FB];
+                float wmax[FB];
 #pragma unroll
                 for (int f = 0; f < FB; ++f) {
                     wmax[f] = 0;
@@ -550,55 +491,52 @@ void k_prune_mfma(PruneParams p)
                             for (int r = 0; r < 4; ++r)
                                 if (kTile * tt[i] + 4 * g + r >= bk.L) v[r] = 0;   // rows past the bound
                         frag[(((long long)out_slot * slot_tiles + tt[i]) * FB + f) * 64 + lane] = v;
-                        if (SCALED)
 #pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                if constexpr (W == 1) wmax[f] = fmax(wmax[f], v[r]);   // entries are >= 0
-                                else wmax[f] = wmax[f] > v[r] ? wmax[f] : v[r];
-                            }
-                    }
-                }
-                if (SCALED) {
-#pragma unroll
-                    for (int f = 0; f < FB; ++f) {
-                        // maximum over the family's four lanes fl, fl+16, fl+32,
-                        // fl+48 (the one-wave kernels use lane swaps; the 4-tile
-                        // multi-wave shapes keep shuffles, which leave them the
-                        // registers for two waves per SIMD)
-                        float m = (float)wmax[f];
-                        if constexpr (W == 1) {
-                            m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(
-                                                                       __builtin_bit_cast(int, m), kSwizzleXor16)));
-                            m = xor32_max(m);
-                        } else {
-                            m = fmaxf(m, __shfl_xor(m, 16));
-                            m = fmaxf(m, __shfl_xor(m, 32));
-                        }
-                        const int q = out_slot * FW + 16 * f + fl;
-                        if (W == 1) {
-                            // finish the stored vector: shift, exponent, flush
-                            // bound re-expressed relative to the new scale (it
-                            // grows by S / m, the factor by which the product
-                            // fell short of its nominal scale)
-                            int e = 0;
-                            const float mant = m > 0.f ? frexpf(m, &e) : 1.f;
-                            if (g == 0) {
-                                m_bsh[q] = a_exp - e;
-                                m_esum[q] = e_sum[f] + e - a_exp;
-                                m_cert[q] = m > 0.f ? (ldexp(cert[f] * 1.01, log2S - e) + ldexp(kTau32, -e)) *
-                                                          rcp_up(mant)
-                                                    : 1e300;
-                            }
-                        } else {
-                            if (g == 0) m_wmax[(out_slot * W + wv) * FW + 16 * f + fl] = m;
-                            if (wv == 0 && g == 0) {
-                                m_esum[q] = e_sum[f];
-                                m_cert[q] = cert[f];
-                            }
+                        for (int r = 0; r < 4; ++r) {
+                            if constexpr (W == 1) wmax[f] = fmaxf(wmax[f], v[r]);   // entries are >= 0
+                            else wmax[f] = wmax[f] > v[r] ? wmax[f] : v[r];
                         }
                     }
-                    if (W > 1 && wv == 0 && lane == 0) m_l2s[out_slot] = log2S;
                 }
+#pragma unroll
+                for (int f = 0; f < FB; ++f) {
+                    // maximum over the family's four lanes fl, fl+16, fl+32,
+                    // fl+48 (the one-wave kernels use lane swaps; the 4-tile
+                    // multi-wave shapes keep shuffles, which leave them the
+                    // registers for two waves per SIMD)
+                    float m = wmax[f];
+                    if constexpr (W == 1) {
+                        m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(
+                                                                   __builtin_bit_cast(int, m), kSwizzleXor16)));
+                        m = xor32_max(m);
+                    } else {
+                        m = fmaxf(m, __shfl_xor(m, 16));
+                        m = fmaxf(m, __shfl_xor(m, 32));
+                    }
+                    const int q = out_slot * FW + 16 * f + fl;
+                    if (W == 1) {
+                        // finish the stored vector: shift, exponent, flush
+                        // bound re-expressed relative to the new scale (it
+                        // grows by S / m, the factor by which the product
+                        // fell short of its nominal scale)
+                        int e = 0;
+                        const float mant = m > 0.f ? frexpf(m, &e) : 1.f;
+                        if (g == 0) {
+                            m_bsh[q] = a_exp - e;
+                            m_esum[q] = e_sum[f] + e - a_exp;
+                            m_cert[q] = m > 0.f ? (ldexp(cert[f] * 1.01, log2S - e) + ldexp(kTau32, -e)) *
+                                                      rcp_up(mant)
+                                                : 1e300;
+                        }
+                    } else {
+                        if (g == 0) m_wmax[(out_slot * W + wv) * FW + 16 * f + fl] = m;
+                        if (wv == 0 && g == 0) {
+                            m_esum[q] = e_sum[f];
+                            m_cert[q] = cert[f];
+                        }
+                    }
+                }
+                if (W > 1 && wv == 0 && lane == 0) m_l2s[out_slot] = log2S;
                 // the node's vector is complete before anyone reads it (one
                 // wave: LDS keeps its own order, only the compiler must not
                 // move accesses across)
@@ -639,7 +577,7 @@ void k_prune_mfma(PruneParams p)
                         if (j < 0 || j >= bk.R) continue;
                         const double xv = (double)acc[f][i][r];
                         if (p.root_out && valid[f])
-                            p.root_out[(long long)dst[f] * p.root_stride + j] = SCALED ? ldexp(xv, e_sum[f]) : xv;
+                            p.root_out[(long long)dst[f] * p.root_stride + j] = ldexp(xv, e_sum[f]);
                         root_take(rb[f], xv * pv[i][r], xv, j);
                     }
                 }
@@ -667,30 +605,22 @@ void k_prune_mfma(PruneParams p)
                 for (int f = 0; f < FB; ++f) {
                     double val;
                     int flag = 0;
-                    if (SCALED) {
-                        // rb.key = x_j * prior_j in units of 2^e_sum
-                        if (!(rb[f].key > 0)) {
-                            flag = kFlagRecompute64;
-                            val = 0.0;
-                        } else {
-                            const double log_scale = (double)e_sum[f] * kLn2;
-                            if (p.model == 0)
-                                val = log(rb[f].x) + log(p.prior64[bk.prior_off + rb[f].j]) + log_scale;
-                            else
-                                val = ldexp(rb[f].key, e_sum[f]);
-                            // flush bound (absolute, in units of 2^e_sum) against
-                            // the likelihood, and FP64 range of the unscaled values
-                            const double bound = (ldexp(cert[f], log2S) + kTau32) * 1.01;
-                            if (!(bound <= kCertEta * rb[f].key)) flag |= kFlagRecompute64;
-                            if (!(log(rb[f].xmax) + log_scale >= log(kFp64Floor))) flag |= kFlagRecompute64;
-                            if (!(log(rb[f].key) + log_scale >= log(kFp64Floor))) flag |= kFlagRecompute64;
-                        }
+                    // rb.key = x_j * prior_j in units of 2^e_sum
+                    if (!(rb[f].key > 0)) {
+                        flag = kFlagRecompute64;
+                        val = 0.0;
                     } else {
-                        // base: log(x_j prior_j) at the best j (base_model.cpp:86
-                        // takes log x_j + log prior_j); gamma: x_j prior_j
-                        val = p.model == 0 ? log(rb[f].key) : rb[f].key;
-                        if (rb[f].xmax == 0.0) flag |= kFlagZeroSum;
-                        if (rb[f].xmax < kFp64Floor || rb[f].key < kFp64Floor) flag |= kFlagRecomputePlain;
+                        const double log_scale = (double)e_sum[f] * kLn2;
+                        if (p.model == 0)
+                            val = log(rb[f].x) + log(p.prior64[bk.prior_off + rb[f].j]) + log_scale;
+                        else
+                            val = ldexp(rb[f].key, e_sum[f]);
+                        // flush bound (absolute, in units of 2^e_sum) against
+                        // the likelihood, and FP64 range of the unscaled values
+                        const double bound = (ldexp(cert[f], log2S) + kTau32) * 1.01;
+                        if (!(bound <= kCertEta * rb[f].key)) flag |= kFlagRecompute64;
+                        if (!(log(rb[f].xmax) + log_scale >= log(kFp64Floor))) flag |= kFlagRecompute64;
+                        if (!(log(rb[f].key) + log_scale >= log(kFp64Floor))) flag |= kFlagRecompute64;
                     }
                     if (valid[f] && g == 0) {
                         p.out_val[(long long)td.point * p.F + dst[f]] = val;
@@ -731,50 +661,45 @@ void k_prune_mfma(PruneParams p)
 // ---------------------------------------------------------------------------
 // The kernel shapes (tiles per wave, waves per workgroup, partials in LDS);
 // (3|4, 16) cover vectors of up to 64 tiles (1024 rows) in one pass.
-#define CAFE_MFMA_SHAPES(X, T, S) \
-    X(T, 1, 1, S, true) X(T, 1, 1, S, false) X(T, 2, 1, S, true) X(T, 2, 1, S, false) \
-    X(T, 3, 1, S, true) X(T, 3, 1, S, false) X(T, 4, 1, S, true) X(T, 4, 1, S, false) \
-    X(T, 3, 2, S, true) X(T, 3, 2, S, false) X(T, 4, 2, S, true) X(T, 4, 2, S, false) \
-    X(T, 3, 4, S, true) X(T, 3, 4, S, false) X(T, 4, 4, S, true) X(T, 4, 4, S, false) \
-    X(T, 3, 8, S, false) X(T, 4, 8, S, false)
-#define CAFE_MFMA_WIDE(X, T, S) X(T, 3, 16, S, false) X(T, 4, 16, S, false)
+#define CAFE_MFMA_SHAPES(X) \
+    X(1, 1, true) X(1, 1, false) X(2, 1, true) X(2, 1, false) \
+    X(3, 1, true) X(3, 1, false) X(4, 1, true) X(4, 1, false) \
+    X(3, 2, true) X(3, 2, false) X(4, 2, true) X(4, 2, false) \
+    X(3, 4, true) X(3, 4, false) X(4, 4, true) X(4, 4, false) \
+    X(3, 8, false) X(4, 8, false)
+#define CAFE_MFMA_WIDE(X) X(3, 16, false) X(4, 16, false)
 // Latency shapes: one or two output tiles per wave, so that one family
-// tile's chain of steps is as short as the workgroup allows (the FP64
-// recompute's few tiles; FP32 classes with fewer tiles than resident slots)
-#define CAFE_MFMA_CHAIN(X, T, S) \
-    X(T, 1, 4, S, true) X(T, 1, 4, S, false) X(T, 1, 8, S, true) X(T, 1, 8, S, false) X(T, 2, 8, S, true) \
-    X(T, 2, 8, S, false) X(T, 2, 16, S, false) X(T, 1, 16, S, true) X(T, 1, 16, S, false)
+// tile's chain of steps is as short as the workgroup allows (classes with
+// fewer tiles than resident slots)
+#define CAFE_MFMA_CHAIN(X) \
+    X(1, 4, true) X(1, 4, false) X(1, 8, true) X(1, 8, false) X(2, 8, true) \
+    X(2, 8, false) X(2, 16, false) X(1, 16, true) X(1, 16, false)
 
-// 32-family tiles (FP32 only: a leaf step's two columns use both prefetch
-// buffers) for vectors of up to 32 tiles, whose k-loops stream their
+// 32-family tiles (a leaf step's two columns use both prefetch buffers) for vectors of up to 32 tiles, whose k-loops stream their
 // matrices.  Two output tiles per wave and block hold ~190 VGPRs, four would
 // spill; sixteen waves of two (the 17-32-tile vectors) are capped at 128
 // VGPRs and keep ~30 values in scratch.
-#define CAFE_MFMA_FB2(X, T, S) \
-    X(T, 2, 4, S, true) X(T, 2, 4, S, false) X(T, 1, 8, S, true) X(T, 1, 8, S, false) X(T, 2, 8, S, true) \
-    X(T, 2, 8, S, false) X(T, 1, 16, S, false) X(T, 2, 16, S, false)
+#define CAFE_MFMA_FB2(X) \
+    X(2, 4, true) X(2, 4, false) X(1, 8, true) X(1, 8, false) X(2, 8, true) \
+    X(2, 8, false) X(1, 16, false) X(2, 16, false)
 
 // One instance per shape; with per_cu set, reports how many workgroups of it
 // fit on one CU instead of launching.
-template <typename T, bool SCALED>
 static hipError_t shape_dispatch(const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st, int* per_cu)
 {
-#define CAFE_MFMA_CASE_FB(T_, NTW, W, S_, LDSP, FB)                                                          \
+#define CAFE_MFMA_CASE_FB(NTW, W, LDSP, FB)                                                                  \
     if (s.ntw == NTW && s.w == W && s.lds == LDSP && s.fb == FB) {                                          \
         if (per_cu)                                                                                         \
-            return hipOccupancyMaxActiveBlocksPerMultiprocessor(                                            \
-                per_cu, k_prune_mfma<T, NTW, W, SCALED, LDSP, FB>, 64 * W, s.shm);                          \
-        hipLaunchKernelGGL((k_prune_mfma<T, NTW, W, SCALED, LDSP, FB>), dim3(grid), dim3(64 * W), s.shm, st, p); \
+            return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, k_prune_mfma<NTW, W, LDSP, FB>, 64 * W, s.shm); \
+        hipLaunchKernelGGL((k_prune_mfma<NTW, W, LDSP, FB>), dim3(grid), dim3(64 * W), s.shm, st, p);       \
         return hipGetLastError();                                                                           \
     }
-#define CAFE_MFMA_CASE(T_, NTW, W, S_, LDSP) CAFE_MFMA_CASE_FB(T_, NTW, W, S_, LDSP, 1)
-#define CAFE_MFMA_CASE2(T_, NTW, W, S_, LDSP) CAFE_MFMA_CASE_FB(T_, NTW, W, S_, LDSP, 2)
-    CAFE_MFMA_SHAPES(CAFE_MFMA_CASE, T, SCALED)
-    CAFE_MFMA_WIDE(CAFE_MFMA_CASE, T, SCALED)
-    CAFE_MFMA_CHAIN(CAFE_MFMA_CASE, T, SCALED)
-    if constexpr (sizeof(T) == 4) {
-        CAFE_MFMA_FB2(CAFE_MFMA_CASE2, T, SCALED)
-    }
+#define CAFE_MFMA_CASE(NTW, W, LDSP) CAFE_MFMA_CASE_FB(NTW, W, LDSP, 1)
+#define CAFE_MFMA_CASE2(NTW, W, LDSP) CAFE_MFMA_CASE_FB(NTW, W, LDSP, 2)
+    CAFE_MFMA_SHAPES(CAFE_MFMA_CASE)
+    CAFE_MFMA_WIDE(CAFE_MFMA_CASE)
+    CAFE_MFMA_CHAIN(CAFE_MFMA_CASE)
+    CAFE_MFMA_FB2(CAFE_MFMA_CASE2)
 #undef CAFE_MFMA_CASE2
 #undef CAFE_MFMA_CASE
 #undef CAFE_MFMA_CASE_FB
@@ -785,19 +710,17 @@ static hipError_t shape_dispatch(const MfmaShape& s, int grid, const PruneParams
 // launch can size its grid to what is resident: the static tile split gives
 // every workgroup an equal share, and a workgroup that has to wait for a
 // slot would finish its share after all the others.
-hipError_t mfma_occupancy(bool fp64, const MfmaShape& s, int* per_cu)
+hipError_t mfma_occupancy(const MfmaShape& s, int* per_cu)
 {
     *per_cu = 0;
     const PruneParams none{};
-    return fp64 ? shape_dispatch<double, false>(s, 0, none, nullptr, per_cu)
-                : shape_dispatch<float, true>(s, 0, none, nullptr, per_cu);
+    return shape_dispatch(s, 0, none, nullptr, per_cu);
 }
 
-hipError_t launch_prune_mfma(bool fp64, const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st)
+hipError_t launch_prune_mfma(const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st)
 {
     if (grid < 1) grid = 1;
-    return fp64 ? shape_dispatch<double, false>(s, grid, p, st, nullptr)
-                : shape_dispatch<float, true>(s, grid, p, st, nullptr);
+    return shape_dispatch(s, grid, p, st, nullptr);
 }
 
 }  // namespace cafe

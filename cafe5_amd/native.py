@@ -324,10 +324,11 @@ class Plan:
     def class_times(self):
         """Per size class of the main pass, from the last profile() run:
         (16-row tiles per vector, tiles, kernel ms, launch) arrays; launch
-        rows are (kernel: 0 matrix-core, 1 one family per lane, 2 PLAIN64,
-        3 split-FP16; tiles per wave or rows per lane; waves per workgroup;
-        partials in LDS; workgroups; families per tile: 16 or 32 for the
-        matrix-core kernel, 64 per lane)."""
+        rows are (kernel: 0 matrix-core, 1 one family per lane, 2 the FP64
+        kernel on PLAIN64 and for vectors over 1,024 rows, 3 split-FP16; tiles
+        per wave, or rows per lane; waves per workgroup; partials in LDS;
+        workgroups; families per tile: 16 or 32 for the matrix-core kernels,
+        64 per lane)."""
         n = ctypes.c_int(0)
         self.eng._check(self.lib.cafe_gpu_plan_class_times(self.h, 0, ctypes.byref(n), None, None, None, None))
         nt = np.zeros(n.value, dtype=np.int32)
@@ -339,7 +340,8 @@ class Plan:
         return nt, tiles, ms, launch
 
     def recompute_counts(self):
-        """(families redone on BATCHED64, families redone on PLAIN64)."""
+        """(families redone in FP64, families with FP64 values near the subnormal
+        range)."""
         a, b = ctypes.c_longlong(0), ctypes.c_longlong(0)
         self.eng._check(self.lib.cafe_gpu_plan_recompute_counts(self.h, ctypes.byref(a), ctypes.byref(b)))
         return a.value, b.value

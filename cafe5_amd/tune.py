@@ -40,6 +40,9 @@ F16_SHAPES = [s for s in MFMA_SHAPES[:12] if s[1] <= 8]
 # partials only
 FB2_SHAPES = [(2, 4), (1, 8), (2, 8), (1, 16), (2, 16)]
 FB2_MAX_TILES = 32
+# the FP64 kernel's instances with 16-family tiles (tiles per wave, partials in
+# LDS); its rule takes 32-family ones where they pay
+F64_SHAPES = [(1, 1), (1, 0), (2, 0)]
 LANE_TILES = 3          # the per-lane kernel takes vectors of up to 33 rows (3 tiles)
 MAX_SHAPE_TILES = 64    # the matrix-core shapes' largest vectors (1,024 rows)
 
@@ -47,6 +50,12 @@ MAX_SHAPE_TILES = 64    # the matrix-core shapes' largest vectors (1,024 rows)
 def candidates(path: int, nt: int) -> List[Tuple[int, int, int, int, int]]:
     """(kernel, ntw, w, lds, grid_mult) candidates for a class of nt tiles."""
     out = []
+    if path == native.PATH_BATCHED64:   # the FP64 kernel's instances that cover the class in one pass
+        for ntw, lds in F64_SHAPES:
+            w = (nt + ntw - 1) // ntw
+            if w <= 16:
+                out += [(0, ntw, w, lds, gm) for gm in ((4, 8, 16) if lds else (1, 2, 4))]
+        return out
     if path in (native.PATH_BATCHED32, native.PATH_BATCHED16) and nt <= LANE_TILES:
         for gm in (8, 16, 32):
             out.append((1, 0, 0, 0, gm))
@@ -71,7 +80,7 @@ def candidates(path: int, nt: int) -> List[Tuple[int, int, int, int, int]]:
 
 def plan_key_of(nts) -> str:
     """The plan= key of a plan's size classes: their tiles per vector, up to
-    64 (classes of larger vectors run the plain FP64 kernel, which has no
+    64 (classes of larger vectors run the FP64 kernel on every path, with no
     launch shape to tune and no place in the engine's key)."""
     return ",".join(str(int(n)) for n in sorted(nts) if int(n) <= MAX_SHAPE_TILES)
 

@@ -55,16 +55,19 @@ enum {
 
 /* Pruning paths. */
 enum {
-    /* per-family FP64 matrix-vector products in the reference's summation
-     * order (the drop-in); no rescaling */
+    /* FP64 in the reference's summation order (the drop-in): families as
+     * columns of FP64 MFMA contractions whose sums run over ascending sizes,
+     * each term one fused multiply-add; no rescaling */
     CAFE_GPU_PATH_PLAIN64 = 0,
-    /* families as columns, FP64 MFMA contractions; no rescaling */
+    /* the same kernel and values, in the size classes of the reduced paths
+     * (tunable launch shapes), counting the families whose values come near
+     * the subnormal range */
     CAFE_GPU_PATH_BATCHED64 = 1,
     /* families as columns, FP32 MFMA contractions with per-family
      * power-of-two rescaling and an exponent carry; each family gets a bound
      * on what FP32 flushing could have lost, and families whose bound is not
      * below 1e-9 of their likelihood (or whose FP64 value would be
-     * subnormal) are recomputed on the BATCHED64 path */
+     * subnormal) are recomputed on the FP64 kernel */
     CAFE_GPU_PATH_BATCHED32 = 2,
     /* families as columns, split-FP16 MFMA contractions (each operand as two
      * FP16 halves, three products with FP32 accumulation, about FP32
@@ -72,7 +75,7 @@ enum {
      * exponent carry; every partial vector carries a per-entry bound on what
      * FP16's narrow range can lose, propagated by a fourth MFMA, and families
      * whose bound is not below 1e-9 of their likelihood are recomputed on the
-     * BATCHED64 path.  Vectors of at most 33 rows run the FP32 per-lane
+     * FP64 kernel.  Vectors of at most 33 rows run the FP32 per-lane
      * kernel of BATCHED32 (no matrix-core work there). */
     CAFE_GPU_PATH_BATCHED16 = 3
 };
@@ -98,8 +101,8 @@ const char *cafe_gpu_last_error(void);
  * dimension N = max(R, B) + 1 and the pool capacity in matrices; drops all
  * built matrices.  2 <= N <= 2047 (the log-gamma table holds 0..4095).  On
  * every path, size classes whose vectors exceed 1,024 rows (64 tiles of 16)
- * run their main pass on the PLAIN64 kernel (final FP64 values, the
- * reference's summation order), the role of the reference's heap-allocated
+ * run their main pass on the FP64 kernel (final values in the reference's
+ * summation order), the role of the reference's heap-allocated
  * path for large families (src/probability.cpp:239-310). */
 int cafe_gpu_matrix_reset(cafe_gpu_ctx *ctx, int N, int capacity);
 
@@ -165,7 +168,8 @@ typedef struct {
  *                           gamma_core.cpp:102)
  *   total[t]                -sum_f lnl (compensated sum), +inf when any
  *                           gamma family has a zero-sum root vector
- *   n_fallback              families recomputed on the FP64 path (BATCHED32)
+ *   n_fallback              families recomputed in FP64, plus those whose FP64
+ *                           values are near the subnormal range
  */
 int cafe_gpu_eval(cafe_gpu_ctx *ctx, const cafe_gpu_eval_desc *desc, double *lnl,
                   double *cat, double *post, double *total, long long *n_fallback);
@@ -239,9 +243,10 @@ int cafe_gpu_plan_results(cafe_gpu_plan *plan, double *lnl, double *cat, double 
  * [0] matrix build, [1] main prune, [2] recompute passes, [3] finalize.
  * *graph_ok = 1 when plan_execute replays a captured graph. */
 int cafe_gpu_plan_profile(cafe_gpu_plan *plan, double *ms4, int *graph_ok);
-/* Families of the last execution recomputed on BATCHED64 (FP32 results the
- * flush bound did not certify) and on PLAIN64 (FP64 values near the
- * subnormal range, redone in the reference's summation order). */
+/* Families of the last execution recomputed in FP64 (results of a reduced
+ * path its bound did not certify), and families of BATCHED64 or of that
+ * recompute whose FP64 values are near the subnormal range (below 1e-290;
+ * they are in the reference's summation order as they are). */
 int cafe_gpu_plan_recompute_counts(cafe_gpu_plan *plan, long long *fp64, long long *plain);
 /* Per size class of the main pruning pass, from the last
  * cafe_gpu_plan_profile run (no reference counterpart; measurement): the
@@ -249,10 +254,11 @@ int cafe_gpu_plan_recompute_counts(cafe_gpu_plan *plan, long long *fp64, long lo
  * families per tile given in launch) and the milliseconds of its kernel
  * launch (HIP events on the context stream),
  * and, in launch[6 i .. 6 i + 5], that launch's shape: kernel (0 matrix-core
- * k_prune_mfma, 1 one-family-per-lane k_prune_lane, 2 PLAIN64 k_prune_plain),
- * 16-row tiles per wave (lane and PLAIN64 kernels: rows per lane), waves per
- * workgroup, partial vectors in LDS (0/1), workgroups, and families per tile
- * (matrix-core kernel: 16, or 32 with two 16-family blocks per operand).
+ * k_prune_mfma, or k_prune_f64 on BATCHED64; 1 one-family-per-lane
+ * k_prune_lane; 2 k_prune_f64 on PLAIN64 and for vectors over 1,024 rows),
+ * 16-row tiles per wave (lane kernel: rows per lane), waves per workgroup,
+ * partial vectors in LDS (0/1), workgroups, and families per tile
+ * (matrix-core kernels: 16, or 32 with two 16-family blocks per operand).
  * Writes at most cap entries (any output may be null); *n_classes is the
  * number of classes. */
 int cafe_gpu_plan_class_times(cafe_gpu_plan *plan, int cap, int *n_classes, int *class_nt,
@@ -263,8 +269,9 @@ int cafe_gpu_plan_destroy(cafe_gpu_plan *plan);
  * Plans and evaluations pick a launch shape for every size class (the
  * buckets whose vectors have the same number of 16-row tiles): the
  * one-family-per-lane kernel or the matrix-core kernel, and for the latter
- * its families per tile (16, or 32 for the FP32 kernel on vectors of up to 32
- * tiles: each matrix operand then feeds two 16-family blocks), output tiles
+ * its families per tile (16, or 32 for the FP64 kernel and for the FP32 kernel
+ * on vectors of up to 32 tiles: each matrix operand then feeds two 16-family
+ * blocks), output tiles
  * per wave, waves per workgroup, partials in LDS or global scratch, and the
  * grid (workgroups per resident slot).  The context holds a
  * table of measured choices keyed by (path, tiles per vector, leaves of the
