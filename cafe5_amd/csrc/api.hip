@@ -23,10 +23,13 @@ hipError_t launch_build(int algo, const double* d_lam, const double* d_t, const 
                         int first_slot, int N, int Np, long long slot_elems, double* mt64, float* mt32,
                         float* lf32, hipStream_t stream, const unsigned char* copies, int top, int* band);
 hipError_t launch_fill_zero(void* p, long long bytes, hipStream_t stream);
-hipError_t launch_reconstruct(const ReconNode* nodes, int n_nodes, const int* kids, const int* parent,
-                              const double* mt64, int N, int Np, long long slot_elems, const int* counts_T, int F,
-                              const int* fam_sorted, int nf, const double* prior, int B, int Rr, double* L_all,
-                              int* C_all, double* prod_all, int Lp, int* states, int* err, hipStream_t st);
+size_t recon_table_doubles(int n_prog, int Lp);
+hipError_t launch_block_max(const ReconNode* nodes, int n_prog, const double* mt64, int Np, long long slot_elems,
+                            int Lp, double* tab, hipStream_t st);
+hipError_t launch_reconstruct(const ReconNode* nodes, int n_prog, const ReconKid* kids, const double* mt64, int N,
+                              int Np, long long slot_elems, const double* tab, const int* counts_T, int F,
+                              const int2* fams, int nf, const double* prior, int B, int Rr, double* L_all, int Lp,
+                              int n_nodes, int* states, int* err, hipStream_t st);
 hipError_t launch_fold(const double* mt64, const float* lf32, double* out64, float* out32, const double* err64,
                        const float* err32, int n_dev, int n_rows, int N, int Np, long long slot_elems,
                        int first_slot, int n, hipStream_t stream);
@@ -170,6 +173,7 @@ struct cafe_gpu_ctx {
     // families
     int F = 0, n_leaves = 0;
     std::vector<int> perm;
+    std::vector<int> fam_max;   // per family of the caller: its largest count
     std::vector<BucketHost> buckets;
     DevBuf d_counts, d_perm;
 
@@ -598,7 +602,7 @@ int cafe_gpu_set_families(cafe_gpu_ctx* ctx, int F, int n_leaves, const int* cou
 {
     if (int rc = check_ctx(ctx)) return rc;
     if (F < 1 || n_leaves < 1 || !counts) return fail(CAFE_GPU_EINVAL, "need at least one family and leaf");
-    std::vector<int> fb(F), fr(F);
+    std::vector<int> fb(F), fr(F), top(F, 0);
     for (int f = 0; f < F; ++f) {
         fb[f] = bound_B ? bound_B[f] : B;
         fr[f] = bound_R ? bound_R[f] : R;
@@ -607,6 +611,7 @@ int cafe_gpu_set_families(cafe_gpu_ctx* ctx, int F, int n_leaves, const int* cou
             const int c = counts[(size_t)f * n_leaves + i];
             if (c < 0 || c > fb[f])
                 return fail(CAFE_GPU_EINVAL, "family %d leaf %d count %d outside 0..%d", f, i, c, fb[f]);
+            top[f] = std::max(top[f], c);
         }
     }
     std::vector<int> order(F);
@@ -621,7 +626,7 @@ int cafe_gpu_set_families(cafe_gpu_ctx* ctx, int F, int n_leaves, const int* cou
             ctx->buckets.push_back(BucketHost{fb[f], fr[f], 0, k, 0});
         auto& b = ctx->buckets.back();
         b.count++;
-        for (int i = 0; i < n_leaves; ++i) b.max_count = std::max(b.max_count, counts[(size_t)f * n_leaves + i]);
+        b.max_count = std::max(b.max_count, top[f]);
     }
     ctx->input_gen++;
     std::vector<int> cT((size_t)n_leaves * F);
@@ -632,6 +637,7 @@ int cafe_gpu_set_families(cafe_gpu_ctx* ctx, int F, int n_leaves, const int* cou
     HIP_OR_FAIL(hipMemcpy(ctx->d_counts.p, cT.data(), sizeof(int) * cT.size(), hipMemcpyHostToDevice));
     HIP_OR_FAIL(hipMemcpy(ctx->d_perm.p, order.data(), sizeof(int) * F, hipMemcpyHostToDevice));
     ctx->perm = order;
+    ctx->fam_max = top;
     ctx->F = F;
     ctx->n_leaves = n_leaves;
     return CAFE_GPU_OK;
@@ -1511,12 +1517,12 @@ double elapsed_ms(hipEvent_t a, hipEvent_t b)
 }
 
 // Pupko reconstruction of families f0 .. f0+nf-1 (cafe_gpu_reconstruct).  The
-// device working memory -- program, child lists, parents, prior, a launch's
-// family list, its state rows and the two error flags, then per family the
-// L, C and product rows -- comes from the context's grow-only buffers when
-// `fixed` is null, else from the fixed region [fixed, fixed + fixed_bytes),
-// in which case nothing is allocated: launches are sized to fit the region
-// and a family that does not fit on its own is rejected.
+// device working memory -- program, child lists, prior, the resident families'
+// list and state rows, the error flag, the table of block maxima and then per
+// family of a launch the L rows -- comes from the context's grow-only buffers
+// when `fixed` is null, else from the fixed region [fixed, fixed +
+// fixed_bytes), in which case nothing is allocated: launches are sized to fit
+// the region and a family that does not fit on its own is rejected.
 int reconstruct_impl(cafe_gpu_ctx* ctx, const int* node_slot, const double* prior, int B, int R, int f0, int nf,
                      int* states, char* fixed, size_t fixed_bytes)
 {
@@ -1532,31 +1538,23 @@ int reconstruct_impl(cafe_gpu_ctx* ctx, const int* node_slot, const double* prio
     const int n = ctx->n_nodes;
     const int Rr = std::min(B, R) + 1;   // gene_family_reconstructor.cpp:149-151
     const int Lp = B + 1;
-    // device layout: program | kids | parent | prior | families | states | flags,
-    // then the per-family L, product and C rows (the program has one record
-    // per node, the child lists one entry per non-root node)
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t fam_bytes = (size_t)Lp * ((size_t)n * (sizeof(double) + sizeof(int)) + sizeof(double));
-    const size_t o_kids = up(sizeof(ReconNode) * n);
-    const size_t o_par = o_kids + up(sizeof(int) * std::max(1, n - 1));
-    const size_t o_pri = o_par + up(sizeof(int) * n);
-    const size_t o_fam = o_pri + up(sizeof(double) * Rr);
-    // families per launch: enough workgroups to fill the device several times
-    // over, with the per-family scratch within 2 GB (or within the fixed region)
-    size_t cap = std::min<size_t>(8192, std::max<size_t>(64, ((size_t)2 << 30) / fam_bytes));
     if (fixed) {
-        // o_fam + up(4 c) + up(4 c n) + 256 + c fam_bytes <= fixed_bytes
-        const size_t per = sizeof(int) + sizeof(int) * (size_t)n + fam_bytes;
-        const size_t head = o_fam + 3 * 256 + 256;
-        const size_t fit = fixed_bytes > head ? (fixed_bytes - head) / per : 0;
-        if (fit < 1)
+        // the documented limit: a family's rows at 12 bytes per node and size,
+        // its list entry and states, and 28 bytes of program per node (what is
+        // laid out below stays under it)
+        const size_t per = sizeof(int) + sizeof(int) * (size_t)n +
+                           (size_t)Lp * ((size_t)n * (sizeof(double) + sizeof(int)) + sizeof(double));
+        const size_t head = up((size_t)20 * n) + up(sizeof(int) * std::max(1, n - 1)) + up(sizeof(int) * n) +
+                            up(sizeof(double) * Rr) + 4 * 256;
+        if (fixed_bytes <= head || (fixed_bytes - head) / per < 1)
             return fail(CAFE_GPU_EINVAL,
                         "one family of %d nodes with vectors of %d sizes needs %zu bytes of scratch; the fixed "
                         "scratch holds %zu",
                         n, Lp, head + per, fixed_bytes);
-        cap = std::min(cap, fit);
     }
-    // children first (depth first, children in increasing index)
+    // the interior nodes, children first (depth first, children in increasing
+    // index)
     std::vector<std::vector<int>> kids(n);
     int root = -1;
     for (int i = 0; i < n; ++i) {
@@ -1564,7 +1562,8 @@ int reconstruct_impl(cafe_gpu_ctx* ctx, const int* node_slot, const double* prio
         else kids[ctx->parent_h[i]].push_back(i);
     }
     std::vector<ReconNode> prog;
-    std::vector<int> kid_list;
+    std::vector<ReconKid> kid_list;
+    std::vector<int> place(n, -1);
     std::vector<std::pair<int, int>> stack{{root, 0}};
     while (!stack.empty()) {
         auto& top = stack.back();
@@ -1574,68 +1573,104 @@ int reconstruct_impl(cafe_gpu_ctx* ctx, const int* node_slot, const double* prio
             continue;
         }
         stack.pop_back();
-        ReconNode nd{u, ctx->leaf_col_h[u], (int)kid_list.size(), (int)kids[u].size(), -1};
-        for (int c : kids[u]) kid_list.push_back(c);
+        int slot = -1;
         if (u != root) {
-            nd.slot = node_slot[u];
-            if (nd.slot < 0 || nd.slot >= ctx->capacity)
-                return fail(CAFE_GPU_EINVAL, "node %d: matrix slot %d outside the pool", u, nd.slot);
-            if (!ctx->built[nd.slot])   // matrix_cache::get_matrix throws on a miss (matrix_cache.cpp:88-104)
-                return fail(CAFE_GPU_ENOTFOUND, "node %d uses matrix slot %d, which is not built", u, nd.slot);
+            slot = node_slot[u];
+            if (slot < 0 || slot >= ctx->capacity)
+                return fail(CAFE_GPU_EINVAL, "node %d: matrix slot %d outside the pool", u, slot);
+            if (!ctx->built[slot])   // matrix_cache::get_matrix throws on a miss (matrix_cache.cpp:88-104)
+                return fail(CAFE_GPU_ENOTFOUND, "node %d uses matrix slot %d, which is not built", u, slot);
         }
-        prog.push_back(nd);
+        if (ctx->leaf_col_h[u] >= 0) continue;
+        place[u] = (int)prog.size();
+        prog.push_back(ReconNode{u, (int)kid_list.size(), (int)kids[u].size(), slot});
+        for (int c : kids[u]) {
+            const int col = ctx->leaf_col_h[c];
+            kid_list.push_back(ReconKid{col, node_slot[c], col >= 0 ? c : place[c], 0});
+        }
     }
+    if (kid_list.size() + 1 != (size_t)n)
+        return fail(CAFE_GPU_EINVAL, "reconstruction program does not cover the tree (internal)");
+    const int n_prog = (int)prog.size();
     // count-row (sorted) index of each caller family
     std::vector<int> sorted_of(ctx->F);
     for (int s = 0; s < ctx->F; ++s) sorted_of[ctx->perm[s]] = s;
-    if (prog.size() != (size_t)n || kid_list.size() + 1 != (size_t)n)
-        return fail(CAFE_GPU_EINVAL, "reconstruction program does not cover the tree (internal)");
-    const int chunk = (int)std::min<size_t>((size_t)nf, cap);
-    const size_t o_st = o_fam + up(sizeof(int) * chunk);
-    const size_t o_err = o_st + up(sizeof(int) * (size_t)chunk * n);
-    const size_t o_scr = o_err + 256;
+    // Device layout: program | kids | prior | flag | table | families | states,
+    // then the L rows.  `chunk` families run per launch (their L rows within 2
+    // GB), `held` have their list entries and states on the device at once
+    // (all of them, or the fixed region's launch).
+    const size_t o_kids = up(sizeof(ReconNode) * n_prog);
+    const size_t o_pri = o_kids + up(sizeof(ReconKid) * kid_list.size());
+    const size_t o_err = o_pri + up(sizeof(double) * Rr);
+    const size_t o_tab = o_err + 256;
+    const size_t row_bytes = sizeof(double) * (size_t)(n_prog - 1) * (Lp + (Lp & 1));
+    const size_t list_bytes = sizeof(int2) + sizeof(int) * (size_t)n;
+    size_t tab_bytes = up(sizeof(double) * recon_table_doubles(n_prog, Lp));
+    size_t held = (size_t)nf, chunk;
+    if (fixed) {
+        // the table where it leaves the families half of the region (without
+        // it no block is skipped)
+        if (o_tab + tab_bytes > fixed_bytes / 2) tab_bytes = 0;
+        const size_t head = o_tab + tab_bytes + 2 * 256;
+        size_t fit = fixed_bytes > head ? (fixed_bytes - head) / (row_bytes + list_bytes) : 0;
+        if (fit >= (size_t)kRecFew) fit = fit / kRecFT * kRecFT;
+        if (fit < 1) return fail(CAFE_GPU_EINVAL, "fixed scratch layout overflows (internal)");
+        held = chunk = std::min(held, fit);
+        if (chunk % kRecFT && chunk >= (size_t)kRecFew) held = chunk = chunk / kRecFT * kRecFT;
+    } else {
+        chunk = std::max<size_t>(64, ((size_t)2 << 30) / std::max<size_t>(row_bytes, 1) / kRecFT * kRecFT);
+        chunk = std::min(chunk, (held + kRecFT - 1) / kRecFT * kRecFT);
+    }
+    const size_t o_fam = o_tab + tab_bytes;
+    const size_t o_st = o_fam + up(sizeof(int2) * held);
+    const size_t o_rows = o_st + up(sizeof(int) * held * n);
     char* base;
-    char* scr;
+    double* rows;
     if (fixed) {
         base = fixed;
-        scr = fixed + o_scr;
-        if (o_scr + (size_t)chunk * fam_bytes > fixed_bytes)
+        rows = (double*)(fixed + o_rows);
+        if (o_rows + chunk * row_bytes > fixed_bytes)
             return fail(CAFE_GPU_EINVAL, "fixed scratch layout overflows (internal)");
     } else {
-        HIP_OR_FAIL(ctx->d_recon.ensure(o_scr));
-        HIP_OR_FAIL(ctx->d_recon_scratch.ensure((size_t)chunk * fam_bytes));
+        HIP_OR_FAIL(ctx->d_recon.ensure(o_rows));
+        HIP_OR_FAIL(ctx->d_recon_scratch.ensure(std::max<size_t>(chunk * row_bytes, 256)));
         base = (char*)ctx->d_recon.p;
-        scr = (char*)ctx->d_recon_scratch.p;
+        rows = ctx->d_recon_scratch.as<double>();
     }
-    double* L_all = (double*)scr;   // doubles first: every row stays 8-byte aligned
-    double* prod_all = L_all + (size_t)chunk * n * Lp;
-    int* C_all = (int*)(prod_all + (size_t)chunk * Lp);
+    const ReconNode* d_prog = (const ReconNode*)base;
+    double* tab = tab_bytes ? (double*)(base + o_tab) : nullptr;
     hipStream_t st = ctx->stream;
     HIP_OR_FAIL(hipMemcpyAsync(base, prog.data(), sizeof(ReconNode) * prog.size(), hipMemcpyHostToDevice, st));
-    if (!kid_list.empty())
-        HIP_OR_FAIL(hipMemcpyAsync(base + o_kids, kid_list.data(), sizeof(int) * kid_list.size(), hipMemcpyHostToDevice, st));
-    HIP_OR_FAIL(hipMemcpyAsync(base + o_par, ctx->parent_h.data(), sizeof(int) * n, hipMemcpyHostToDevice, st));
+    HIP_OR_FAIL(hipMemcpyAsync(base + o_kids, kid_list.data(), sizeof(ReconKid) * kid_list.size(), hipMemcpyHostToDevice, st));
     HIP_OR_FAIL(hipMemcpyAsync(base + o_pri, prior, sizeof(double) * Rr, hipMemcpyHostToDevice, st));
-    HIP_OR_FAIL(launch_fill_zero(base + o_err, 2 * sizeof(int), st));
-    std::vector<int> fams(chunk);
-    for (int c0 = 0; c0 < nf; c0 += chunk) {
-        const int m = std::min(chunk, nf - c0);
-        for (int k = 0; k < m; ++k) fams[k] = sorted_of[f0 + c0 + k];
-        HIP_OR_FAIL(hipMemcpyAsync(base + o_fam, fams.data(), sizeof(int) * m, hipMemcpyHostToDevice, st));
-        HIP_OR_FAIL(launch_reconstruct((const ReconNode*)base, (int)prog.size(), (const int*)(base + o_kids),
-                                       (const int*)(base + o_par), ctx->mt64.as<double>(), ctx->N, ctx->Np,
-                                       ctx->slot_elems, ctx->d_counts.as<int>(), ctx->F, (const int*)(base + o_fam), m,
-                                       (const double*)(base + o_pri), B, Rr, L_all, C_all, prod_all, Lp,
-                                       (int*)(base + o_st), (int*)(base + o_err), st));
-        HIP_OR_FAIL(hipMemcpyAsync(states + (size_t)c0 * n, base + o_st, sizeof(int) * (size_t)m * n,
-                                   hipMemcpyDeviceToHost, st));
-        HIP_OR_FAIL(hipStreamSynchronize(st));   // fams and the state rows are reused by the next chunk
+    HIP_OR_FAIL(launch_fill_zero(base + o_err, sizeof(int), st));
+    if (tab)
+        HIP_OR_FAIL(launch_block_max(d_prog, n_prog, ctx->mt64.as<double>(), ctx->Np, ctx->slot_elems, Lp, tab, st));
+    // large families first: their products fall off later, so they take several
+    // times longer, and four of a size share a wave's matrix blocks
+    std::vector<int2> fams(held);
+    std::vector<int> at(ctx->N + 1);
+    for (size_t h0 = 0; h0 < (size_t)nf; h0 += held) {
+        const size_t nh = std::min(held, (size_t)nf - h0);
+        auto key = [&](size_t k) { return ctx->N - 1 - std::min(ctx->fam_max[f0 + h0 + k], ctx->N - 1); };
+        std::fill(at.begin(), at.end(), 0);
+        for (size_t k = 0; k < nh; ++k) ++at[key(k) + 1];
+        for (int i = 0; i < ctx->N; ++i) at[i + 1] += at[i];
+        for (size_t k = 0; k < nh; ++k) fams[at[key(k)]++] = int2{sorted_of[f0 + h0 + k], (int)k};
+        HIP_OR_FAIL(hipMemcpyAsync(base + o_fam, fams.data(), sizeof(int2) * nh, hipMemcpyHostToDevice, st));
+        for (size_t c0 = 0; c0 < nh; c0 += chunk)
+            HIP_OR_FAIL(launch_reconstruct(d_prog, n_prog, (const ReconKid*)(base + o_kids), ctx->mt64.as<double>(),
+                                           ctx->N, ctx->Np, ctx->slot_elems, tab, ctx->d_counts.as<int>(), ctx->F,
+                                           (const int2*)(base + o_fam) + c0, (int)std::min(chunk, nh - c0),
+                                           (const double*)(base + o_pri), B, Rr, rows, Lp, n,
+                                           (int*)(base + o_st), (int*)(base + o_err), st));
+        HIP_OR_FAIL(hipMemcpyAsync(states + h0 * n, base + o_st, sizeof(int) * nh * n, hipMemcpyDeviceToHost, st));
+        HIP_OR_FAIL(hipStreamSynchronize(st));   // fams and the state rows are used again
     }
-    int flags[2] = {0, 0};
-    HIP_OR_FAIL(hipMemcpyAsync(flags, base + o_err, sizeof(flags), hipMemcpyDeviceToHost, st));
+    int flag = 0;
+    HIP_OR_FAIL(hipMemcpyAsync(&flag, base + o_err, sizeof(flag), hipMemcpyDeviceToHost, st));
     HIP_OR_FAIL(hipStreamSynchronize(st));
-    if (flags[0]) return fail(CAFE_GPU_EINVAL, "a leaf count is outside the matrices (N = %d)", ctx->N);
-    if (flags[1]) return fail(CAFE_GPU_EINVAL, "a reconstructed state fell outside 0..%d", B);
+    if (flag) return fail(CAFE_GPU_EINVAL, "a leaf count is outside the matrices (N = %d)", ctx->N);
     return CAFE_GPU_OK;
 }
 

@@ -167,14 +167,28 @@ struct PruneParams {
     int band_stride;
 };
 
-// One node of the reconstruction program (children before parents).
+// Interior nodes of the reconstruction program, children before parents, the
+// root last; their children in increasing node order.
 struct ReconNode {
     int node;       // engine node index
-    int leaf_col;   // >= 0: a leaf's column in the count rows
     int kid0;       // first child in the program's kids list
     int n_kids;
     int slot;       // matrix slot of the branch above the node (-1: root)
 };
+struct ReconKid {
+    int leaf_col;   // >= 0: a leaf's column in the count rows
+    int slot;       // matrix slot of its branch
+    int ref;        // leaf: engine node index; interior: its place in the program
+    int pad;
+};
+// Families per wave of the reconstruction: four share a matrix block (5,000
+// of 60 taxa at B = 320: 5.0 ms against 5.8 with one per wave).  Few families
+// leave SIMDs idle, one per wave spreads them (300 of 12 taxa: 161 us against
+// 203; 1,000 of 34 taxa: 1,658 against 1,482), and longer vectors' products
+// would leave a CU a few waves' LDS.
+constexpr int kRecFT = 4;
+constexpr int kRecFew = 512;
+constexpr int kRecMaxShared = 512;
 
 // Launch shape of the MFMA pruning kernel: ntw 16-row output tiles per wave,
 // w waves per workgroup, partial vectors in LDS or global scratch, dynamic

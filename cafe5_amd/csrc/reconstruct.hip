@@ -2,294 +2,340 @@
 // (replaces pupko_reconstructor::reconstruct_gene_family and its node steps,
 // src/gene_family_reconstructor.cpp:30-189).
 //
-// One wave per family.  Nodes run children first; for every node the wave
-// keeps, per parent size i (lanes over i), the best child-size value
-//     L[i] = max_j  (prod_children L_child[j]) * M[i][j]
-// and its argmax C[i] (the first j reaching the maximum, as the reference's
-// strict ">" scan from j = 0 keeps it).  The product over children is formed
-// once per j in the reference's order (1.0 times each child's entry in
-// descendant order) and then multiplied by the matrix entry, so every value
-// and every comparison is the reference's, bit for bit.  Leaves hold column
-// `count` of their matrix.  The root scans j = 1..Rr-1 against the prior
-// (root_equilibrium_distribution::compute(j)) and keeps its argmax as the
-// root's state; the wave's first lane then walks the tree parents-first and
-// reads each interior node's state from C at its parent's state.
+// Up the tree (children first) a node's row over parent sizes i is
+//     L[i] = max_j  (prod_children L_child[j]) * M[i][j],
+// with the product formed in the reference's order (1.0 times each child's
+// entry in descendant order; a leaf's row is column `count` of its matrix).
+// The reference also keeps the first j that reaches each maximum; of those a
+// family needs one per node, the one at its parent's state, so it is looked up
+// on the way down: the first j whose value equals L[i].  Values and
+// comparisons are the reference's, bit for bit, so the states are.  The root
+// takes the first best j = 1..Rr-1 of the product times the prior
+// (root_equilibrium_distribution::compute(j)).
 //
-// The matrix-vector work is max-times, not a sum of products, so it runs on
-// the vector units (FP64), with the matrix column j read coalesced across the
-// lanes (c-major FP64 pool: entry (i, j) at j * Np + i).
+// The contraction is a max of products, so it runs on the vector units: two
+// neighbouring parent sizes per lane (one 16-byte load per child size), FT
+// families per wave, a matrix block of kRecJB child sizes by 128 parent sizes
+// in registers for all of them, the products broadcast from LDS.  A block is
+// skipped where (its largest product) x (the largest matrix entry of the two
+// rows in it) exceeds no row's maximum so far: rounding is monotonic, so no
+// value of it could.  The products fall off past the family's own sizes;
+// 20,000 families of 34 taxa at B = 200 keep a quarter of their blocks.
+//
+// Bound by: the vector units half of the time (670 M instructions), the rest
+// latency of the matrix blocks (16 loads each) with three waves per SIMD, and
+// 1 GB of rows written and read again.  20,000 families of 34 taxa at B = 200:
+// 2.4 ms, against 17.4 ms for one family per wave with every block taken, the
+// argmax kept along and the matrix through LDS.  Blocks of 8 halve the
+// registers but double the tests (3.0 ms), loading a block ahead costs a wave
+// per SIMD (3.4 ms), one row per lane doubles the loads (3.5 ms).
 #include <algorithm>
 
 #include "engine.h"
+#include "prune_common.h"
 
 namespace cafe {
 
-// Families fam_sorted[0 .. nf-1] (count-row order), one per workgroup; L, C
-// and the children's product in per-family scratch rows of Lp entries.
-// err[0]: a count outside the matrix, err[1]: a parent state outside a node's
-// rows (plain stores of 1; any family may set them).
-__global__ __launch_bounds__(64) void k_reconstruct(const ReconNode* __restrict__ nodes, int n_nodes,
-                                                    const int* __restrict__ kids, const int* __restrict__ parent,
+constexpr int kRecJB = 16;   // child sizes per block
+typedef double d2 __attribute__((ext_vector_type(2)));
+
+// The largest entry of every pair of rows in every block of child sizes:
+// tab[(node, block)][i / 2] for the interior branches of the program.
+__global__ __launch_bounds__(256) void k_block_max(const ReconNode* __restrict__ nodes, const double* __restrict__ mt64,
+                                                   int Np, long long slot_elems, int Lq, double* __restrict__ tab)
+{
+    const int h = blockIdx.x * 256 + threadIdx.x;
+    if (2 * h >= Lq) return;
+    const int J = blockIdx.y, s = blockIdx.z;
+    const double* M = mt64 + (long long)nodes[s].slot * slot_elems + (long long)J * kRecJB * Np + 2 * h;
+    double m = 0.0;
+#pragma unroll
+    for (int jj = 0; jj < kRecJB; ++jj) {   // (rows and columns past N are 0)
+        const d2 v = *(const d2*)(M + (long long)jj * Np);
+        m = fmax(m, fmax(v[0], v[1]));
+    }
+    tab[((long long)s * gridDim.y + J) * (Lq / 2) + h] = m;
+}
+
+// max over kRecJB / 2 lanes of a DPP row, in the last of them (entries >= 0)
+__device__ __forceinline__ double block_max(double v)
+{
+    auto shr = [](double x, auto ctrl) {
+        const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, decltype(ctrl)::value, 0xF, 0xF, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), decltype(ctrl)::value, 0xF, 0xF, false);
+        return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
+    };
+    v = fmax(v, shr(v, std::integral_constant<int, 0x111>{}));
+    v = fmax(v, shr(v, std::integral_constant<int, 0x112>{}));
+    if constexpr (kRecJB == 16) v = fmax(v, shr(v, std::integral_constant<int, 0x114>{}));
+    return v;
+}
+
+// Families fams[0 .. nf-1] (count row, row of states), FT per workgroup of one
+// wave; L_all holds [family rounded up to FT][interior node but the root][Ls].
+// tab: k_block_max's (null: no block is skipped).  err[0]: a count outside the
+// matrix (a plain store of 1; any family may set it).
+template <int FT>
+__global__ __launch_bounds__(64) void k_reconstruct(const ReconNode* __restrict__ nodes, int n_prog,
+                                                    const ReconKid* __restrict__ kids,
                                                     const double* __restrict__ mt64, int N, int Np,
-                                                    long long slot_elems, const int* __restrict__ counts_T, int F,
-                                                    const int* __restrict__ fam_sorted, int nf,
+                                                    long long slot_elems, const double* __restrict__ tab,
+                                                    const int* __restrict__ counts_T, int F,
+                                                    const int2* __restrict__ fams, int nf,
                                                     const double* __restrict__ prior, int B, int Rr,
-                                                    double* __restrict__ L_all, int* __restrict__ C_all,
-                                                    double* __restrict__ prod_all, int Lp,
-                                                    int* __restrict__ states, int* __restrict__ err)
+                                                    double* L_all, int Lp, int n_nodes, int* states,
+                                                    int* __restrict__ err)
 {
     const int lane = threadIdx.x;
-    const int k = blockIdx.x;
-    if (k >= nf) return;
-    const int fs = fam_sorted[k];
-    double* L = L_all + (long long)k * n_nodes * Lp;   // [node][i]
-    int* C = C_all + (long long)k * n_nodes * Lp;
-    double* prod = prod_all + (long long)k * Lp;
-    int root = -1, root_state = 0;
-
-    for (int s = 0; s < n_nodes; ++s) {
-        const ReconNode nd = nodes[s];
-        double* Lu = L + (long long)nd.node * Lp;
-        if (nd.leaf_col >= 0) {
-            // gene_family_reconstructor.cpp:30-46: column `count`, i = parent size
-            int obs = counts_T[(long long)nd.leaf_col * F + fs];
-            if (obs < 0 || obs >= N) {   // outside the matrix: flagged, read as 0
-                if (lane == 0) err[0] = 1;
-                obs = 0;
-            }
-            const double* M = mt64 + (long long)nd.slot * slot_elems + (long long)obs * Np;
-            for (int i = lane; i <= B; i += 64) {
-                Lu[i] = M[i];
-                C[(long long)nd.node * Lp + i] = obs;
-            }
-            __syncthreads();
-            continue;
-        }
-        // the children's product for every child size j (reference order)
-        const int jmax = nd.slot < 0 ? Rr - 1 : B;
-        for (int j = lane; j <= jmax; j += 64) {
-            double v = 1.0;
-            for (int c = 0; c < nd.n_kids; ++c) v *= L[(long long)kids[nd.kid0 + c] * Lp + j];
-            prod[j] = v;
-        }
-        __syncthreads();
-        if (nd.slot < 0) {
-            // :48-74: the best j = 1..Rr-1 of prod[j] * prior(j); every L[i],
-            // i >= 1, is that maximum and C[0] its j
-            root = nd.node;
-            if (lane == 0) {
-                double best = -1;
-                int arg = 0;
-                for (int j = 1; j < Rr; ++j) {
-                    const double val = prod[j] * prior[j];
-                    if (val > best) {
-                        best = val;
-                        arg = j;
-                    }
-                }
-                root_state = arg;
-                for (int i = 1; i < Rr; ++i) Lu[i] = best;
-            }
-            __syncthreads();
-            continue;
-        }
-        // :76-111: L[i] = max_j prod[j] * M[i][j], C[i] = its first argmax
-        const double* M = mt64 + (long long)nd.slot * slot_elems;
-        for (int i = lane; i <= B; i += 64) {
-            double best = -1;
-            int arg = 0;
-            for (int j = 0; j <= B; ++j) {
-                const double val = prod[j] * M[(long long)j * Np + i];
-                if (val > best) {
-                    best = val;
-                    arg = j;
-                }
-            }
-            Lu[i] = best;
-            C[(long long)nd.node * Lp + i] = arg;
-        }
-        __syncthreads();
-    }
-    // :170-189: states parents first (the reverse of the children-first order)
-    if (lane == 0) {
-        int* st = states + (long long)k * n_nodes;
-        for (int s = n_nodes - 1; s >= 0; --s) {
-            const ReconNode nd = nodes[s];
-            if (nd.node == root) st[nd.node] = root_state;
-            else if (nd.leaf_col >= 0) st[nd.node] = C[(long long)nd.node * Lp];
-            else {
-                int ps = st[parent[nd.node]];
-                if (ps < 0 || ps > B) {   // a parent state past this node's rows
-                    err[1] = 1;
-                    ps = 0;
-                }
-                st[nd.node] = C[(long long)nd.node * Lp + ps];
-            }
-        }
-    }
-}
-
-// The same reconstruction with kRecW families per workgroup (one wave each)
-// for vectors of at most 64 * kRecQ entries (B < 256).  Every family of a
-// launch uses the same matrices, so the workgroup stages each interior
-// branch's matrix in LDS, a chunk of jc child sizes j at a time, and all its
-// waves take their max-times over the staged rows: the matrix is read from
-// memory once per workgroup instead of once per family.  Within a family the
-// comparisons run over j in ascending order with the first strict maximum
-// kept, as in k_reconstruct, so the states are the same.  Waves past the
-// launch's last family take part in the loads and barriers only.
-constexpr int kRecW = 8;
-constexpr int kRecQ = 4;
-
-__global__ __launch_bounds__(64 * kRecW) void k_reconstruct_shared(
-    const ReconNode* __restrict__ nodes, int n_nodes, const int* __restrict__ kids, const int* __restrict__ parent,
-    const double* __restrict__ mt64, int N, int Np, long long slot_elems, const int* __restrict__ counts_T, int F,
-    const int* __restrict__ fam_sorted, int nf, const double* __restrict__ prior, int B, int Rr,
-    double* __restrict__ L_all, int* __restrict__ C_all, double* __restrict__ prod_all, int Lp,
-    int* __restrict__ states, int* __restrict__ err, int jc)
-{
-    extern __shared__ double sM[];   // [jc][B + 1]: child sizes j0 .. j0+jc-1, parent sizes 0..B
-    const int lane = threadIdx.x & 63;
-    const int k = blockIdx.x * kRecW + (int)(threadIdx.x >> 6);
-    const bool valid = k < nf;
-    const int kk = valid ? k : 0;
-    const int fs = fam_sorted[kk];
-    const int R1 = B + 1;
-    double* L = L_all + (long long)kk * n_nodes * Lp;   // [node][i]
-    int* C = C_all + (long long)kk * n_nodes * Lp;
-    double* prod = prod_all + (long long)kk * Lp;
-    int root = -1, root_state = 0;
-
-    for (int s = 0; s < n_nodes; ++s) {
-        const ReconNode nd = nodes[s];
-        double* Lu = L + (long long)nd.node * Lp;
-        if (nd.leaf_col >= 0) {
-            if (valid) {
-                int obs = counts_T[(long long)nd.leaf_col * F + fs];
-                if (obs < 0 || obs >= N) {
-                    if (lane == 0) err[0] = 1;
-                    obs = 0;
-                }
-                const double* M = mt64 + (long long)nd.slot * slot_elems + (long long)obs * Np;
-                for (int i = lane; i <= B; i += 64) {
-                    Lu[i] = M[i];
-                    C[(long long)nd.node * Lp + i] = obs;
-                }
-            }
-            __syncthreads();
-            continue;
-        }
-        const int jmax = nd.slot < 0 ? Rr - 1 : B;
-        if (valid) {
-            for (int j = lane; j <= jmax; j += 64) {
-                double v = 1.0;
-                for (int c = 0; c < nd.n_kids; ++c) v *= L[(long long)kids[nd.kid0 + c] * Lp + j];
-                prod[j] = v;
-            }
-        }
-        __syncthreads();
-        if (nd.slot < 0) {
-            root = nd.node;
-            if (valid && lane == 0) {
-                double best = -1;
-                int arg = 0;
-                for (int j = 1; j < Rr; ++j) {
-                    const double val = prod[j] * prior[j];
-                    if (val > best) {
-                        best = val;
-                        arg = j;
-                    }
-                }
-                root_state = arg;
-                for (int i = 1; i < Rr; ++i) Lu[i] = best;
-            }
-            __syncthreads();
-            continue;
-        }
-        const double* M = mt64 + (long long)nd.slot * slot_elems;
-        double best[kRecQ];
-        int arg[kRecQ];
+    const int Lq = (Lp + kRecJB - 1) / kRecJB * kRecJB, nj = Lq / kRecJB, Ls = Lp + (Lp & 1);
+    extern __shared__ __align__(16) double s_rec[];
+    double* s_prod = s_rec;              // [FT][Lq] the node's products
+    double* s_pm = s_rec + FT * Lq;      // [nj][FT] their maxima per block
+    int fs[FT];
+    bool valid[FT];
+    double* L[FT];
+    int* st[FT];
 #pragma unroll
-        for (int q = 0; q < kRecQ; ++q) {
-            best[q] = -1;
-            arg[q] = 0;
-        }
-        for (int j0 = 0; j0 <= B; j0 += jc) {
-            const int jn = min(jc, R1 - j0);
-            // rows j0 .. j0+jn-1 of the matrix's parent-size columns 0..B
-            for (int t = threadIdx.x; t < jn * R1; t += 64 * kRecW) {
-                const int r = t / R1;
-                const int i = t - r * R1;
-                sM[t] = M[(long long)(j0 + r) * Np + i];
-            }
-            __syncthreads();
-            if (valid) {
-                for (int r = 0; r < jn; ++r) {
-                    const double pj = prod[j0 + r];
+    for (int f = 0; f < FT; ++f) {
+        const int k = (int)blockIdx.x * FT + f;
+        valid[f] = k < nf;   // past the last family: the last one again, in rows of its own
+        const int kk = valid[f] ? k : nf - 1;
+        fs[f] = __builtin_amdgcn_readfirstlane(fams[kk].x);
+        L[f] = L_all + (long long)k * (n_prog - 1) * Ls;
+        st[f] = states + (long long)__builtin_amdgcn_readfirstlane(fams[kk].y) * n_nodes;
+    }
+    auto count_of = [&](int leaf_col, int f) {
+        const int obs = as_const(counts_T)[(long long)leaf_col * F + fs[f]];
+        if (obs >= 0 && obs < N) return obs;
+        if (lane == 0) err[0] = 1;   // flagged, read as 0
+        return 0;
+    };
+    // family f's row of a child
+    auto row_of = [&](const ReconKid& kd, int f) -> const double* {
+        return kd.leaf_col >= 0 ? mt64 + (long long)kd.slot * slot_elems + (long long)count_of(kd.leaf_col, f) * Np
+                                : L[f] + (long long)kd.ref * Ls;
+    };
+    // a node's children: the first two's rows at hand
+    struct Family2 {
+        const double* r0[FT];
+        const double* r1[FT];
+    };
+    auto children = [&](const ReconNode& nd) {
+        const ReconKid k0 = ld_const(kids, nd.kid0), k1 = ld_const(kids, nd.kid0 + (nd.n_kids > 1 ? 1 : 0));
+        Family2 r;
 #pragma unroll
-                    for (int q = 0; q < kRecQ; ++q) {
-                        const int i = lane + 64 * q;
-                        if (i <= B) {
-                            const double val = pj * sM[r * R1 + i];
-                            if (val > best[q]) {
-                                best[q] = val;
-                                arg[q] = j0 + r;
-                            }
+        for (int f = 0; f < FT; ++f) {
+            r.r0[f] = row_of(k0, f);
+            r.r1[f] = row_of(k1, f);
+        }
+        return r;
+    };
+    // their product at size j (of sizes j and j + 1: V = d2), in descendant order
+    auto product = [&](const ReconNode& nd, const Family2& r, int j, auto (&v)[FT]) {
+        typedef std::remove_reference_t<decltype(v[0])> V;
+        V w[FT];
+#pragma unroll
+        for (int f = 0; f < FT; ++f) {
+            v[f] = *(const V*)(r.r0[f] + j);
+            w[f] = *(const V*)(r.r1[f] + j);
+        }
+        if (nd.n_kids > 1)
+#pragma unroll
+            for (int f = 0; f < FT; ++f) v[f] *= w[f];
+        for (int c = 2; c < nd.n_kids; ++c) {
+            const ReconKid kd = ld_const(kids, nd.kid0 + c);
+#pragma unroll
+            for (int f = 0; f < FT; ++f) v[f] *= *(const V*)(row_of(kd, f) + j);
+        }
+    };
+
+    for (int s = 0; s + 1 < n_prog; ++s) {
+        const ReconNode nd = ld_const(nodes, s);
+        const Family2 r = children(nd);
+        for (int j0 = 0; j0 < Lq; j0 += 128) {
+            const int j = j0 + 2 * lane;
+            d2 v[FT];
+            product(nd, r, j < Ls ? j : Ls - 2, v);
+#pragma unroll
+            for (int f = 0; f < FT; ++f) {
+                if (j >= Lp) v[f][0] = 0.0;
+                if (j + 1 >= Lp) v[f][1] = 0.0;
+                const double m = block_max(fmax(v[f][0], v[f][1]));
+                if (j < Lq) {
+                    *(d2*)(s_prod + f * Lq + j) = v[f];
+                    if (2 * lane % kRecJB == kRecJB - 2) s_pm[j / kRecJB * FT + f] = m;
+                }
+            }
+        }
+        __syncthreads();   // (one wave: orders its accesses)
+        const double* M = mt64 + (long long)nd.slot * slot_elems;
+        const double* T = tab ? tab + (long long)s * nj * (Lq / 2) : nullptr;
+        // rows 128 g + 2 lane and the next one (past the last block: that one's again)
+        for (int i0 = 2 * lane; __builtin_amdgcn_readfirstlane(i0) < Lp; i0 += 128) {
+            const int i = i0 < Lq ? i0 : Lq - 2;
+            d2 best[FT];
+            double low[FT];   // the smaller of the two
+#pragma unroll
+            for (int f = 0; f < FT; ++f) {
+                best[f] = d2{-1, -1};
+                low[f] = -1;
+            }
+            double next = T ? T[i / 2] : 0.0;
+            for (int J = 0; J < nj; ++J) {
+                const double top = next;
+                if (T) next = T[(J + 1 < nj ? J + 1 : J) * (Lq / 2) + i / 2];
+                unsigned need = 0;
+#pragma unroll
+                for (int f = 0; f < FT; ++f)
+                    if (__ballot(!T || s_pm[J * FT + f] * top > low[f])) need |= 1u << f;
+                if (!need) continue;
+                d2 m[kRecJB];
+                const double* C = M + (long long)J * kRecJB * Np + i;
+#pragma unroll
+                for (int jj = 0; jj < kRecJB; ++jj) m[jj] = *(const d2*)(C + jj * Np);
+#pragma unroll
+                for (int f = 0; f < FT; ++f) {
+                    if (!(need >> f & 1)) continue;
+                    const d2* p = (const d2*)(s_prod + f * Lq + J * kRecJB);
+#pragma unroll
+                    for (int jj = 0; jj < kRecJB; jj += 2) {
+                        const d2 w = p[jj / 2];
+#pragma unroll
+                        for (int q = 0; q < 2; ++q) {
+                            best[f][q] = fmax(best[f][q], w[0] * m[jj][q]);
+                            best[f][q] = fmax(best[f][q], w[1] * m[jj + 1][q]);
                         }
                     }
+                    low[f] = fmin(best[f][0], best[f][1]);
                 }
             }
-            __syncthreads();
-        }
-        if (valid) {
+            if (i0 < Ls)
 #pragma unroll
-            for (int q = 0; q < kRecQ; ++q) {
-                const int i = lane + 64 * q;
-                if (i <= B) {
-                    Lu[i] = best[q];
-                    C[(long long)nd.node * Lp + i] = arg[q];
-                }
-            }
+                for (int f = 0; f < FT; ++f) *(d2*)(L[f] + (long long)s * Ls + i0) = best[f];
         }
         __syncthreads();
     }
-    if (valid && lane == 0) {
-        int* st = states + (long long)k * n_nodes;
-        for (int s = n_nodes - 1; s >= 0; --s) {
-            const ReconNode nd = nodes[s];
-            if (nd.node == root) st[nd.node] = root_state;
-            else if (nd.leaf_col >= 0) st[nd.node] = C[(long long)nd.node * Lp];
-            else {
-                int ps = st[parent[nd.node]];
-                if (ps < 0 || ps > B) {
-                    err[1] = 1;
-                    ps = 0;
+
+    // the root: the first best j = 1..Rr-1 (0 where none exceeds -1)
+    {
+        const ReconNode nd = ld_const(nodes, n_prog - 1);
+        double best[FT];
+        int arg[FT];
+#pragma unroll
+        for (int f = 0; f < FT; ++f) {
+            best[f] = -1;
+            arg[f] = 0;
+        }
+        const Family2 r = children(nd);
+        for (int j0 = 1; j0 < Rr; j0 += 64) {
+            const int j = j0 + lane;
+            double v[FT];
+            product(nd, r, j < Rr ? j : Rr - 1, v);
+            const double pr = prior[j < Rr ? j : Rr - 1];
+#pragma unroll
+            for (int f = 0; f < FT; ++f) {
+                const double val = v[f] * pr;
+                if (j < Rr && val > best[f]) {
+                    best[f] = val;
+                    arg[f] = j;
                 }
-                st[nd.node] = C[(long long)nd.node * Lp + ps];
             }
+        }
+#pragma unroll
+        for (int f = 0; f < FT; ++f) {
+            for (int d = 1; d < 64; d <<= 1) {
+                const double ob = __shfl_xor(best[f], d);
+                const int oa = __shfl_xor(arg[f], d);
+                if (ob > best[f] || (ob == best[f] && oa < arg[f])) {
+                    best[f] = ob;
+                    arg[f] = oa;
+                }
+            }
+            if (valid[f]) st[f][nd.node] = arg[f];
+        }
+    }
+    // parents first: each child's state at its parent's (every lane stores the
+    // states it reads back)
+    for (int s = n_prog - 1; s >= 0; --s) {
+        const ReconNode nd = ld_const(nodes, s);
+        int ps[FT];
+#pragma unroll
+        for (int f = 0; f < FT; ++f) ps[f] = st[f][nd.node];
+        for (int c = 0; c < nd.n_kids; ++c) {
+            const ReconKid kd = ld_const(kids, nd.kid0 + c);
+            if (kd.leaf_col >= 0) {
+#pragma unroll
+                for (int f = 0; f < FT; ++f)
+                    if (valid[f]) st[f][kd.ref] = count_of(kd.leaf_col, f);
+                continue;
+            }
+            const ReconNode ch = ld_const(nodes, kd.ref);
+            const Family2 r = children(ch);
+            const double* M = mt64 + (long long)kd.slot * slot_elems;
+            double want[FT];
+            int arg[FT];
+            unsigned open = 0;
+#pragma unroll
+            for (int f = 0; f < FT; ++f) {
+                want[f] = L[f][(long long)kd.ref * Ls + ps[f]];
+                arg[f] = 0;
+                if (valid[f]) open |= 1u << f;
+            }
+            for (int j0 = 0; j0 < Lp && open; j0 += 64) {
+                const int j = j0 + lane < Lp ? j0 + lane : B;   // (B again finds nothing that B did not)
+                double v[FT];
+                product(ch, r, j, v);
+#pragma unroll
+                for (int f = 0; f < FT; ++f) {
+                    const unsigned long long hit = __ballot(v[f] * M[(long long)j * Np + ps[f]] == want[f]);
+                    if (hit && (open >> f & 1)) {
+                        arg[f] = min(j0 + __builtin_ctzll(hit), B);
+                        open &= ~(1u << f);
+                    }
+                }
+            }
+#pragma unroll
+            for (int f = 0; f < FT; ++f)
+                if (valid[f]) st[f][ch.node] = arg[f];
         }
     }
 }
 
-hipError_t launch_reconstruct(const ReconNode* nodes, int n_nodes, const int* kids, const int* parent,
-                              const double* mt64, int N, int Np, long long slot_elems, const int* counts_T, int F,
-                              const int* fam_sorted, int nf, const double* prior, int B, int Rr, double* L_all,
-                              int* C_all, double* prod_all, int Lp, int* states, int* err, hipStream_t st)
+static int block_rows(int Lp) { return (Lp + kRecJB - 1) / kRecJB * kRecJB; }
+
+// Doubles of k_block_max's table.
+size_t recon_table_doubles(int n_prog, int Lp)
+{
+    return (size_t)(n_prog - 1) * (block_rows(Lp) / kRecJB) * (block_rows(Lp) / 2);
+}
+
+hipError_t launch_block_max(const ReconNode* nodes, int n_prog, const double* mt64, int Np, long long slot_elems,
+                            int Lp, double* tab, hipStream_t st)
+{
+    const int Lq = block_rows(Lp), nj = Lq / kRecJB;
+    for (int s0 = 0; s0 < n_prog - 1; s0 += 65535)   // grid.z
+        hipLaunchKernelGGL(k_block_max, dim3((Lq / 2 + 255) / 256, nj, std::min(65535, n_prog - 1 - s0)), dim3(256), 0, st,
+                           nodes + s0, mt64, Np, slot_elems, Lq, tab + (size_t)s0 * nj * (Lq / 2));
+    return hipGetLastError();
+}
+
+hipError_t launch_reconstruct(const ReconNode* nodes, int n_prog, const ReconKid* kids, const double* mt64, int N,
+                              int Np, long long slot_elems, const double* tab, const int* counts_T, int F,
+                              const int2* fams, int nf, const double* prior, int B, int Rr, double* L_all, int Lp,
+                              int n_nodes, int* states, int* err, hipStream_t st)
 {
     if (nf <= 0) return hipSuccess;
-    if (B + 1 <= 64 * kRecQ && B + 1 <= N) {
-        // staged rows: as many as fit in 48 KB, at most 32
-        const int jc = std::max(1, std::min(32, (48 * 1024) / (8 * (B + 1))));
-        const size_t shm = sizeof(double) * (size_t)jc * (B + 1);
-        hipLaunchKernelGGL(k_reconstruct_shared, dim3((nf + kRecW - 1) / kRecW), dim3(64 * kRecW), shm, st, nodes,
-                           n_nodes, kids, parent, mt64, N, Np, slot_elems, counts_T, F, fam_sorted, nf, prior, B, Rr,
-                           L_all, C_all, prod_all, Lp, states, err, jc);
+    const int Lq = block_rows(Lp);
+    auto go = [&](auto ft) {
+        constexpr int FT = decltype(ft)::value;
+        const size_t shm = sizeof(double) * (size_t)FT * (Lq + Lq / kRecJB);
+        hipLaunchKernelGGL(k_reconstruct<FT>, dim3((nf + FT - 1) / FT), dim3(64), shm, st, nodes, n_prog, kids, mt64, N,
+                           Np, slot_elems, tab, counts_T, F, fams, nf, prior, B, Rr, L_all, Lp, n_nodes, states,
+                           err);
         return hipGetLastError();
-    }
-    hipLaunchKernelGGL(k_reconstruct, dim3(nf), dim3(64), 0, st, nodes, n_nodes, kids, parent, mt64, N, Np,
-                       slot_elems, counts_T, F, fam_sorted, nf, prior, B, Rr, L_all, C_all, prod_all, Lp, states,
-                       err);
-    return hipGetLastError();
+    };
+    return nf >= kRecFew && Lp <= kRecMaxShared ? go(std::integral_constant<int, kRecFT>{}) : go(std::integral_constant<int, 1>{});
 }
 
 }  // namespace cafe
