@@ -122,13 +122,49 @@ struct BucketHost {
 // Device buffers of one evaluation (eager calls or a plan).
 struct EvalBufs {
     DevBuf node_slot, prior64, prior32, catp, buckets, tiles, ntiles, fb_tiles, fb_count, val,
-        flag, lnl, cat, post, fail, total, scratch, root, segs, class_off, fam_list;
+        flag, lnl, cat, post, fail, total, scratch, root, segs, class_off, fam_list, units, cols_x, cols_meta;
+    std::vector<BucketDev> bucket_h;   // the bucket table (plan_prune adds the programs and units, and uploads it)
     void release_all()
     {
         DevBuf* all[] = {&node_slot, &prior64, &prior32, &catp, &buckets, &tiles, &ntiles, &fb_tiles,
                          &fb_count, &val, &flag, &lnl, &cat, &post, &fail, &total, &scratch, &root, &segs,
-                         &class_off, &fam_list};
+                         &class_off, &fam_list, &units, &cols_x, &cols_meta};
         for (DevBuf* b : all) b->release();
+    }
+};
+
+// A program over pattern columns: its steps and columns in Patterns' buffers.
+struct PatternProg {
+    int step0 = 0, n_steps = 0, col0 = 0, n_cols = 0, n_pat = 0;
+    int n_slots = 0, n_slots_reuse = 0;   // of its steps and steps_reuse
+};
+struct PatternUnit {
+    PatternProg prog;
+    int bucket;
+    int n;         // patterns
+    int list0;     // their representatives' place in `reps`
+    int level;     // 1 + the largest level of a unit it reads (0: none)
+};
+// The subtree patterns of the families under the tree (UnitDev), made once per
+// tree and families.
+struct Patterns {
+    bool made = false;
+    std::vector<PatternUnit> units;     // per bucket contiguous
+    std::vector<PatternProg> main;      // per bucket
+    std::vector<int> first_unit;        // per bucket (and the end)
+    DevBuf ext;                         // count table with the units' pattern rows after the leaves'
+    DevBuf steps, steps_reuse;          // programs (steps_reuse: outputs in their children's slots)
+    DevBuf cols, reps;
+    void clear()
+    {
+        made = false;
+        units.clear();
+        main.clear();
+        first_unit.clear();
+    }
+    void release_all()
+    {
+        for (DevBuf* b : {&ext, &steps, &steps_reuse, &cols, &reps}) b->release();
     }
 };
 
@@ -176,6 +212,8 @@ struct cafe_gpu_ctx {
     std::vector<int> fam_max;   // per family of the caller: its largest count
     std::vector<BucketHost> buckets;
     DevBuf d_counts, d_perm;
+    std::vector<int> counts_T;   // as uploaded: [leaf][F], bucket-sorted
+    Patterns pat;
 
     // error model, and the pools with it folded into every matrix (leaf
     // branches read those)
@@ -332,6 +370,277 @@ struct Planner {
     }
 };
 
+// Children of every node, in increasing index, and the root.
+std::vector<std::vector<int>> children_of(const std::vector<int>& parent, int& root)
+{
+    std::vector<std::vector<int>> kids(parent.size());
+    root = -1;
+    for (int i = 0; i < (int)parent.size(); ++i) {
+        if (parent[i] < 0) root = i;
+        else kids[parent[i]].push_back(i);
+    }
+    return kids;
+}
+
+// A flat list of child steps from a planner's ops.
+std::vector<StepDev> flatten_steps(const std::vector<OpDev>& ops, const std::vector<ChildDev>& kids)
+{
+    std::vector<StepDev> steps;
+    for (size_t o = 0; o < ops.size(); ++o) {
+        const OpDev& op = ops[o];
+        for (int k = 0; k < op.n_child; ++k) {
+            const ChildDev& ch = kids[op.child_begin + k];
+            int ctl = op.out_slot;
+            if (k == 0) ctl |= kStepFirst;
+            if (k == op.n_child - 1) ctl |= kStepLast;
+            if (o + 1 == ops.size()) ctl |= kStepRoot;
+            steps.push_back(StepDev{ch.node, ch.leaf_col, ch.in_slot, ctl});
+        }
+    }
+    return steps;
+}
+
+// Buckets of fewer families are not searched for patterns (a few tiles wait for
+// one chain of steps, which more launches only lengthen).
+constexpr int kPatternFamilies = 512;
+// A node is a candidate while its patterns are at most half of the families:
+// one step of 50,000 gamma families 1.49 ms, against 1.52 at a quarter and 1.62
+// at an eighth (16,000 at B = 500: 19.4, 20.5, 21.8); past a half the columns
+// written and read cost what the shared work saves.
+constexpr int kPatternShare = 2;
+// A unit's descendant becomes a unit of its own where that divides its work by
+// three or more; otherwise it is computed along, one launch less (1.51, 1.52
+// and 1.70 ms dividing by 2, by 6 and never; 5,000 families 0.75, 0.78, 0.76).
+constexpr int kPatternNest = 3;
+
+// Pattern ids of the pairs (a[f], b[f]), a < na and b < nb, numbered in order
+// of appearance; 0 where there are more than `limit`.
+int pair_patterns(const std::vector<int>& a, int na, const std::vector<int>& b, int nb, int limit, std::vector<int>& id,
+                  std::vector<int>& table)
+{
+    const int F = (int)a.size();
+    id.resize(F);
+    const long long space = (long long)na * nb;
+    int n = 0;
+    if (space <= 1 << 20) {
+        table.assign(space, -1);
+        for (int f = 0; f < F; ++f) {
+            int& t = table[(size_t)a[f] * nb + b[f]];
+            if (t < 0) {
+                if (n == limit) return 0;
+                t = n++;
+            }
+            id[f] = t;
+        }
+        return n;
+    }
+    // open addressing: slots of (key, id)
+    size_t size = 1024;
+    while (size < 4 * (size_t)limit) size <<= 1;
+    std::vector<std::pair<long long, int>> slots(size, {-1, 0});
+    for (int f = 0; f < F; ++f) {
+        const long long key = (long long)a[f] * nb + b[f];
+        size_t h = (size_t)((unsigned long long)key * 0x9E3779B97F4A7C15ull >> 20) & (size - 1);
+        while (slots[h].first >= 0 && slots[h].first != key) h = (h + 1) & (size - 1);
+        if (slots[h].first < 0) {
+            if (n == limit) return 0;
+            slots[h] = {key, n++};
+        }
+        id[f] = slots[h].second;
+    }
+    return n;
+}
+
+// Finds the units of every bucket, their programs and those of the buckets,
+// and uploads them (once per tree and families).
+int find_patterns(cafe_gpu_ctx* ctx)
+{
+    Patterns& P = ctx->pat;
+    const int F = ctx->F, nl = ctx->n_leaves, n = ctx->n_nodes;
+    const auto& leaf = ctx->leaf_col_h;
+    int root;
+    const auto kids = children_of(ctx->parent_h, root);
+    std::vector<int> order;   // children first
+    {
+        std::vector<std::pair<int, int>> stack{{root, 0}};
+        while (!stack.empty()) {
+            auto& top = stack.back();
+            const int u = top.first;
+            if (top.second < (int)kids[u].size()) {
+                stack.push_back({kids[u][top.second++], 0});
+                continue;
+            }
+            stack.pop_back();
+            if (leaf[u] < 0) order.push_back(u);
+        }
+    }
+    std::vector<int> row(n, -1);   // a unit node's row of the extended count table
+    int n_rows = nl;
+    std::vector<std::vector<int>> rows;   // [n_rows - nl][F]
+    std::vector<StepDev> steps, steps_reuse;
+    std::vector<ColDev> cols;
+    std::vector<int> reps, table;
+    P.main.resize(ctx->buckets.size());
+    for (int bi = 0; bi < (int)ctx->buckets.size(); ++bi) {
+        const BucketHost& bk = ctx->buckets[bi];
+        const int xs = std::max(round_up(bk.B + 1, kTile), round_up(bk.R + 1, kTile));
+        P.first_unit.push_back((int)P.units.size());
+        std::vector<std::vector<int>> ids(n);
+        std::vector<int> count(n, 0);   // patterns of a node (0: not a candidate)
+        if (bk.count >= kPatternFamilies) {
+            const int limit = bk.count / kPatternShare;
+            for (int u = 0; u < n; ++u)
+                if (leaf[u] >= 0) {
+                    const int* c = ctx->counts_T.data() + (size_t)leaf[u] * F + bk.fam_begin;
+                    ids[u].assign(c, c + bk.count);
+                    count[u] = bk.max_count + 1;
+                }
+            for (int u : order) {
+                if (u == root) continue;
+                bool all = true;
+                for (int c : kids[u]) all = all && count[c] > 0;
+                if (!all) continue;
+                std::vector<int> cur = ids[kids[u][0]], next;
+                int m = count[kids[u][0]];
+                for (size_t k = 1; k < kids[u].size() && m > 0; ++k) {
+                    m = pair_patterns(cur, m, ids[kids[u][k]], count[kids[u][k]], limit, next, table);
+                    cur.swap(next);
+                }
+                if (kids[u].size() == 1 && leaf[kids[u][0]] >= 0) {   // (a leaf's counts are not numbered by appearance)
+                    const std::vector<int> one(bk.count, 0);
+                    m = pair_patterns(cur, m, one, 1, limit, next, table);
+                    cur.swap(next);
+                }
+                if (m == 0 || (long long)m * xs >= 1 << 28) continue;
+                ids[u].swap(cur);
+                count[u] = m;
+            }
+        }
+        // units, top down: candidates under a node that is none, and those
+        // under a unit that divide its patterns
+        std::vector<char> unit(n, 0);
+        std::vector<int> inside(n, 0);   // patterns of the unit that computes a node (0: none)
+        for (auto it = order.rbegin(); it != order.rend(); ++it)
+            for (int c : kids[*it]) {
+                if (leaf[c] >= 0 || count[c] == 0) continue;
+                unit[c] = inside[*it] == 0 || (long long)count[c] * kPatternNest <= inside[*it];
+                inside[c] = unit[c] ? count[c] : inside[*it];
+            }
+        std::vector<int> unit_of(n, -1), level(n, 0), code(n, -1);
+        auto program = [&](int top, bool is_unit) {
+            // the tree below top, its leaves and units in columns
+            std::vector<int> walk{top}, pats, leaves;
+            int lev = 0;
+            while (!walk.empty()) {
+                const int u = walk.back();
+                walk.pop_back();
+                for (int c : kids[u]) {
+                    if (leaf[c] >= 0) {
+                        leaves.push_back(c);
+                    } else if (unit[c]) {
+                        pats.push_back(c);
+                        lev = std::max(lev, level[c] + 1);
+                    } else {
+                        walk.push_back(c);
+                    }
+                }
+            }
+            PatternProg pr;
+            pr.col0 = (int)cols.size();
+            pr.n_pat = (int)pats.size();
+            for (int c : pats) {
+                code[c] = (int)cols.size() - pr.col0;
+                cols.push_back(ColDev{row[c], xs});
+            }
+            for (int c : leaves) {
+                code[c] = (int)cols.size() - pr.col0;
+                cols.push_back(ColDev{leaf[c], 0});
+            }
+            pr.n_cols = (int)cols.size() - pr.col0;
+            pr.step0 = (int)steps.size();
+            for (const bool reuse : {false, true}) {
+                Planner pl(kids, code, reuse);
+                pl.compute_need(top);
+                pl.emit(top);
+                (reuse ? pr.n_slots_reuse : pr.n_slots) = pl.max_slot + 1;
+                std::vector<StepDev> st = flatten_steps(pl.ops, pl.out_kids);
+                for (StepDev& s : st) {
+                    if (is_unit) s.ctl &= ~kStepRoot;
+                    if (s.leaf_col >= 0 && s.leaf_col < pr.n_pat) {
+                        s.ctl |= kStepPattern;
+                        s.in_slot = unit_of[s.node];
+                    }
+                }
+                if (is_unit)   // the branch's contraction, written as columns
+                    st.push_back(StepDev{top, -1, pl.slot_of[top],
+                                         kStepFirst | kStepLast | kStepOut |
+                                             (ctx->parent_h[top] == root ? kStepRoot : 0)});
+                pr.n_steps = (int)st.size();
+                auto& all = reuse ? steps_reuse : steps;
+                all.insert(all.end(), st.begin(), st.end());
+            }
+            for (int c : pats) code[c] = -1;
+            for (int c : leaves) code[c] = -1;
+            if (is_unit) level[top] = lev;
+            return pr;
+        };
+        for (int u : order) {
+            if (!unit[u]) continue;
+            if (row[u] < 0) {
+                row[u] = n_rows++;
+                rows.emplace_back(F, 0);
+            }
+            std::copy(ids[u].begin(), ids[u].end(), rows[row[u] - nl].begin() + bk.fam_begin);
+            PatternUnit un;
+            unit_of[u] = (int)P.units.size();
+            un.prog = program(u, true);
+            un.bucket = bi;
+            un.n = count[u];
+            un.list0 = (int)reps.size();
+            un.level = level[u];
+            reps.resize(reps.size() + un.n, -1);
+            for (int f = 0; f < bk.count; ++f) {
+                int& r = reps[un.list0 + ids[u][f]];
+                if (r < 0) r = bk.fam_begin + f;
+            }
+            P.units.push_back(un);
+        }
+        P.main[bi] = program(root, false);
+    }
+    P.first_unit.push_back((int)P.units.size());
+    if (!P.units.empty()) {
+        HIP_OR_FAIL(P.ext.ensure(sizeof(int) * (size_t)n_rows * F));
+        HIP_OR_FAIL(hipMemcpy(P.ext.p, ctx->d_counts.p, sizeof(int) * (size_t)nl * F, hipMemcpyDeviceToDevice));
+        for (int r = nl; r < n_rows; ++r)
+            HIP_OR_FAIL(hipMemcpy(P.ext.as<int>() + (size_t)r * F, rows[r - nl].data(), sizeof(int) * F, hipMemcpyHostToDevice));
+        auto put = [&](DevBuf& b, const void* v, size_t bytes) -> int {
+            HIP_OR_FAIL(b.ensure(bytes));
+            HIP_OR_FAIL(hipMemcpy(b.p, v, bytes, hipMemcpyHostToDevice));
+            return CAFE_GPU_OK;
+        };
+        if (int rc = put(P.steps, steps.data(), sizeof(StepDev) * steps.size())) return rc;
+        if (int rc = put(P.steps_reuse, steps_reuse.data(), sizeof(StepDev) * steps_reuse.size())) return rc;
+        if (int rc = put(P.cols, cols.data(), sizeof(ColDev) * cols.size())) return rc;
+        if (int rc = put(P.reps, reps.data(), sizeof(int) * reps.size())) return rc;
+    }
+    return CAFE_GPU_OK;
+}
+
+// The same for a caller that needs none: without memory for them every bucket
+// keeps its whole program.
+void make_patterns(cafe_gpu_ctx* ctx)
+{
+    Patterns& P = ctx->pat;
+    if (P.made) return;
+    P.clear();
+    if (find_patterns(ctx) != CAFE_GPU_OK) {
+        (void)hipGetLastError();
+        P.clear();
+        P.release_all();
+    }
+    P.made = true;
+}
+
 }  // namespace
 
 // ===========================================================================
@@ -395,6 +704,7 @@ int cafe_gpu_destroy(cafe_gpu_ctx* ctx)
                       &ctx->d_err32, &ctx->mt64e, &ctx->mt32e, &ctx->mt16h, &ctx->mt16l, &ctx->band32};
     for (DevBuf* b : bufs) b->release();
     ctx->eager.release_all();
+    ctx->pat.release_all();
     for (auto& e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : ctx->join_ev)
@@ -545,6 +855,7 @@ int cafe_gpu_set_tree(cafe_gpu_ctx* ctx, int n_nodes, const int* parent, const i
     if (pl.max_slot + 1 > kMaxSlots)
         return fail(CAFE_GPU_EINVAL, "tree needs %d live partial vectors (max %d)", pl.max_slot + 1, kMaxSlots);
     ctx->input_gen++;
+    ctx->pat.clear();
     ctx->n_nodes = n_nodes;
     ctx->tree_leaves = n_leaves;
     ctx->parent_h.assign(parent, parent + n_nodes);
@@ -560,22 +871,7 @@ int cafe_gpu_set_tree(cafe_gpu_ctx* ctx, int n_nodes, const int* parent, const i
     HIP_OR_FAIL(hipMemcpy(ctx->d_kids.p, ctx->kids.data(), sizeof(ChildDev) * ctx->kids.size(),
                           hipMemcpyHostToDevice));
     // the same program as a flat list of child steps
-    auto flatten = [](const std::vector<OpDev>& ops, const std::vector<ChildDev>& kids) {
-        std::vector<StepDev> steps;
-        for (size_t o = 0; o < ops.size(); ++o) {
-            const OpDev& op = ops[o];
-            for (int k = 0; k < op.n_child; ++k) {
-                const ChildDev& ch = kids[op.child_begin + k];
-                int ctl = op.out_slot;
-                if (k == 0) ctl |= kStepFirst;
-                if (k == op.n_child - 1) ctl |= kStepLast;
-                if (o + 1 == ops.size()) ctl |= kStepRoot;
-                steps.push_back(StepDev{ch.node, ch.leaf_col, ch.in_slot, ctl});
-            }
-        }
-        return steps;
-    };
-    const std::vector<StepDev> steps = flatten(ctx->ops, ctx->kids);
+    const std::vector<StepDev> steps = flatten_steps(ctx->ops, ctx->kids);
     ctx->n_steps = (int)steps.size();
     HIP_OR_FAIL(ctx->d_steps.ensure(sizeof(StepDev) * steps.size()));
     HIP_OR_FAIL(hipMemcpy(ctx->d_steps.p, steps.data(), sizeof(StepDev) * steps.size(), hipMemcpyHostToDevice));
@@ -584,12 +880,12 @@ int cafe_gpu_set_tree(cafe_gpu_ctx* ctx, int n_nodes, const int* parent, const i
     pr.compute_need(root);
     pr.used.clear();
     pr.emit(root);
-    const std::vector<StepDev> lsteps = flatten(pr.ops, pr.out_kids);
+    const std::vector<StepDev> lsteps = flatten_steps(pr.ops, pr.out_kids);
     ctx->n_slots_lane = pr.max_slot + 1;
     HIP_OR_FAIL(ctx->d_steps_lane.ensure(sizeof(StepDev) * lsteps.size()));
     HIP_OR_FAIL(hipMemcpy(ctx->d_steps_lane.p, lsteps.data(), sizeof(StepDev) * lsteps.size(),
                           hipMemcpyHostToDevice));
-    const std::vector<StepDev> hsteps = flatten(ph.ops, ph.out_kids);
+    const std::vector<StepDev> hsteps = flatten_steps(ph.ops, ph.out_kids);
     ctx->n_slots_hot = std::max(1, ph.max_slot + 1);
     HIP_OR_FAIL(ctx->d_steps_hot.ensure(sizeof(StepDev) * hsteps.size()));
     HIP_OR_FAIL(hipMemcpy(ctx->d_steps_hot.p, hsteps.data(), sizeof(StepDev) * hsteps.size(),
@@ -629,6 +925,7 @@ int cafe_gpu_set_families(cafe_gpu_ctx* ctx, int F, int n_leaves, const int* cou
         b.max_count = std::max(b.max_count, top[f]);
     }
     ctx->input_gen++;
+    ctx->pat.clear();
     std::vector<int> cT((size_t)n_leaves * F);
     for (int k = 0; k < F; ++k)
         for (int i = 0; i < n_leaves; ++i) cT[(size_t)i * F + k] = counts[(size_t)order[k] * n_leaves + i];
@@ -640,6 +937,8 @@ int cafe_gpu_set_families(cafe_gpu_ctx* ctx, int F, int n_leaves, const int* cou
     ctx->fam_max = top;
     ctx->F = F;
     ctx->n_leaves = n_leaves;
+    ctx->counts_T.swap(cT);
+    if (ctx->tree_leaves == n_leaves) make_patterns(ctx);
     return CAFE_GPU_OK;
 }
 
@@ -718,6 +1017,15 @@ struct KernelClass {
     // class's main pass
     size_t off_main = 0, off_r64 = 0;
     int stream = 0;      // side stream of its launches
+    // subtree patterns: its buckets run their programs over units' columns,
+    // made level by level before the main pass (tiles, their count's place)
+    bool pat = false;
+    int max_pat = 0, n_cols = 0;            // most pattern and leaf columns of a program
+    int n_slots = 0, n_slots_lane = 0;      // most partial vectors of a program (in order, with reuse)
+    struct Level {
+        int begin, n, count_at;
+    };
+    std::vector<Level> levels;
 };
 
 // Host-side description of one pruning sequence over a tile list.
@@ -856,16 +1164,17 @@ size_t f64_scratch_bytes(const MfmaShape& s, int n_slots, int nt, int grid)
 
 // Dynamic LDS of an MFMA launch without its partials: the bookkeeping and the
 // tile's leaf counts.
-size_t mfma_meta_only(const MfmaShape& s, int n_slots, int n_leaves)
+size_t mfma_meta_only(const MfmaShape& s, int n_slots, int n_leaves, int n_pat)
 {
-    return (size_t)mfma_meta_bytes(n_slots, s.w, s.fb) + (size_t)mfma_count_bytes(n_leaves, s.fb);
+    return (size_t)mfma_meta_bytes(n_slots, s.w, s.fb) + (size_t)mfma_count_bytes(n_leaves, s.fb) +
+           (size_t)mfma_pat_bytes(n_pat, s.fb);
 }
 
 // Partial vectors go to LDS when the workgroup's share stays small enough for
 // several workgroups per CU; the rest use the global scratch.
-void place_partials(MfmaShape& s, int n_slots, int slot_tiles, int n_leaves)
+void place_partials(MfmaShape& s, int n_slots, int slot_tiles, int n_leaves, int n_pat)
 {
-    const size_t meta = mfma_meta_only(s, n_slots, n_leaves);
+    const size_t meta = mfma_meta_only(s, n_slots, n_leaves, n_pat);
     const size_t frag = (size_t)n_slots * slot_tiles * s.fb * 64 * 4 * 4;
     if (s.fb > 1)   // two workgroups per CU, or one of 8 waves
         s.lds = s.w <= 8 && meta + frag + 4096 <= (s.w >= 8 ? 144 : 76) * 1024;
@@ -885,9 +1194,14 @@ constexpr int kMaxRows = 2048;        // the largest vectors of any path
 // B operands (hi, lo, bound).
 size_t f16_frag_bytes(int n_slots, int slot_tiles) { return (size_t)3 * n_slots * ((slot_tiles + 1) / 2) * 64 * 16; }
 
-void place_partials16(MfmaShape& s, int n_slots, int slot_tiles, int n_leaves)
+size_t f16_meta_only(const MfmaShape& s, int n_slots, int n_leaves, int n_pat)
 {
-    const size_t meta = (size_t)f16_meta_bytes(n_slots, s.w) + (size_t)mfma_count_bytes(n_leaves);
+    return (size_t)f16_meta_bytes(n_slots, s.w) + (size_t)mfma_count_bytes(n_leaves) + (size_t)f16_pat_bytes(n_pat);
+}
+
+void place_partials16(MfmaShape& s, int n_slots, int slot_tiles, int n_leaves, int n_pat)
+{
+    const size_t meta = f16_meta_only(s, n_slots, n_leaves, n_pat);
     const size_t frag = f16_frag_bytes(n_slots, slot_tiles);
     // two workgroups per CU (its registers allow two waves per SIMD)
     s.lds = s.w <= 4 && meta + frag + 4096 <= 76 * 1024;
@@ -898,6 +1212,13 @@ size_t f16_scratch_bytes(const MfmaShape& s, int n_slots, int slot_tiles, int gr
 {
     return s.lds ? 0 : (size_t)grid * f16_frag_bytes(n_slots, slot_tiles);
 }
+
+// A class runs over subtree patterns from this many family-likelihoods on: each
+// level of units is a launch more (2,000 families of 12 taxa at B = 100, three
+// levels: 305 -> 285 us a step).
+constexpr long long kPatternWork = 1024;
+// Columns of one evaluation, at most.
+constexpr size_t kPatternBytes = (size_t)8 << 30;
 
 // Dynamic LDS of a lane-kernel launch: the tile's leaf counts.
 size_t lane_shm(int n_leaves) { return (size_t)n_leaves * 64 * sizeof(int); }
@@ -928,8 +1249,8 @@ const cafe_gpu_ctx::TuneEntry* find_tuning(const cafe_gpu_ctx* ctx, int path, in
 // stored vectors have slot_tiles tiles, when that kernel instance exists,
 // covers the class (tiles per wave x waves >= nt) and fits a CU (occupancy
 // query; LDS partials only where they fit).
-bool tuned_mfma_shape(cafe_gpu_ctx* ctx, int path, const cafe_gpu_ctx::TuneEntry& e, int nt, int slot_tiles,
-                      MfmaShape& s)
+bool tuned_mfma_shape(cafe_gpu_ctx* ctx, int path, const cafe_gpu_ctx::TuneEntry& e, const KernelClass& kc, int nt,
+                      int slot_tiles, MfmaShape& s)
 {
     if ((e.kernel != 0 && e.kernel != 2) || path == CAFE_GPU_PATH_PLAIN64 || e.ntw < 1 || e.w < 1 || e.ntw * e.w < nt)
         return false;
@@ -945,17 +1266,17 @@ bool tuned_mfma_shape(cafe_gpu_ctx* ctx, int path, const cafe_gpu_ctx::TuneEntry
     hipError_t q = hipSuccess;
     const PruneParams none{};
     if (fp64) {
-        s.shm = f64_shm(s, ctx->n_slots, nt, ctx->n_leaves);
+        s.shm = f64_shm(s, kc.n_slots, nt, kc.n_cols);
         if (s.shm > 150 * 1024 || ctx->n_leaves > 512) return false;   // LDS partials that do not fit
         q = f64_dispatch(s, 0, none, nullptr, &s.per_cu);
     } else {
-        if (f16) place_partials16(s, ctx->n_slots_lane, slot_tiles, ctx->n_leaves);
-        else place_partials(s, ctx->n_slots, slot_tiles, ctx->n_leaves);
+        if (f16) place_partials16(s, kc.n_slots_lane, slot_tiles, kc.n_cols, kc.max_pat);
+        else place_partials(s, kc.n_slots, slot_tiles, kc.n_cols, kc.max_pat);
         if (e.lds && !s.lds) return false;   // LDS partials that do not fit
         if (!e.lds && s.lds) {               // global scratch asked for
             s.lds = false;
-            s.shm = f16 ? (size_t)f16_meta_bytes(ctx->n_slots_lane, s.w) + (size_t)mfma_count_bytes(ctx->n_leaves)
-                        : mfma_meta_only(s, ctx->n_slots, ctx->n_leaves);
+            s.shm = f16 ? f16_meta_only(s, kc.n_slots_lane, kc.n_cols, kc.max_pat)
+                        : mfma_meta_only(s, kc.n_slots, kc.n_cols, kc.max_pat);
         }
         q = f16 ? f16_dispatch(s, 0, none, nullptr, &s.per_cu) : mfma_occupancy(s, &s.per_cu);
     }
@@ -982,7 +1303,7 @@ int apply_tuning(cafe_gpu_ctx* ctx, int path, KernelClass& kc, unsigned long lon
         return CAFE_GPU_OK;
     }
     MfmaShape s;
-    if (!tuned_mfma_shape(ctx, path, *e, kc.nt, kc.slot_tiles, s)) return CAFE_GPU_OK;
+    if (!tuned_mfma_shape(ctx, path, *e, kc, kc.nt, kc.slot_tiles, s)) return CAFE_GPU_OK;
     if (s.fb != kc.fb) return CAFE_GPU_OK;   // the tiles were cut for another width
     if (path == CAFE_GPU_PATH_BATCHED16 && e->kernel == 0) kc.s16 = s;
     else if (path == CAFE_GPU_PATH_BATCHED64) kc.s64 = s;
@@ -1043,7 +1364,8 @@ int upload_eval_inputs(cafe_gpu_ctx* ctx, EvalBufs& b, const cafe_gpu_eval_desc*
     const int nb = (int)ctx->buckets.size();
     std::vector<double> pr64((size_t)nb * d->prior_stride, 0.0);
     std::vector<float> pr32(pr64.size());
-    std::vector<BucketDev> bd(nb);
+    std::vector<BucketDev>& bd = b.bucket_h;
+    bd.assign(nb, BucketDev{});
     for (int i = 0; i < nb; ++i) {
         const auto& bh = ctx->buckets[i];
         for (int j = 0; j < bh.R; ++j) pr64[(size_t)i * d->prior_stride + j] = d->prior[(size_t)i * d->prior_stride + j];
@@ -1055,6 +1377,7 @@ int upload_eval_inputs(cafe_gpu_ctx* ctx, EvalBufs& b, const cafe_gpu_eval_desc*
         bd[i].fam_begin = bh.fam_begin;
         bd[i].count = bh.count;
         bd[i].prior_off = i * d->prior_stride;
+        bd[i].out = -1;
     }
     for (size_t i = 0; i < pr64.size(); ++i) pr32[i] = (float)pr64[i];
     std::vector<double> cp(K, 1.0);
@@ -1062,12 +1385,10 @@ int upload_eval_inputs(cafe_gpu_ctx* ctx, EvalBufs& b, const cafe_gpu_eval_desc*
     HIP_OR_FAIL(b.node_slot.ensure(sizeof(int) * ns));
     HIP_OR_FAIL(b.prior64.ensure(sizeof(double) * pr64.size()));
     HIP_OR_FAIL(b.prior32.ensure(sizeof(float) * pr32.size()));
-    HIP_OR_FAIL(b.buckets.ensure(sizeof(BucketDev) * nb));
     HIP_OR_FAIL(b.catp.ensure(sizeof(double) * K));
     HIP_OR_FAIL(hipMemcpy(b.node_slot.p, slot.data(), sizeof(int) * ns, hipMemcpyHostToDevice));
     HIP_OR_FAIL(hipMemcpy(b.prior64.p, pr64.data(), sizeof(double) * pr64.size(), hipMemcpyHostToDevice));
     HIP_OR_FAIL(hipMemcpy(b.prior32.p, pr32.data(), sizeof(float) * pr32.size(), hipMemcpyHostToDevice));
-    HIP_OR_FAIL(hipMemcpy(b.buckets.p, bd.data(), sizeof(BucketDev) * nb, hipMemcpyHostToDevice));
     HIP_OR_FAIL(hipMemcpy(b.catp.p, cp.data(), sizeof(double) * K, hipMemcpyHostToDevice));
     const size_t PF = (size_t)P * ctx->F;
     HIP_OR_FAIL(b.val.ensure(sizeof(double) * PF));
@@ -1150,6 +1471,33 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     unsigned long long plan_classes = 0;
     for (const auto& kr : key_rows)
         if (kr.first >= 1 && kr.first <= 64) plan_classes |= 1ull << (kr.first - 1);
+    // the classes that run over subtree patterns: those with units, enough
+    // family-likelihoods, on a kernel that reads columns, with their columns
+    // within the memory set aside
+    make_patterns(ctx);
+    const Patterns& pat = ctx->pat;
+    const int nb = (int)ctx->buckets.size();
+    int max_point = 0;
+    for (int i = 0; i < n_points; ++i) max_point = std::max(max_point, point_ids[i] + 1);
+    std::map<int, bool> key_pat;
+    size_t pat_bytes = 0;
+    if (!pat.units.empty() && !root_out)
+        for (const auto& kr : key_rows) {
+            const int key = kr.first;
+            const bool f64 = path == CAFE_GPU_PATH_PLAIN64 || path == CAFE_GPU_PATH_BATCHED64 || key > kMfmaMaxTiles;
+            if (lane_rows_of(key) > 0 || (f64 && ctx->n_leaves > 512)) continue;
+            long long fams = 0;
+            size_t bytes = 0;
+            for (auto& bc : bucket_class) {
+                if (bc.first != key || pat.first_unit[bc.second] == pat.first_unit[bc.second + 1]) continue;
+                fams += (long long)ctx->buckets[bc.second].count * n_points;
+                for (int u = pat.first_unit[bc.second]; u < pat.first_unit[bc.second + 1]; ++u)
+                    bytes += 8 * (size_t)pat.units[u].n * max_point * kTile * key_nt[key];
+            }
+            if (fams < kPatternWork || pat_bytes + bytes > kPatternBytes) continue;
+            key_pat[key] = true;
+            pat_bytes += bytes;
+        }
     std::vector<TileDesc> tiles;
     std::vector<SegDesc> segs;
     int prev_key = -1;
@@ -1160,19 +1508,36 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
             kc.begin = kc.end = (int)tiles.size();
             kc.fams = key_fams[bc.first];
             kc.seg_begin = kc.seg_end = (int)segs.size();
+            kc.pat = key_pat.count(bc.first) > 0;
+            kc.n_cols = kc.pat ? 0 : ctx->n_leaves;
+            kc.n_slots = kc.pat ? 0 : ctx->n_slots;
+            kc.n_slots_lane = kc.pat ? 0 : ctx->n_slots_lane;
+            if (kc.pat) {
+                auto add = [&](const PatternProg& pr) {
+                    kc.max_pat = std::max(kc.max_pat, pr.n_pat);
+                    kc.n_cols = std::max(kc.n_cols, pr.n_cols);
+                    kc.n_slots = std::max(kc.n_slots, pr.n_slots);
+                    kc.n_slots_lane = std::max(kc.n_slots_lane, pr.n_slots_reuse);
+                };
+                for (auto& o : bucket_class) {
+                    if (o.first != bc.first) continue;
+                    add(pat.main[o.second]);
+                    for (int u = pat.first_unit[o.second]; u < pat.first_unit[o.second + 1]; ++u) add(pat.units[u].prog);
+                }
+            }
             // the kernel is chosen here: its tiles carry 64 families (per
             // lane) or 16 (matrix cores)
             kc.plain = path == CAFE_GPU_PATH_PLAIN64 || bc.first > kMfmaMaxTiles;
             kc.f64 = kc.plain || path == CAFE_GPU_PATH_BATCHED64;
             kc.lane_rows = kc.plain ? 0 : lane_rows_of(bc.first);
             if (kc.f64)
-                kc.fb = f64_shape(key_nt[bc.first], kc.fams / kTile, ctx->n_slots, ctx->n_leaves, ctx->n_cu).fb;
+                kc.fb = f64_shape(key_nt[bc.first], kc.fams / kTile, kc.n_slots, kc.n_cols, ctx->n_cu).fb;
             kc.fb = kc.lane_rows > 0 ? 1
                   : kc.f64           ? kc.fb
                                      : builtin_fb32(path, bc.first, n_mfma_keys == 1, key_fams[bc.first], ctx->n_cu);
             if (const cafe_gpu_ctx::TuneEntry* te = kc.plain ? nullptr : find_tuning(ctx, path, bc.first, plan_classes)) {
                 MfmaShape probe;
-                if (tuned_mfma_shape(ctx, path, *te, bc.first, bc.first, probe)) {
+                if (tuned_mfma_shape(ctx, path, *te, kc, bc.first, bc.first, probe)) {
                     kc.lane_rows = 0;
                     kc.fb = probe.fb;
                 }
@@ -1206,25 +1571,25 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     for (auto& kc : pp.classes) {
         if (kc.f64) {
             pp.has_f64 = true;
-            kc.s64 = f64_shape(kc.nt, kc.fams / kTile, ctx->n_slots, ctx->n_leaves, ctx->n_cu);
+            kc.s64 = f64_shape(kc.nt, kc.fams / kTile, kc.n_slots, kc.n_cols, ctx->n_cu);
             if (int rc = f64_occupancy(kc.s64)) return rc;
             continue;
         }
         kc.s32 = kc.fb == 2 ? mfma_shape_fb2(kc.nt) : mfma_shape(kc.nt);
         kc.r64 = f64_shape(kc.nt, 1, ctx->n_slots, ctx->n_leaves, ctx->n_cu);
-        place_partials(kc.s32, ctx->n_slots, kc.slot_tiles, ctx->n_leaves);
+        place_partials(kc.s32, kc.n_slots, kc.slot_tiles, kc.n_cols, kc.max_pat);
         HIP_OR_FAIL(mfma_occupancy(kc.s32, &kc.s32.per_cu));
         if (int rc = f64_occupancy(kc.r64)) return rc;
         if (path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles) {
             // the program whose outputs reuse a child's slot (the store's
             // maxima exchange orders all reads before the writes)
             kc.s16 = mfma_shape(kc.nt);
-            place_partials16(kc.s16, ctx->n_slots_lane, kc.slot_tiles, ctx->n_leaves);
+            place_partials16(kc.s16, kc.n_slots_lane, kc.slot_tiles, kc.n_cols, kc.max_pat);
             const PruneParams none{};
             HIP_OR_FAIL(f16_dispatch(kc.s16, 0, none, nullptr, &kc.s16.per_cu));
             if (kc.s16.per_cu == 0 && kc.s16.lds) {   // LDS does not fit: global scratch
                 kc.s16.lds = false;
-                kc.s16.shm = (size_t)f16_meta_bytes(ctx->n_slots_lane, kc.s16.w) + (size_t)mfma_count_bytes(ctx->n_leaves);
+                kc.s16.shm = f16_meta_only(kc.s16, kc.n_slots_lane, kc.n_cols, kc.max_pat);
                 HIP_OR_FAIL(f16_dispatch(kc.s16, 0, none, nullptr, &kc.s16.per_cu));
             }
         }
@@ -1271,6 +1636,61 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     pp.n_tiles = (int)tiles.size();
     pp.class_counts.assign(n_cls + 4, 0);
     for (int i = 0; i < n_cls; ++i) pp.class_counts[i] = pp.classes[i].end - pp.classes[i].begin;
+    // the units: bucket-table entries after the buckets', columns, and per
+    // class and level their tiles (lists of representatives)
+    std::vector<BucketDev>& bd = b.bucket_h;
+    std::vector<UnitDev> units(pat.units.size(), UnitDev{});
+    long long n64 = 0, n32 = 0, n_meta = 0;
+    if (pat_bytes > 0) {
+        auto set_prog = [](BucketDev& d, const PatternProg& pr) {
+            d.step0 = pr.step0;
+            d.n_steps = pr.n_steps;
+            d.col0 = pr.col0;
+            d.n_cols = pr.n_cols;
+            d.n_pat = pr.n_pat;
+        };
+        bd.resize(nb);
+        for (int i = 0; i < nb; ++i) set_prog(bd[i], pat.main[i]);
+        for (int u = 0; u < (int)pat.units.size(); ++u) {
+            BucketDev d = bd[pat.units[u].bucket];
+            set_prog(d, pat.units[u].prog);
+            d.out = u;
+            d.list0 = pat.units[u].list0;
+            d.fam_begin = 0;
+            d.count = pat.units[u].n;
+            bd.push_back(d);
+        }
+        for (auto& kc : pp.classes) {
+            if (!kc.pat) continue;
+            const int tw = kTile * kc.fb;
+            std::vector<std::vector<TileDesc>> level;
+            for (auto& bc : bucket_class) {
+                if (key_nt[bc.first] != kc.nt || !key_pat.count(bc.first)) continue;
+                for (int u = pat.first_unit[bc.second]; u < pat.first_unit[bc.second + 1]; ++u) {
+                    const PatternUnit& pu = pat.units[u];
+                    UnitDev& ud = units[u];
+                    ud.n = pu.n;
+                    // (a column covers the bucket's own rows)
+                    const BucketHost& bk = ctx->buckets[bc.second];
+                    ud.xs = std::max(round_up(bk.B + 1, kTile), round_up(bk.R + 1, kTile));
+                    long long& top = kc.f64 ? n64 : n32;
+                    ud.x0 = top;
+                    top += (long long)pu.n * max_point * ud.xs;
+                    ud.m0 = n_meta;
+                    n_meta += (long long)pu.n * max_point;
+                    if ((int)level.size() <= pu.level) level.resize(pu.level + 1);
+                    for (int pi = 0; pi < n_points; ++pi)
+                        for (int i0 = 0; i0 < pu.n; i0 += tw)
+                            level[pu.level].push_back(TileDesc{nb + u, point_ids[pi], pu.list0 + i0, -std::min(tw, pu.n - i0)});
+                }
+            }
+            for (auto& l : level) {
+                kc.levels.push_back(KernelClass::Level{(int)tiles.size(), (int)l.size(), (int)pp.class_counts.size()});
+                pp.class_counts.push_back((int)l.size());
+                tiles.insert(tiles.end(), l.begin(), l.end());
+            }
+        }
+    }
     // [0, n_cls] offsets of the 16-family recompute lists (room for all of a
     // class's families in 16-family tiles)
     std::vector<int> class_off(n_cls + 1, 0);
@@ -1281,9 +1701,9 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     pp.r16_total = class_off[n_cls];
     pp.n_segs = (int)segs.size();
 
-    HIP_OR_FAIL(b.tiles.ensure(sizeof(TileDesc) * std::max(1, pp.n_tiles)));
+    HIP_OR_FAIL(b.tiles.ensure(sizeof(TileDesc) * std::max<size_t>(1, tiles.size())));
     HIP_OR_FAIL(b.fb_tiles.ensure(sizeof(TileDesc) * (size_t)std::max(1, pp.r16_total)));
-    HIP_OR_FAIL(b.ntiles.ensure(sizeof(int) * (n_cls + 4)));
+    HIP_OR_FAIL(b.ntiles.ensure(sizeof(int) * pp.class_counts.size()));
     HIP_OR_FAIL(b.fb_count.ensure(sizeof(int) * (n_cls + 2)));
     HIP_OR_FAIL(b.segs.ensure(sizeof(SegDesc) * std::max(1, pp.n_segs)));
     HIP_OR_FAIL(b.class_off.ensure(sizeof(int) * (n_cls + 1)));
@@ -1292,7 +1712,15 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
         for (int i = 0; i < n_points; ++i) maxp = std::max(maxp, (size_t)point_ids[i] + 1);
         HIP_OR_FAIL(b.fam_list.ensure(sizeof(int) * maxp * (size_t)ctx->F));
     }
-    HIP_OR_FAIL(hipMemcpy(b.tiles.p, tiles.data(), sizeof(TileDesc) * pp.n_tiles, hipMemcpyHostToDevice));
+    HIP_OR_FAIL(hipMemcpy(b.tiles.p, tiles.data(), sizeof(TileDesc) * tiles.size(), hipMemcpyHostToDevice));
+    HIP_OR_FAIL(b.buckets.ensure(sizeof(BucketDev) * bd.size()));
+    HIP_OR_FAIL(hipMemcpy(b.buckets.p, bd.data(), sizeof(BucketDev) * bd.size(), hipMemcpyHostToDevice));
+    if (pat_bytes > 0) {
+        HIP_OR_FAIL(b.units.ensure(sizeof(UnitDev) * units.size()));
+        HIP_OR_FAIL(hipMemcpy(b.units.p, units.data(), sizeof(UnitDev) * units.size(), hipMemcpyHostToDevice));
+        HIP_OR_FAIL(b.cols_x.ensure(sizeof(double) * n64 + sizeof(float) * n32 * (path == CAFE_GPU_PATH_BATCHED16 ? 2 : 1)));
+        HIP_OR_FAIL(b.cols_meta.ensure((sizeof(double) + sizeof(int)) * n_meta));
+    }
     HIP_OR_FAIL(hipMemcpy(b.ntiles.p, pp.class_counts.data(), sizeof(int) * pp.class_counts.size(),
                           hipMemcpyHostToDevice));
     HIP_OR_FAIL(hipMemcpy(b.segs.p, segs.data(), sizeof(SegDesc) * pp.n_segs, hipMemcpyHostToDevice));
@@ -1303,12 +1731,13 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     size_t main_sz = 0, r64_sz = 0;
     for (int ci = 0; ci < n_cls; ++ci) {
         KernelClass& kc = pp.classes[ci];
-        const int n = pp.class_counts[ci];
+        int n = pp.class_counts[ci];
+        for (const auto& l : kc.levels) n = std::max(n, l.n);
         size_t mb = 0;
-        if (kc.f64) mb = f64_scratch_bytes(kc.s64, ctx->n_slots, kc.nt, pp.grid(kc.s64, n));
+        if (kc.f64) mb = f64_scratch_bytes(kc.s64, kc.n_slots, kc.nt, pp.grid(kc.s64, n));
         else if (kc.lane_rows > 0) mb = 0;
-        else if (path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles) mb = f16_scratch_bytes(kc.s16, ctx->n_slots_lane, kc.slot_tiles, pp.grid(kc.s16, n));
-        else mb = mfma_scratch_bytes(kc.s32, ctx->n_slots, kc.slot_tiles, pp.grid(kc.s32, n));
+        else if (path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles) mb = f16_scratch_bytes(kc.s16, kc.n_slots_lane, kc.slot_tiles, pp.grid(kc.s16, n));
+        else mb = mfma_scratch_bytes(kc.s32, kc.n_slots, kc.slot_tiles, pp.grid(kc.s32, n));
         kc.off_main = main_sz;
         main_sz += align256(mb);
         if (!kc.f64) {
@@ -1365,6 +1794,16 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     p.scratch = b.scratch.p;
     p.n_slots = ctx->n_slots;
     p.zero = 0;
+    p.units = nullptr;   // (set for the launches of the classes that use them)
+    p.max_pat = 0;
+    if (pat_bytes > 0) {
+        p.cols = pat.cols.as<ColDev>();
+        p.x64 = b.cols_x.as<double>();
+        p.x32 = (float*)(p.x64 + n64);
+        p.xe32 = p.x32 + n32;
+        p.xm_c = b.cols_meta.as<double>();
+        p.xm_e = (int*)(p.xm_c + n_meta);
+    }
     return CAFE_GPU_OK;
 }
 
@@ -1402,23 +1841,43 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
         q.n_tiles_dev = d_cnt + ci;
         q.slot_tiles = kc.slot_tiles;
         q.scratch = scratch + kc.off_main;
-        if (kc.f64) {   // final FP64 values: nothing to recompute
-            q.slot_tiles = kc.nt;
-            if (!kc.plain) q.near_floor = fbc + fam_off + 1;
-            HIP_OR_FAIL(f64_dispatch(kc.s64, pp.grid(kc.s64, n), q, s, nullptr));
-        } else if (kc.lane_rows > 0) {   // BATCHED32 / BATCHED16: small vectors, one family per lane
+        q.n_slots = kc.n_slots;
+        if (kc.lane_rows > 0) {   // BATCHED32 / BATCHED16: small vectors, one family per lane
             q.steps = ctx->d_steps_hot.as<StepDev>();
             q.n_slots = ctx->n_slots_hot;
             HIP_OR_FAIL(lane_dispatch(kc.lane_rows, kc.lane_slots, pp.grid_lane(kc.lane_per_cu, n, kc.lane_grid_mult),
                                       lane_shm(ctx->n_leaves), q, s, nullptr));
-        } else if (pp.path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles) {
-            q.steps = ctx->d_steps_lane.as<StepDev>();
-            q.n_slots = ctx->n_slots_lane;
-            HIP_OR_FAIL(f16_dispatch(kc.s16, pp.grid(kc.s16, n), q, s, nullptr));
-        } else {
-            HIP_OR_FAIL(launch_prune_mfma(kc.s32, pp.grid(kc.s32, n), q, s));
+            return CAFE_GPU_OK;
         }
-        return CAFE_GPU_OK;
+        const bool f16 = !kc.f64 && pp.path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles;
+        if (f16) {
+            q.steps = ctx->d_steps_lane.as<StepDev>();
+            q.n_slots = kc.n_slots_lane;
+        }
+        if (kc.f64) q.slot_tiles = kc.nt;
+        auto launch = [&](const PruneParams& a, int tiles) -> int {
+            if (kc.f64) HIP_OR_FAIL(f64_dispatch(kc.s64, pp.grid(kc.s64, tiles), a, s, nullptr));
+            else if (f16) HIP_OR_FAIL(f16_dispatch(kc.s16, pp.grid(kc.s16, tiles), a, s, nullptr));
+            else HIP_OR_FAIL(launch_prune_mfma(kc.s32, pp.grid(kc.s32, tiles), a, s));
+            return CAFE_GPU_OK;
+        };
+        if (kc.pat) {
+            q.units = b.units.as<UnitDev>();
+            q.max_pat = kc.max_pat;
+            q.n_leaves = kc.n_cols;
+            q.steps = (f16 ? ctx->pat.steps_reuse : ctx->pat.steps).as<StepDev>();
+            q.counts_T = ctx->pat.ext.as<int>();
+            for (const auto& l : kc.levels) {
+                PruneParams a = q;
+                a.tiles = b.tiles.as<TileDesc>() + l.begin;
+                a.n_tiles_dev = d_cnt + l.count_at;
+                a.fam_list = ctx->pat.reps.as<int>();
+                if (int rc = launch(a, l.n)) return rc;
+            }
+        }
+        // (final FP64 values: nothing to recompute)
+        if (kc.f64 && !kc.plain) q.near_floor = fbc + fam_off + 1;
+        return launch(q, n);
     };
     auto stage_r64 = [&](int ci, hipStream_t s) -> int {
         const KernelClass& kc = pp.classes[ci];

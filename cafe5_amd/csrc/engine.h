@@ -66,6 +66,34 @@ struct BucketDev {
     int fam_begin;     // first family (bucket-sorted order)
     int count;
     int prior_off;     // offset of this bucket's prior in the prior tables
+    // its program where the launch uses subtree patterns (PruneParams::units)
+    int step0, n_steps;   // steps [step0, step0 + n_steps)
+    int col0, n_cols;     // columns [col0, col0 + n_cols) its leaf steps read
+    int n_pat;            // the first n_pat of them are pattern columns
+    int out;              // >= 0: a unit, whose columns these tiles write; -1: the bucket itself
+    int list0;            // unit: its first pattern's place in the list of representatives
+    int pad;
+};
+
+// Subtree patterns.  Families of a bucket with the same counts at every leaf
+// under a node have the same factor at that node's branch, so each distinct
+// combination (pattern) is computed once: a unit is such a node, its program the
+// subtree below it (down to units of its own) and its branch's contraction, run
+// over one representative family per pattern.  The results are columns, and a
+// family's program reads column `pattern` of a unit as it reads column `count`
+// of a leaf's matrix.
+struct UnitDev {
+    long long x0;   // its columns: x0 + (point n + pattern) xs
+    long long m0;   // their exponents and bounds: m0 + point n + pattern
+    int n;          // patterns
+    int xs;         // entries per column
+    int pad[2];
+};
+// A column of a program's leaf steps: the row of the count table with each
+// family's index, and the entries per index.
+struct ColDev {
+    int row;
+    int stride;   // 0: a leaf's counts, columns of its matrix
 };
 
 // Internal node of the evaluation program (Sethi-Ullman order, root last).
@@ -95,6 +123,8 @@ enum : int {
     kStepFirst = 1 << 8,   // first child of its op: the product starts at 1
     kStepLast = 1 << 9,    // last child: the op's vector is complete
     kStepRoot = 1 << 10,   // the op is the root
+    kStepPattern = 1 << 11,   // a leaf step over a unit's columns (in_slot: the unit)
+    kStepOut = 1 << 12,       // a unit's last step: the factor is written as columns
     kStepSlotMask = 0xff,
     // per-lane kernel: a vector kept in registers (the output the next op
     // reads, read by that op), as in_slot and out_slot
@@ -165,6 +195,15 @@ struct PruneParams {
     // outside of which the tile's entries are exactly 0 (null: no band)
     const int* band;
     int band_stride;
+    // subtree patterns (null: every bucket runs steps / n_steps over its leaves)
+    const UnitDev* units;
+    const ColDev* cols;
+    int max_pat;              // most pattern columns of a program of the launch
+    double* x64;              // the units' columns
+    float* x32;
+    float* xe32;              // split FP16: their bounds' columns
+    int* xm_e;                // per column: exponent (FP32, split FP16)
+    double* xm_c;             // and flush bound (FP32)
 };
 
 // Interior nodes of the reconstruction program, children before parents, the
@@ -230,6 +269,11 @@ __host__ __device__ inline int f64_meta_bytes(int w, int fb, int n_leaves, bool 
     const int b = w * 16 * fb * 16 + (staged ? n_leaves * 16 * fb * 4 : 0);
     return (b + 31) & ~31;
 }
+
+// Dynamic LDS of a tile's pattern columns: exponent and flush bound per family
+// (split FP16: the exponent).
+__host__ __device__ inline int mfma_pat_bytes(int n_pat, int fb = 1) { return (n_pat * 16 * fb * 12 + 31) & ~31; }
+__host__ __device__ inline int f16_pat_bytes(int n_pat) { return (n_pat * 16 * 4 + 31) & ~31; }
 
 // Dynamic-LDS copy of a tile's leaf counts: n_leaves x 16 fb ints.
 __host__ __device__ inline int mfma_count_bytes(int n_leaves, int fb = 1)

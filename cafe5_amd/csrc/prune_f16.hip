@@ -132,8 +132,10 @@ __device__ __forceinline__ RootBest16 root_combine16(RootBest16 r)
 // ---------------------------------------------------------------------------
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 
+// (three tiles per wave fit two waves per SIMD; the compiler needs telling)
 template <int NTW, int W, bool LDSP>
-__global__ __launch_bounds__(64 * W) void k_prune_f16(PruneParams p)
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(NTW <= 3 ? 2 : 1)))
+void k_prune_f16(PruneParams p)
 {
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -146,7 +148,6 @@ __global__ __launch_bounds__(64 * W) void k_prune_f16(PruneParams p)
     const int n_slots = p.n_slots;
     const int slot_blocks = (p.slot_tiles + 1) >> 1;
     const int a_exp = p.vec_exp16;
-    const int n_steps = p.n_steps;
     const int zero = __builtin_amdgcn_readfirstlane(p.zero);
     const float leaf_e = (float)((p.n_dev > 1 ? p.n_dev : 1) * kTau32);
     constexpr float kTau = 1.1754943508222875e-38f;
@@ -162,8 +163,10 @@ __global__ __launch_bounds__(64 * W) void k_prune_f16(PruneParams p)
     int* m_esum = (int*)(m_wmax + W * 16);
     const int meta = f16_meta_bytes(n_slots, W);
     int* s_cnt = (int*)(s_dyn + meta);
+    const int cnt_bytes = mfma_count_bytes(p.n_leaves);
+    int* m_pe = (int*)(s_dyn + meta + cnt_bytes);   // [pattern column][16]: exponent
     const long long part = (long long)n_slots * slot_blocks * 64;   // half8 per part
-    half8* fh = LDSP ? (half8*)(s_dyn + meta + mfma_count_bytes(p.n_leaves))
+    half8* fh = LDSP ? (half8*)(s_dyn + meta + cnt_bytes + f16_pat_bytes(p.max_pat))
                      : (half8*)p.scratch + (long long)blockIdx.x * 3 * part;
     half8* flo = fh + part;
     half8* fe = flo + part;
@@ -180,12 +183,27 @@ __global__ __launch_bounds__(64 * W) void k_prune_f16(PruneParams p)
         const TileDesc td = ld_const(p.tiles, tile);
         const BucketDev bk = ld_const(p.buckets, td.bucket);
         const int nf = td.nf < 0 ? -td.nf : td.nf;
-        for (int i = threadIdx.x; i < p.n_leaves * 16; i += 64 * W) {
-            const int f = i & 15;
+        const StepDev* __restrict__ steps = p.steps + (p.units ? bk.step0 : 0);
+        const int n_steps = p.units ? bk.n_steps : p.n_steps;
+        const int n_cols = p.units ? bk.n_cols : p.n_leaves;
+        for (int i = threadIdx.x; i < n_cols * 16; i += 64 * W) {
+            const int f = i & 15, c = i >> 4;
             const int ff = f < nf ? f : 0;
             const int fam = td.nf < 0 ? p.fam_list[td.fam0 + ff] : bk.fam_begin + td.fam0 + ff;
-            s_cnt[i] = p.counts_T[(long long)(i >> 4) * p.F + fam];
+            const ColDev cd = p.units ? p.cols[bk.col0 + c] : ColDev{c, 0};
+            s_cnt[i] = p.counts_T[(long long)cd.row * p.F + fam] * (cd.stride ? cd.stride : Np);
         }
+        if (p.units)   // the pattern columns' exponents
+            for (int st = wv; st < n_steps; st += W) {
+                const StepDev sd = ld_const(steps, __builtin_amdgcn_readfirstlane(st));
+                if (!(sd.ctl & kStepPattern) || lane >= 16) continue;
+                const UnitDev u = ld_const(p.units, sd.in_slot);
+                const int ff = lane < nf ? lane : 0;
+                const int fam = td.nf < 0 ? p.fam_list[td.fam0 + ff] : bk.fam_begin + td.fam0 + ff;
+                m_pe[sd.leaf_col * 16 + lane] =
+                    p.xm_e[u.m0 + (long long)td.point * u.n +
+                           p.counts_T[(long long)p.cols[bk.col0 + sd.leaf_col].row * p.F + fam]];
+            }
         __syncthreads();
         const bool valid = fl < nf;
         const int fi = valid ? fl : 0;
@@ -240,7 +258,7 @@ __global__ __launch_bounds__(64 * W) void k_prune_f16(PruneParams p)
         };
         auto prefetch = [&](floatx4 (&pf)[2][NTW], StepDev& sd, int& kbl, int& kbh, int st) {
             st = __builtin_amdgcn_readfirstlane(st < n_steps ? st : n_steps - 1);
-            sd = ld_const(p.steps, st);
+            sd = ld_const(steps, st);
             const bool root = (sd.ctl & kStepRoot) != 0;
             const bool leaf = sd.leaf_col >= 0;
             const int slot = nslot[sd.node];
@@ -248,15 +266,24 @@ __global__ __launch_bounds__(64 * W) void k_prune_f16(PruneParams p)
             kbl = 0;
             kbh = nkb;
             if (!leaf) kband(slot, root, kbl, kbh);
-            const int cn = s_cnt[(leaf ? sd.leaf_col : 0) * 16 + fl] * Np;
+            const int cn = s_cnt[(leaf ? sd.leaf_col : 0) * 16 + fl];
+            // a leaf's column, twice (the second with the opaque 0 added); a
+            // unit's column and its bound's
+            const float* __restrict__ C = lpool + mo;
+            const float* __restrict__ C2 = C + 4 * zero;
+            if (sd.ctl & kStepPattern) {
+                const UnitDev u = ld_const(p.units, sd.in_slot);
+                const long long x0 = u.x0 + (long long)td.point * u.n * u.xs;
+                C = p.x32 + x0;
+                C2 = p.xe32 + x0;
+            }
 #pragma unroll
             for (int i = 0; i < NTW; ++i) {
                 const int oa = root ? offA1[i] : offA0[i];
                 const int ol = cn + (root ? offL1[i] : offL0[i]);
                 if (leaf) {
-                    const floatx4* q = (const floatx4*)(lpool + mo + ol);
-                    pf[0][i] = q[0];
-                    pf[1][i] = q[zero];
+                    pf[0][i] = *(const floatx4*)(C + ol);
+                    pf[1][i] = *(const floatx4*)(C2 + ol);
                 } else {
                     pf[0][i] = *(const floatx4*)(poolh + mo + oa + 32 * kbl);
                     pf[1][i] = *(const floatx4*)(pooll + mo + oa + 32 * kbl);
@@ -283,12 +310,13 @@ __global__ __launch_bounds__(64 * W) void k_prune_f16(PruneParams p)
             if (first) e_sum = 0;
             floatx4 x[NTW], xe[NTW];
             if (sd.leaf_col >= 0) {
-                e_sum -= kMatExp;
+                const bool pattern = (sd.ctl & kStepPattern) != 0;
+                e_sum += pattern ? m_pe[sd.leaf_col * 16 + fl] : -kMatExp;
 #pragma unroll
                 for (int i = 0; i < NTW; ++i) {
                     x[i] = pf[0][i];
                     await16(pf[1][i]);
-                    xe[i] = floatx4{leaf_e, leaf_e, leaf_e, leaf_e};
+                    xe[i] = pattern ? pf[1][i] : floatx4{leaf_e, leaf_e, leaf_e, leaf_e};
                 }
             } else {
                 e_sum += m_esum[sd.in_slot * 16 + fl] - kMatExp16;
@@ -407,6 +435,20 @@ __global__ __launch_bounds__(64 * W) void k_prune_f16(PruneParams p)
             }
             if (!(sd.ctl & kStepLast)) return;
 
+            if (sd.ctl & kStepOut) {   // the branch's factor (its one step's) and bound as columns
+                const UnitDev u = ld_const(p.units, bk.out);
+                const long long c = (long long)td.point * u.n + td.fam0 - bk.list0 + fl;
+                if (!valid) return;
+#pragma unroll
+                for (int i = 0; i < NTW; ++i)
+                    if (live[i]) {
+                        const long long at = u.x0 + c * u.xs + kTile * tt[i] + 4 * g;
+                        *(floatx4*)(p.x32 + at) = acc[i];
+                        *(floatx4*)(p.xe32 + at) = acc_e[i];
+                    }
+                if (wv == 0 && g == 0) p.xm_e[u.m0 + c] = e_sum;
+                return;
+            }
             if (!root) {
                 // finish the node: per-family maximum over every wave's rows
                 // (rows past the bound are 0), shift to just below 2^a, split

@@ -104,11 +104,16 @@ __global__ __launch_bounds__((64 * F64Waves<NTW, FB>::v)) void k_prune_f64(Prune
         const TileDesc td = ld_const(p.tiles, tile);
         const BucketDev bk = ld_const(p.buckets, td.bucket);
         const int nf = td.nf < 0 ? -td.nf : td.nf;
-        for (int i = threadIdx.x; STAGED && i < p.n_leaves * FW; i += 64 * W) {
-            const int f = i & (FW - 1);
+        const bool units = STAGED && p.units;
+        const StepDev* __restrict__ steps = p.steps + (units ? bk.step0 : 0);
+        const int n_steps = units ? bk.n_steps : p.n_steps;
+        const int n_cols = units ? bk.n_cols : p.n_leaves;
+        for (int i = threadIdx.x; STAGED && i < n_cols * FW; i += 64 * W) {
+            const int f = i & (FW - 1), c = i / FW;
             const int ff = td.fam0 + (f < nf ? f : 0);
             const int fam = td.nf < 0 ? p.fam_list[ff] : bk.fam_begin + ff;
-            s_cnt[i] = 8u * Np * p.counts_T[(long long)(i / FW) * p.F + fam];
+            const ColDev cd = units ? p.cols[bk.col0 + c] : ColDev{c, 0};
+            s_cnt[i] = 8u * (cd.stride ? cd.stride : Np) * p.counts_T[(long long)cd.row * p.F + fam];
         }
         int fam[FB], dst[FB];   // this lane's families, and their places in the caller's order
 #pragma unroll
@@ -145,6 +150,10 @@ __global__ __launch_bounds__((64 * F64Waves<NTW, FB>::v)) void k_prune_f64(Prune
         auto issue = [&](d4 (&pf)[FB][NTW], const Step& s) {
             const bool leaf = s.sd.leaf_col >= 0;
             const double* M = (leaf ? p.leaf64 : p.mt64) + base_of(s);
+            if (STAGED && (s.sd.ctl & kStepPattern)) {   // columns of the rows themselves
+                const UnitDev u = ld_const(p.units, s.sd.in_slot);
+                M = p.x64 + u.x0 + (long long)td.point * u.n * u.xs;
+            }
 #pragma unroll
             for (int f = 0; f < FB; ++f) {
                 const int col = leaf ? s.sd.leaf_col : 0;
@@ -240,6 +249,23 @@ __global__ __launch_bounds__((64 * F64Waves<NTW, FB>::v)) void k_prune_f64(Prune
             }
             if (!(s.sd.ctl & kStepLast)) return;
             const int len = root ? bk.R : bk.L, nrt = tiles_of(root);
+            if (STAGED && (s.sd.ctl & kStepOut)) {   // the branch's factor (its one step's) as columns
+                const UnitDev u = ld_const(p.units, bk.out);
+                const long long c = (long long)td.point * u.n + td.fam0 - bk.list0;
+#pragma unroll
+                for (int f = 0; f < FB; ++f) {
+                    if (16 * f + fl >= nf) continue;
+                    double* X = p.x64 + u.x0 + (c + 16 * f + fl) * u.xs + g;
+#pragma unroll
+                    for (int i = 0; i < NTW; ++i) {
+                        const int t = s.c * NTW + i;
+                        if (t >= nrt) break;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) X[kTile * t + 4 * r] = acc[f][i][r];
+                    }
+                }
+                return;
+            }
             const Frag out = frag + (s.sd.ctl & kStepSlotMask) * slot_tiles * FB * 64 + lane;
 #pragma unroll
             for (int i = 0; i < NTW; ++i) {
@@ -274,10 +300,10 @@ __global__ __launch_bounds__((64 * F64Waves<NTW, FB>::v)) void k_prune_f64(Prune
                 s.c = wv;
                 s.first = ++s.st;
             }
-            s.sd = ld_const(p.steps, s.st < p.n_steps ? s.st : p.n_steps - 1);
+            s.sd = ld_const(steps, s.st < n_steps ? s.st : n_steps - 1);
         };
         d4 pfa[FB][NTW], pfb[FB][NTW];
-        Step sa{ld_const(p.steps, 0), 0, 0, wv}, sb;
+        Step sa{ld_const(steps, 0), 0, 0, wv}, sb;
         issue(pfa, sa);
         // an op ends where the following step is another op's
         for (;;) {
@@ -286,15 +312,18 @@ __global__ __launch_bounds__((64 * F64Waves<NTW, FB>::v)) void k_prune_f64(Prune
             issue(pfb, sb);
             compute(pfa, sa);
             if (sb.first != sa.first) __syncthreads();
-            if (sb.st >= p.n_steps) break;
+            if (sb.st >= n_steps) break;
             sa = sb;
             advance(sa);
             issue(pfa, sa);
             compute(pfb, sb);
             if (sa.first != sb.first) __syncthreads();
-            if (sa.st >= p.n_steps) break;
+            if (sa.st >= n_steps) break;
         }
-        const int root_slot = ld_const(p.steps, p.n_steps - 1).ctl & kStepSlotMask;
+        if (units && bk.out >= 0) {   // (the last step has ended behind a barrier)
+            continue;
+        }
+        const int root_slot = ld_const(steps, n_steps - 1).ctl & kStepSlotMask;
 
         // max_j log x_j + log prior_j (base_model.cpp:84-90) or x_j prior_j
         // (gamma_core.cpp:156-161): the largest product first, then the

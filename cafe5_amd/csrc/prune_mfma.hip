@@ -222,7 +222,6 @@ void k_prune_mfma(PruneParams p)
     const int n_slots = p.n_slots;
     const int slot_tiles = p.slot_tiles;
     const int a_exp = p.vec_exp;
-    const int n_steps = p.n_steps;
     const int zero = __builtin_amdgcn_readfirstlane(p.zero);   // 0, opaque to the compiler
     // FP32 leaf factors: up to n_dev flushed terms (one without an error model)
     const double leaf_cert = (p.n_dev > 1 ? p.n_dev : 1) * kTau32 * kTwoPowMinusMatExp;
@@ -241,8 +240,11 @@ void k_prune_mfma(PruneParams p)
     int* m_bsh = m_esum + n_slots * FW;
     int* m_l2s = m_bsh + n_slots * FW;
     const int meta = mfma_meta_bytes(n_slots, W, FB);
-    int* s_cnt = (int*)(s_dyn + meta);                // [leaf][FW]
-    V4* frag = LDSP ? (V4*)(s_dyn + meta + mfma_count_bytes(p.n_leaves, FB))
+    int* s_cnt = (int*)(s_dyn + meta);                // [column][FW]: offset of the family's column
+    const int cnt_bytes = mfma_count_bytes(p.n_leaves, FB);
+    double* m_pc = (double*)(s_dyn + meta + cnt_bytes);   // [pattern column][FW]: flush bound
+    int* m_pe = (int*)(m_pc + p.max_pat * FW);            // and exponent
+    V4* frag = LDSP ? (V4*)(s_dyn + meta + cnt_bytes + mfma_pat_bytes(p.max_pat, FB))
                     : (V4*)p.scratch + (long long)blockIdx.x * n_slots * slot_tiles * FB * 64;
     __shared__ double s_rkey[W][FW], s_rx[W][FW], s_rxmax[W][FW];
     __shared__ int s_rj[W][FW];
@@ -262,13 +264,30 @@ void k_prune_mfma(PruneParams p)
         const TileDesc td = ld_const(p.tiles, tile);
         const BucketDev bk = ld_const(p.buckets, td.bucket);
         const int nf = td.nf < 0 ? -td.nf : td.nf;
-        // the tile's leaf counts -> LDS (lane fl of block f holds family 16 f + fl)
-        for (int i = threadIdx.x; i < p.n_leaves * FW; i += 64 * W) {
-            const int f = i & (FW - 1);
+        const StepDev* __restrict__ steps = p.steps + (p.units ? bk.step0 : 0);
+        const int n_steps = p.units ? bk.n_steps : p.n_steps;
+        const int n_cols = p.units ? bk.n_cols : p.n_leaves;
+        // the tile's leaf and pattern columns -> LDS (lane fl of block f holds family 16 f + fl)
+        for (int i = threadIdx.x; i < n_cols * FW; i += 64 * W) {
+            const int f = i & (FW - 1), c = i / FW;
             const int ff = f < nf ? f : 0;
             const int fam = td.nf < 0 ? p.fam_list[td.fam0 + ff] : bk.fam_begin + td.fam0 + ff;
-            s_cnt[i] = p.counts_T[(long long)(i / FW) * p.F + fam];
+            const ColDev cd = p.units ? p.cols[bk.col0 + c] : ColDev{c, 0};
+            const int id = p.counts_T[(long long)cd.row * p.F + fam];
+            s_cnt[i] = id * (cd.stride ? cd.stride : Np);
         }
+        if (p.units)   // the pattern columns' exponents and bounds
+            for (int st = wv; st < n_steps; st += W) {
+                const StepDev sd = ld_const(steps, __builtin_amdgcn_readfirstlane(st));
+                if (!(sd.ctl & kStepPattern) || lane >= FW) continue;
+                const UnitDev u = ld_const(p.units, sd.in_slot);
+                const int ff = lane < nf ? lane : 0;
+                const int fam = td.nf < 0 ? p.fam_list[td.fam0 + ff] : bk.fam_begin + td.fam0 + ff;
+                const long long at = u.m0 + (long long)td.point * u.n +
+                                     p.counts_T[(long long)p.cols[bk.col0 + sd.leaf_col].row * p.F + fam];
+                m_pc[sd.leaf_col * FW + lane] = p.xm_c[at];
+                m_pe[sd.leaf_col * FW + lane] = p.xm_e[at];
+            }
         __syncthreads();   // counts visible
         bool valid[FB];
         int dst[FB];
@@ -348,17 +367,21 @@ void k_prune_mfma(PruneParams p)
             // wave-uniform index: the descriptor comes through the scalar
             // cache, so waiting for it does not wait for vector loads
             st = __builtin_amdgcn_readfirstlane(st < n_steps ? st : n_steps - 1);
-            sd = ld_const(p.steps, st);
+            sd = ld_const(steps, st);
             const bool root = (sd.ctl & kStepRoot) != 0;
             const bool leaf = sd.leaf_col >= 0;
             const int slot = nslot[sd.node];
             const float* __restrict__ M = (leaf ? lpool : pool) + (long long)slot * p.slot_elems;
+            if (sd.ctl & kStepPattern) {
+                const UnitDev u = ld_const(p.units, sd.in_slot);
+                M = p.x32 + u.x0 + (long long)td.point * u.n * u.xs;
+            }
             klo = 0;
             kn = nts;
             if (!leaf) kband(slot, root, klo, kn);
 #pragma unroll
             for (int k = 0; k < PK; ++k) {
-                const int cn = s_cnt[(leaf ? sd.leaf_col : 0) * FW + (FB > 1 ? 16 * k : 0) + fl] * Np;
+                const int cn = s_cnt[(leaf ? sd.leaf_col : 0) * FW + (FB > 1 ? 16 * k : 0) + fl];
 #pragma unroll
                 for (int i = 0; i < NTW; ++i) {
                     const int oa = root ? offA1[i] : offA0[i];
@@ -415,12 +438,21 @@ void k_prune_mfma(PruneParams p)
             }
             V4 x[FB][NTW];
             if (sd.leaf_col >= 0) {
+                if (sd.ctl & kStepPattern) {   // a unit's factor: an interior child's terms
 #pragma unroll
-                for (int f = 0; f < FB; ++f) {
-                    e_sum[f] -= kMatExp;
-                    cert[f] += leaf_cert;
+                    for (int f = 0; f < FB; ++f) {
+                        e_sum[f] += m_pe[sd.leaf_col * FW + 16 * f + fl];
+                        cert[f] += m_pc[sd.leaf_col * FW + 16 * f + fl];
+                    }
+                    log2S += kMatExp + a_exp;
+                } else {
+#pragma unroll
+                    for (int f = 0; f < FB; ++f) {
+                        e_sum[f] -= kMatExp;
+                        cert[f] += leaf_cert;
+                    }
+                    log2S += kMatExp;
                 }
-                log2S += kMatExp;
 #pragma unroll
                 for (int f = 0; f < FB; ++f)
 #pragma unroll
@@ -477,6 +509,23 @@ void k_prune_mfma(PruneParams p)
                 for (int i = 0; i < NTW; ++i) acc[f][i] *= x[f][i];
             if (!(sd.ctl & kStepLast)) return;
 
+            if (sd.ctl & kStepOut) {   // the branch's factor (1 x, from its one step) as columns
+                const UnitDev u = ld_const(p.units, bk.out);
+                const long long at = (long long)td.point * u.n + td.fam0 - bk.list0;
+#pragma unroll
+                for (int f = 0; f < FB; ++f) {
+                    if (!valid[f]) continue;
+                    const long long c = at + 16 * f + fl;
+#pragma unroll
+                    for (int i = 0; i < NTW; ++i)
+                        if (live[i]) *(V4*)(p.x32 + u.x0 + c * u.xs + kTile * tt[i] + 4 * g) = acc[f][i];
+                    if (wv == 0 && g == 0) {
+                        p.xm_e[u.m0 + c] = e_sum[f];
+                        p.xm_c[u.m0 + c] = cert[f];
+                    }
+                }
+                return;
+            }
             if (!root) {
                 float wmax[FB];
 #pragma unroll
