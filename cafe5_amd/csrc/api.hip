@@ -115,20 +115,58 @@ struct DevBuf {
     template <typename T> T* as() const { return (T*)p; }
 };
 
+// Grow-only pinned host memory.
+struct PinnedBuf {
+    char* p = nullptr;
+    size_t bytes = 0;
+    hipError_t ensure(size_t need)
+    {
+        if (need <= bytes) return hipSuccess;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        bytes = 0;
+        hipError_t e = hipHostMalloc((void**)&p, need);
+        if (e == hipSuccess) bytes = need;
+        return e;
+    }
+    void release()
+    {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
+};
+
 struct BucketHost {
     int B, R, count, fam_begin, max_count;
 };
 
+// A table of an evaluation's input block.
+struct DevView {
+    void* p = nullptr;
+    template <typename T> T* as() const { return (T*)p; }
+};
+
 // Device buffers of one evaluation (eager calls or a plan).
 struct EvalBufs {
-    DevBuf node_slot, prior64, prior32, catp, buckets, tiles, ntiles, fb_tiles, fb_count, val,
-        flag, lnl, cat, post, fail, total, scratch, root, segs, class_off, fam_list, units, cols_x, cols_meta;
-    std::vector<BucketDev> bucket_h;   // the bucket table (plan_prune adds the programs and units, and uploads it)
+    DevBuf fb_tiles, fb_count, val, flag, lnl, cat, post, fail, total, scratch, root, fam_list, cols_x, cols_meta;
+    // the inputs: put() together on the host, then one block (commit_inputs)
+    DevBuf inputs;
+    DevView node_slot, prior64, prior32, catp, buckets, tiles, ntiles, segs, class_off, units;
+    std::vector<char> block;
+    std::vector<std::pair<DevView*, size_t>> views;
+    std::vector<BucketDev> bucket_h;   // the bucket table (plan_prune adds the programs and units)
+    void put(DevView& v, const void* src, size_t bytes)
+    {
+        const size_t at = align256(block.size());
+        block.resize(at + bytes);
+        if (bytes) memcpy(block.data() + at, src, bytes);
+        views.push_back({&v, at});
+    }
     void release_all()
     {
-        DevBuf* all[] = {&node_slot, &prior64, &prior32, &catp, &buckets, &tiles, &ntiles, &fb_tiles,
-                         &fb_count, &val, &flag, &lnl, &cat, &post, &fail, &total, &scratch, &root, &segs,
-                         &class_off, &fam_list, &units, &cols_x, &cols_meta};
+        DevBuf* all[] = {&fb_tiles, &fb_count, &val, &flag, &lnl, &cat, &post, &fail, &total, &scratch, &root,
+                         &fam_list, &cols_x, &cols_meta, &inputs};
         for (DevBuf* b : all) b->release();
     }
 };
@@ -180,13 +218,16 @@ struct cafe_gpu_ctx {
     std::vector<hipEvent_t> join_ev;
     hipEvent_t ev[6] = {};
     double timings[4] = {0, 0, 0, 0};
-    bool build_timed = false;
+    bool build_timed = false;   // ev[4], ev[5] bracket a build that timings[0] does not hold yet
+    PinnedBuf stage_in;         // uploads; stage_ev: the last one has left it
+    hipEvent_t stage_ev = nullptr;
+    PinnedBuf stage_out;        // downloads
     DevBuf lg;
 
     // matrix pool
     int N = 0, Np = 0, capacity = 0;
     long long slot_elems = 0;
-    DevBuf mt64, mt32, lf32, key_lam, key_t;
+    DevBuf mt64, mt32, lf32, keys;
     DevBuf band32;         // per slot and 16-row tile of mt32: its nonzero k-tiles (band_entry)
     DevBuf mt16h, mt16l;   // split-FP16 halves of mt32 (BATCHED16; made by its evaluations)
     std::vector<char> built;   // per slot: 0 no, 1 every copy, 2 FP64 and the FP32 copies a plan read
@@ -243,6 +284,63 @@ int check_ctx(cafe_gpu_ctx* ctx)
 {
     if (!ctx) return fail(CAFE_GPU_EINVAL, "null context");
     if (hipSetDevice(ctx->device) != hipSuccess) return fail(CAFE_GPU_EDEVICE, "hipSetDevice failed");
+    return CAFE_GPU_OK;
+}
+
+// Host transfers go through pinned memory on the context's stream: a copy from
+// or to pageable memory is staged by the runtime in small pieces, waits for the
+// device each time (10 us and more per table; 85 us per MB), and is not ordered
+// with the stream.
+
+// Enqueues a copy of `bytes` at src to the device; src is free on return.
+int upload(cafe_gpu_ctx* ctx, void* dst, const void* src, size_t bytes)
+{
+    if (!bytes) return CAFE_GPU_OK;
+    HIP_OR_FAIL(hipEventSynchronize(ctx->stage_ev));   // (an event never recorded is complete)
+    HIP_OR_FAIL(ctx->stage_in.ensure(std::max<size_t>(bytes, 64 * 1024)));
+    memcpy(ctx->stage_in.p, src, bytes);
+    HIP_OR_FAIL(hipMemcpyAsync(dst, ctx->stage_in.p, bytes, hipMemcpyHostToDevice, ctx->stream));
+    HIP_OR_FAIL(hipEventRecord(ctx->stage_ev, ctx->stream));
+    return CAFE_GPU_OK;
+}
+
+// The evaluation's input tables as one block.
+int commit_inputs(cafe_gpu_ctx* ctx, EvalBufs& b)
+{
+    HIP_OR_FAIL(b.inputs.ensure(std::max<size_t>(b.block.size(), 256)));
+    if (int rc = upload(ctx, b.inputs.p, b.block.data(), b.block.size())) return rc;
+    for (auto& v : b.views) v.first->p = (char*)b.inputs.p + v.second;
+    return CAFE_GPU_OK;
+}
+
+// Device to host, after the stream's work so far; returns with the data.  Copies
+// from kDirectCopy on go to their place at once (the runtime pins it; through
+// here 3 MB of root vectors took 640 us, this way 360), smaller ones through
+// the staging buffer (200 KB: 775 us a step against 865).
+struct Fetch {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+constexpr size_t kDirectCopy = (size_t)256 << 10;
+constexpr size_t kStageOut = 8 * kDirectCopy;   // a list has at most five
+
+int fetch(cafe_gpu_ctx* ctx, const std::vector<Fetch>& list)
+{
+    size_t used = 0;
+    for (const Fetch& f : list) {
+        const bool staged = f.bytes < kDirectCopy && used + f.bytes <= kStageOut;
+        HIP_OR_FAIL(hipMemcpyAsync(staged ? ctx->stage_out.p + used : f.dst, f.src, f.bytes, hipMemcpyDeviceToHost,
+                                   ctx->stream));
+        if (staged) used += align256(f.bytes);
+    }
+    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
+    used = 0;
+    for (const Fetch& f : list) {
+        if (!(f.bytes < kDirectCopy && used + f.bytes <= kStageOut)) continue;
+        memcpy(f.dst, ctx->stage_out.p + used, f.bytes);
+        used += align256(f.bytes);
+    }
     return CAFE_GPU_OK;
 }
 
@@ -668,6 +766,7 @@ int cafe_gpu_create(int device, cafe_gpu_ctx** out)
         return fail(CAFE_GPU_EDEVICE, "hipStreamCreate failed");
     }
     for (auto& e : ctx->ev) (void)hipEventCreate(&e);
+    (void)hipEventCreateWithFlags(&ctx->stage_ev, hipEventDisableTiming);
     ctx->side.assign(kSideStreams, nullptr);
     for (auto& st : ctx->side)
         if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) {
@@ -690,6 +789,11 @@ int cafe_gpu_create(int device, cafe_gpu_ctx** out)
         cafe_gpu_destroy(ctx);
         return fail(CAFE_GPU_ENOMEM, "log-gamma table upload failed");
     }
+    // (here, so that the calls that allocate nothing find it)
+    if (ctx->stage_out.ensure(kStageOut) != hipSuccess) {
+        cafe_gpu_destroy(ctx);
+        return fail(CAFE_GPU_ENOMEM, "pinned staging buffer");
+    }
     *out = ctx;
     return CAFE_GPU_OK;
 }
@@ -699,7 +803,7 @@ int cafe_gpu_destroy(cafe_gpu_ctx* ctx)
     if (!ctx) return CAFE_GPU_OK;
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    DevBuf* bufs[] = {&ctx->lg, &ctx->mt64, &ctx->mt32, &ctx->lf32, &ctx->key_lam, &ctx->key_t, &ctx->d_ops,
+    DevBuf* bufs[] = {&ctx->lg, &ctx->mt64, &ctx->mt32, &ctx->lf32, &ctx->keys, &ctx->d_ops,
                       &ctx->d_kids, &ctx->d_steps, &ctx->d_steps_lane, &ctx->d_steps_hot, &ctx->d_counts, &ctx->d_perm, &ctx->d_err64,
                       &ctx->d_err32, &ctx->mt64e, &ctx->mt32e, &ctx->mt16h, &ctx->mt16l, &ctx->band32};
     for (DevBuf* b : bufs) b->release();
@@ -709,6 +813,9 @@ int cafe_gpu_destroy(cafe_gpu_ctx* ctx)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : ctx->join_ev)
         if (e) (void)hipEventDestroy(e);
+    if (ctx->stage_ev) (void)hipEventDestroy(ctx->stage_ev);
+    ctx->stage_in.release();
+    ctx->stage_out.release();
     for (auto& st : ctx->side)
         if (st) {
             (void)hipStreamSynchronize(st);
@@ -730,6 +837,7 @@ int cafe_gpu_matrix_reset(cafe_gpu_ctx* ctx, int N, int capacity)
     const size_t n32 = sizeof(float) * slot_elems * capacity;
     // every plan made over the old pool is stale from here on, and until the
     // new pool is complete the context has none
+    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
     ctx->pool_gen++;
     ctx->N = ctx->Np = ctx->capacity = 0;
     ctx->slot_elems = 0;
@@ -773,21 +881,20 @@ int cafe_gpu_matrix_build(cafe_gpu_ctx* ctx, int n, const double* lambda_q, cons
     for (int i = 0; i < n; ++i)
         if (!(lambda_q[i] >= 0) || !(t_q[i] >= 0) || !std::isfinite(lambda_q[i]) || !std::isfinite(t_q[i]))
             return fail(CAFE_GPU_EINVAL, "key %d has an invalid lambda or branch length", i);
-    HIP_OR_FAIL(ctx->key_lam.ensure(sizeof(double) * n));
-    HIP_OR_FAIL(ctx->key_t.ensure(sizeof(double) * n));
-    HIP_OR_FAIL(hipMemcpyAsync(ctx->key_lam.p, lambda_q, sizeof(double) * n, hipMemcpyHostToDevice, ctx->stream));
-    HIP_OR_FAIL(hipMemcpyAsync(ctx->key_t.p, t_q, sizeof(double) * n, hipMemcpyHostToDevice, ctx->stream));
+    HIP_OR_FAIL(ctx->keys.ensure(sizeof(double) * 2 * n));
+    double* d_lam = ctx->keys.as<double>();
+    double* d_t = d_lam + n;
+    std::vector<double> both(lambda_q, lambda_q + n);
+    both.insert(both.end(), t_q, t_q + n);
+    if (int rc = upload(ctx, d_lam, both.data(), sizeof(double) * 2 * n)) return rc;
     HIP_OR_FAIL(hipEventRecord(ctx->ev[4], ctx->stream));
-    HIP_OR_FAIL(launch_build(algo, ctx->key_lam.as<double>(), ctx->key_t.as<double>(), ctx->lg.as<double>(), n,
+    HIP_OR_FAIL(launch_build(algo, d_lam, d_t, ctx->lg.as<double>(), n,
                              first_slot, ctx->N, ctx->Np, ctx->slot_elems, ctx->mt64.as<double>(),
                              ctx->mt32.as<float>(), ctx->lf32.as<float>(), ctx->stream, nullptr, 0,
                              ctx->band32.as<int>()));
     if (int rc = enqueue_fold(ctx, first_slot, n, ctx->stream)) return rc;
     HIP_OR_FAIL(hipEventRecord(ctx->ev[5], ctx->stream));
-    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
-    float ms = 0;
-    (void)hipEventElapsedTime(&ms, ctx->ev[4], ctx->ev[5]);
-    ctx->timings[0] = ms;
+    ctx->build_timed = true;   // (everything that reads the matrices runs on the stream)
     for (int i = 0; i < n; ++i) ctx->built[first_slot + i] = 1;
     return CAFE_GPU_OK;
 }
@@ -800,8 +907,9 @@ int cafe_gpu_matrix_get(cafe_gpu_ctx* ctx, int slot, double* out)
         return fail(CAFE_GPU_ENOTFOUND, "matrix slot %d is not built", slot);
     const int N = ctx->N, Np = ctx->Np;
     std::vector<double> cm((size_t)N * Np);
-    HIP_OR_FAIL(hipMemcpy(cm.data(), ctx->mt64.as<double>() + (long long)slot * ctx->slot_elems,
-                          sizeof(double) * cm.size(), hipMemcpyDeviceToHost));
+    if (int rc = fetch(ctx, {{cm.data(), ctx->mt64.as<double>() + (long long)slot * ctx->slot_elems,
+                              sizeof(double) * cm.size()}}))
+        return rc;
     for (int s = 0; s < N; ++s)
         for (int c = 0; c < N; ++c) out[(size_t)s * N + c] = cm[(size_t)c * Np + s];
     return CAFE_GPU_OK;
@@ -854,6 +962,7 @@ int cafe_gpu_set_tree(cafe_gpu_ctx* ctx, int n_nodes, const int* parent, const i
     ph.emit(root, false);
     if (pl.max_slot + 1 > kMaxSlots)
         return fail(CAFE_GPU_EINVAL, "tree needs %d live partial vectors (max %d)", pl.max_slot + 1, kMaxSlots);
+    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));   // nothing reads what is replaced here
     ctx->input_gen++;
     ctx->pat.clear();
     ctx->n_nodes = n_nodes;
@@ -924,6 +1033,7 @@ int cafe_gpu_set_families(cafe_gpu_ctx* ctx, int F, int n_leaves, const int* cou
         b.count++;
         b.max_count = std::max(b.max_count, top[f]);
     }
+    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
     ctx->input_gen++;
     ctx->pat.clear();
     std::vector<int> cT((size_t)n_leaves * F);
@@ -971,6 +1081,7 @@ int cafe_gpu_set_error_model(cafe_gpu_ctx* ctx, int n_dev, int n_rows, const dou
     if (n_dev < 1 || n_dev % 2 == 0 || n_rows < 1)
         return fail(CAFE_GPU_EINVAL, "error model needs an odd number of deviations and >= 1 row");
     if (n_dev != ctx->n_dev || n_rows != ctx->err_rows) ctx->input_gen++;   // same shape: in place
+    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
     const size_t n = (size_t)n_dev * n_rows;
     std::vector<float> r32(rows, rows + n);
     HIP_OR_FAIL(ctx->d_err64.ensure(sizeof(double) * n));
@@ -1312,8 +1423,9 @@ int apply_tuning(cafe_gpu_ctx* ctx, int path, KernelClass& kc, unsigned long lon
     return CAFE_GPU_OK;
 }
 
-// Validates a descriptor and uploads node slots, priors, bucket table and
-// category probabilities into b; sizes the per-point outputs.
+// Validates a descriptor and puts node slots, priors and category probabilities
+// into b's input block (plan_prune completes and uploads it); sizes the
+// per-point outputs.
 int upload_eval_inputs(cafe_gpu_ctx* ctx, EvalBufs& b, const cafe_gpu_eval_desc* d, int& P)
 {
     if (!d) return fail(CAFE_GPU_EINVAL, "null descriptor");
@@ -1382,14 +1494,12 @@ int upload_eval_inputs(cafe_gpu_ctx* ctx, EvalBufs& b, const cafe_gpu_eval_desc*
     for (size_t i = 0; i < pr64.size(); ++i) pr32[i] = (float)pr64[i];
     std::vector<double> cp(K, 1.0);
     if (d->cat_probs) cp.assign(d->cat_probs, d->cat_probs + K);
-    HIP_OR_FAIL(b.node_slot.ensure(sizeof(int) * ns));
-    HIP_OR_FAIL(b.prior64.ensure(sizeof(double) * pr64.size()));
-    HIP_OR_FAIL(b.prior32.ensure(sizeof(float) * pr32.size()));
-    HIP_OR_FAIL(b.catp.ensure(sizeof(double) * K));
-    HIP_OR_FAIL(hipMemcpy(b.node_slot.p, slot.data(), sizeof(int) * ns, hipMemcpyHostToDevice));
-    HIP_OR_FAIL(hipMemcpy(b.prior64.p, pr64.data(), sizeof(double) * pr64.size(), hipMemcpyHostToDevice));
-    HIP_OR_FAIL(hipMemcpy(b.prior32.p, pr32.data(), sizeof(float) * pr32.size(), hipMemcpyHostToDevice));
-    HIP_OR_FAIL(hipMemcpy(b.catp.p, cp.data(), sizeof(double) * K, hipMemcpyHostToDevice));
+    b.block.clear();
+    b.views.clear();
+    b.put(b.node_slot, slot.data(), sizeof(int) * ns);
+    b.put(b.prior64, pr64.data(), sizeof(double) * pr64.size());
+    b.put(b.prior32, pr32.data(), sizeof(float) * pr32.size());
+    b.put(b.catp, cp.data(), sizeof(double) * K);
     const size_t PF = (size_t)P * ctx->F;
     HIP_OR_FAIL(b.val.ensure(sizeof(double) * PF));
     HIP_OR_FAIL(b.flag.ensure(sizeof(int) * PF));
@@ -1701,30 +1811,20 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     pp.r16_total = class_off[n_cls];
     pp.n_segs = (int)segs.size();
 
-    HIP_OR_FAIL(b.tiles.ensure(sizeof(TileDesc) * std::max<size_t>(1, tiles.size())));
     HIP_OR_FAIL(b.fb_tiles.ensure(sizeof(TileDesc) * (size_t)std::max(1, pp.r16_total)));
-    HIP_OR_FAIL(b.ntiles.ensure(sizeof(int) * pp.class_counts.size()));
     HIP_OR_FAIL(b.fb_count.ensure(sizeof(int) * (n_cls + 2)));
-    HIP_OR_FAIL(b.segs.ensure(sizeof(SegDesc) * std::max(1, pp.n_segs)));
-    HIP_OR_FAIL(b.class_off.ensure(sizeof(int) * (n_cls + 1)));
-    {
-        size_t maxp = 0;
-        for (int i = 0; i < n_points; ++i) maxp = std::max(maxp, (size_t)point_ids[i] + 1);
-        HIP_OR_FAIL(b.fam_list.ensure(sizeof(int) * maxp * (size_t)ctx->F));
-    }
-    HIP_OR_FAIL(hipMemcpy(b.tiles.p, tiles.data(), sizeof(TileDesc) * tiles.size(), hipMemcpyHostToDevice));
-    HIP_OR_FAIL(b.buckets.ensure(sizeof(BucketDev) * bd.size()));
-    HIP_OR_FAIL(hipMemcpy(b.buckets.p, bd.data(), sizeof(BucketDev) * bd.size(), hipMemcpyHostToDevice));
+    HIP_OR_FAIL(b.fam_list.ensure(sizeof(int) * (size_t)max_point * (size_t)ctx->F));
+    b.put(b.tiles, tiles.data(), sizeof(TileDesc) * tiles.size());
+    b.put(b.ntiles, pp.class_counts.data(), sizeof(int) * pp.class_counts.size());
+    b.put(b.segs, segs.data(), sizeof(SegDesc) * pp.n_segs);
+    b.put(b.class_off, class_off.data(), sizeof(int) * (n_cls + 1));
+    b.put(b.buckets, bd.data(), sizeof(BucketDev) * bd.size());
     if (pat_bytes > 0) {
-        HIP_OR_FAIL(b.units.ensure(sizeof(UnitDev) * units.size()));
-        HIP_OR_FAIL(hipMemcpy(b.units.p, units.data(), sizeof(UnitDev) * units.size(), hipMemcpyHostToDevice));
+        b.put(b.units, units.data(), sizeof(UnitDev) * units.size());
         HIP_OR_FAIL(b.cols_x.ensure(sizeof(double) * n64 + sizeof(float) * n32 * (path == CAFE_GPU_PATH_BATCHED16 ? 2 : 1)));
         HIP_OR_FAIL(b.cols_meta.ensure((sizeof(double) + sizeof(int)) * n_meta));
     }
-    HIP_OR_FAIL(hipMemcpy(b.ntiles.p, pp.class_counts.data(), sizeof(int) * pp.class_counts.size(),
-                          hipMemcpyHostToDevice));
-    HIP_OR_FAIL(hipMemcpy(b.segs.p, segs.data(), sizeof(SegDesc) * pp.n_segs, hipMemcpyHostToDevice));
-    HIP_OR_FAIL(hipMemcpy(b.class_off.p, class_off.data(), sizeof(int) * (n_cls + 1), hipMemcpyHostToDevice));
+    if (int rc = commit_inputs(ctx, b)) return rc;
 
     // Global scratch: per class and pass (classes of one pass run
     // concurrently, passes one after another).
@@ -1952,18 +2052,14 @@ int copy_results(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, int model,
                  double* cat, double* post, double* total, long long* n_fallback)
 {
     const size_t TF = (size_t)T * ctx->F;
-    hipStream_t st = ctx->stream;
-    if (lnl) HIP_OR_FAIL(hipMemcpyAsync(lnl, b.lnl.p, sizeof(double) * TF, hipMemcpyDeviceToHost, st));
-    if (cat && model == CAFE_GPU_MODEL_GAMMA)
-        HIP_OR_FAIL(hipMemcpyAsync(cat, b.cat.p, sizeof(double) * TF * K, hipMemcpyDeviceToHost, st));
-    if (post && model == CAFE_GPU_MODEL_GAMMA)
-        HIP_OR_FAIL(hipMemcpyAsync(post, b.post.p, sizeof(double) * TF * K, hipMemcpyDeviceToHost, st));
-    if (total) HIP_OR_FAIL(hipMemcpyAsync(total, b.total.p, sizeof(double) * T, hipMemcpyDeviceToHost, st));
     int h[2] = {0, 0};
-    if (n_fallback)
-        HIP_OR_FAIL(hipMemcpyAsync(h, b.fb_count.as<int>() + pp.fam_count_off(), sizeof(int) * 2,
-                                   hipMemcpyDeviceToHost, st));
-    HIP_OR_FAIL(hipStreamSynchronize(st));
+    std::vector<Fetch> list;
+    if (total) list.push_back({total, b.total.p, sizeof(double) * T});
+    if (n_fallback) list.push_back({h, b.fb_count.as<int>() + pp.fam_count_off(), sizeof(int) * 2});
+    if (lnl) list.push_back({lnl, b.lnl.p, sizeof(double) * TF});
+    if (cat && model == CAFE_GPU_MODEL_GAMMA) list.push_back({cat, b.cat.p, sizeof(double) * TF * K});
+    if (post && model == CAFE_GPU_MODEL_GAMMA) list.push_back({post, b.post.p, sizeof(double) * TF * K});
+    if (int rc = fetch(ctx, list)) return rc;
     if (n_fallback) *n_fallback = (long long)h[0] + (long long)h[1];
     return CAFE_GPU_OK;
 }
@@ -2107,6 +2203,7 @@ int reconstruct_impl(cafe_gpu_ctx* ctx, const int* node_slot, const double* prio
         HIP_OR_FAIL(launch_block_max(d_prog, n_prog, ctx->mt64.as<double>(), ctx->Np, ctx->slot_elems, Lp, tab, st));
     // large families first: their products fall off later, so they take several
     // times longer, and four of a size share a wave's matrix blocks
+    int flag = 0;
     std::vector<int2> fams(held);
     std::vector<int> at(ctx->N + 1);
     for (size_t h0 = 0; h0 < (size_t)nf; h0 += held) {
@@ -2123,12 +2220,10 @@ int reconstruct_impl(cafe_gpu_ctx* ctx, const int* node_slot, const double* prio
                                            (const int2*)(base + o_fam) + c0, (int)std::min(chunk, nh - c0),
                                            (const double*)(base + o_pri), B, Rr, rows, Lp, n,
                                            (int*)(base + o_st), (int*)(base + o_err), st));
-        HIP_OR_FAIL(hipMemcpyAsync(states + h0 * n, base + o_st, sizeof(int) * nh * n, hipMemcpyDeviceToHost, st));
-        HIP_OR_FAIL(hipStreamSynchronize(st));   // fams and the state rows are used again
+        // (fams and the state rows are used again)
+        if (int rc = fetch(ctx, {{states + h0 * n, base + o_st, sizeof(int) * nh * n}, {&flag, base + o_err, sizeof(int)}}))
+            return rc;
     }
-    int flag = 0;
-    HIP_OR_FAIL(hipMemcpyAsync(&flag, base + o_err, sizeof(flag), hipMemcpyDeviceToHost, st));
-    HIP_OR_FAIL(hipStreamSynchronize(st));
     if (flag) return fail(CAFE_GPU_EINVAL, "a leaf count is outside the matrices (N = %d)", ctx->N);
     return CAFE_GPU_OK;
 }
@@ -2141,7 +2236,9 @@ struct cafe_gpu_plan {
     EvalBufs bufs;
     PrunePlan pp;
     int model = 0, path = 0, T = 0, K = 0, n_keys = 0, algo = 0;
-    DevBuf d_lam, d_t;
+    DevBuf d_keys;           // lambdas, then branch lengths
+    double* lam() const { return d_keys.as<double>(); }
+    double* t() const { return d_keys.as<double>() + n_keys; }
     DevBuf d_copies;         // per key: the FP32 copies the plan's kernels read (kCopy* bits)
     int copy_top = 0;        // kCopyColTop: rows and columns of the per-lane classes
     long long pool_gen = 0, input_gen = 0;
@@ -2168,7 +2265,7 @@ int plan_enqueue(cafe_gpu_plan* pl, bool timed)
     const bool split = !timed && pl->algo != 0 && !pl->pp.has_f64 &&
                        (pl->pp.path == CAFE_GPU_PATH_BATCHED32 || pl->pp.path == CAFE_GPU_PATH_BATCHED16);
     if (timed) HIP_OR_FAIL(hipEventRecord(pl->ev[0], st));
-    HIP_OR_FAIL(launch_build(pl->algo, pl->d_lam.as<double>(), pl->d_t.as<double>(), ctx->lg.as<double>(), pl->n_keys,
+    HIP_OR_FAIL(launch_build(pl->algo, pl->lam(), pl->t(), ctx->lg.as<double>(), pl->n_keys,
                              0, ctx->N, ctx->Np, ctx->slot_elems, split ? nullptr : ctx->mt64.as<double>(),
                              ctx->mt32.as<float>(), ctx->lf32.as<float>(), st, pl->d_copies.as<unsigned char>(),
                              pl->copy_top, ctx->band32.as<int>()));
@@ -2177,7 +2274,7 @@ int plan_enqueue(cafe_gpu_plan* pl, bool timed)
     if (int rc = enqueue_fold(ctx, 0, pl->n_keys, st, !split, reduced)) return rc;
     if (timed) HIP_OR_FAIL(hipEventRecord(pl->ev[1], st));
     const std::function<int(hipStream_t)> build64 = [&](hipStream_t s) -> int {
-        HIP_OR_FAIL(launch_build(pl->algo, pl->d_lam.as<double>(), pl->d_t.as<double>(), ctx->lg.as<double>(),
+        HIP_OR_FAIL(launch_build(pl->algo, pl->lam(), pl->t(), ctx->lg.as<double>(),
                                  pl->n_keys, 0, ctx->N, ctx->Np, ctx->slot_elems, ctx->mt64.as<double>(), nullptr,
                                  nullptr, s, nullptr, 0, nullptr));
         return enqueue_fold(ctx, 0, pl->n_keys, s, true, false);
@@ -2305,15 +2402,18 @@ int cafe_gpu_root_vectors(cafe_gpu_ctx* ctx, const cafe_gpu_eval_desc* d, int tr
     PrunePlan pp;
     if (int rc = plan_prune(ctx, b, d->path, d->model, 1, &point, b.root.as<double>(), maxR, pp)) return rc;
     if (int rc = enqueue_prune(ctx, b, pp, ctx->stream, nullptr, nullptr, true)) return rc;
-    std::vector<double> h((size_t)ctx->F * maxR);
-    HIP_OR_FAIL(hipMemcpyAsync(h.data(), b.root.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
+    bool same = true;   // one R: the rows as they are
+    for (auto& bk : ctx->buckets) same = same && bk.R == maxR;
+    if (same)
+        return fetch(ctx, {{out, b.root.as<double>() + (size_t)f0 * maxR, sizeof(double) * (size_t)nf * maxR}});
+    std::vector<double> h((size_t)nf * maxR);
+    if (int rc = fetch(ctx, {{h.data(), b.root.as<double>() + (size_t)f0 * maxR, sizeof(double) * h.size()}})) return rc;
     std::vector<int> famR(ctx->F);
     for (auto& bk : ctx->buckets)
         for (int k = 0; k < bk.count; ++k) famR[ctx->perm[bk.fam_begin + k]] = bk.R;
     size_t o = 0;
     for (int f = f0; f < f0 + nf; ++f)
-        for (int j = 0; j < famR[f]; ++j) out[o++] = h[(size_t)f * maxR + j];
+        for (int j = 0; j < famR[f]; ++j) out[o++] = h[(size_t)(f - f0) * maxR + j];
     return CAFE_GPU_OK;
 }
 
@@ -2409,6 +2509,12 @@ int cafe_gpu_tuning_load(cafe_gpu_ctx* ctx, const char* path, int* n_loaded)
 int cafe_gpu_last_timings(cafe_gpu_ctx* ctx, double* ms4)
 {
     if (!ctx || !ms4) return fail(CAFE_GPU_EINVAL, "null argument");
+    if (ctx->build_timed) {
+        float ms = 0;
+        if (hipEventSynchronize(ctx->ev[5]) == hipSuccess && hipEventElapsedTime(&ms, ctx->ev[4], ctx->ev[5]) == hipSuccess)
+            ctx->timings[0] = ms;
+        ctx->build_timed = false;
+    }
     for (int i = 0; i < 4; ++i) ms4[i] = ctx->timings[i];
     return CAFE_GPU_OK;
 }
@@ -2437,8 +2543,7 @@ int cafe_gpu_plan_create(cafe_gpu_ctx* ctx, const cafe_gpu_eval_desc* d, int n_k
     std::vector<int> pts(P);
     std::iota(pts.begin(), pts.end(), 0);
     if (rc == CAFE_GPU_OK) rc = plan_prune(ctx, pl->bufs, d->path, d->model, P, pts.data(), nullptr, 0, pl->pp);
-    if (rc == CAFE_GPU_OK && (pl->d_lam.ensure(sizeof(double) * n_keys) != hipSuccess ||
-                              pl->d_t.ensure(sizeof(double) * n_keys) != hipSuccess))
+    if (rc == CAFE_GPU_OK && pl->d_keys.ensure(sizeof(double) * 2 * n_keys) != hipSuccess)
         rc = fail(CAFE_GPU_ENOMEM, "key upload buffers");
     if (rc != CAFE_GPU_OK) {
         pl->bufs.release_all();
@@ -2482,10 +2587,10 @@ int cafe_gpu_plan_set_keys(cafe_gpu_plan* pl, const double* lambda_q, const doub
         if (!(lambda_q[i] >= 0) || !(t_q[i] >= 0) || !std::isfinite(lambda_q[i]) || !std::isfinite(t_q[i]))
             return fail(CAFE_GPU_EINVAL, "key %d has an invalid lambda or branch length", i);
     HIP_OR_FAIL(hipSetDevice(pl->ctx->device));
-    HIP_OR_FAIL(hipStreamSynchronize(pl->ctx->stream));
-    HIP_OR_FAIL(hipMemcpy(pl->d_lam.p, lambda_q, sizeof(double) * pl->n_keys, hipMemcpyHostToDevice));
-    HIP_OR_FAIL(hipMemcpy(pl->d_t.p, t_q, sizeof(double) * pl->n_keys, hipMemcpyHostToDevice));
-    return CAFE_GPU_OK;
+    // (the executions before read theirs: the copy is behind them on the stream)
+    std::vector<double> both(lambda_q, lambda_q + pl->n_keys);
+    both.insert(both.end(), t_q, t_q + pl->n_keys);
+    return upload(pl->ctx, pl->lam(), both.data(), sizeof(double) * both.size());
 }
 
 int cafe_gpu_plan_execute(cafe_gpu_plan* pl)
@@ -2603,8 +2708,7 @@ int cafe_gpu_plan_destroy(cafe_gpu_plan* pl)
     for (auto& e : pl->cls_ev)
         if (e) (void)hipEventDestroy(e);
     pl->bufs.release_all();
-    pl->d_lam.release();
-    pl->d_t.release();
+    pl->d_keys.release();
     pl->d_copies.release();
     delete pl;
     return CAFE_GPU_OK;

@@ -75,9 +75,9 @@ class _ModelBase:
             eng.matrix_reset(self.N, max(len(lam_q), 1))
             eng._capacity = max(len(lam_q), 1)
         eng.matrix_build(lam_q, t_q, 0, self.build_algo)
-        self.build_ms = eng.timings()[0]
         res = eng.evaluate(slots, self._prior_table(prior), self.path, model, cat_probs)
-        self.prune_ms = eng.timings()[1:]
+        ms = eng.timings()
+        self.build_ms, self.prune_ms = ms[0], ms[1:]
         self.last = res
         return res
 

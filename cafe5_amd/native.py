@@ -377,12 +377,20 @@ class KeyTable:
 
     def node_slots(self, tree: Tree, node_lambdas: np.ndarray) -> np.ndarray:
         """node_lambdas: (P, n_nodes) lambda of every branch at every point."""
-        P = node_lambdas.shape[0]
-        out = np.zeros((P, tree.n_nodes), dtype=np.int32)
-        for p in range(P):
-            for i in range(tree.n_nodes):
-                if i != tree.root:
-                    out[p, i] = self.slot(float(node_lambdas[p, i]), float(tree.length[i]))
+        lams = np.asarray(node_lambdas, dtype=np.float64)
+        t = np.asarray(tree.length, dtype=np.float64)
+        out = np.zeros((lams.shape[0], tree.n_nodes), dtype=np.int32)
+        root = tree.root
+        branches = [i for i in range(tree.n_nodes) if i != root]
+        if not (np.isfinite(lams[:, branches]).all() and np.isfinite(t[branches]).all()):
+            for p, i in ((p, i) for p in range(lams.shape[0]) for i in branches):
+                out[p, i] = self.slot(float(lams[p, i]), float(t[i]))   # (raises at the first of them)
+            return out
+        # key_lambda and key_branch_length of all of them (+ 0.0: no negative zero)
+        tq = (np.trunc(t * 1000) / 1000.0 + 0.0)[branches].tolist()
+        keys = self.keys
+        for row, dst in zip((np.trunc(lams * 1000000000) / 1000000000.0 + 0.0)[:, branches].tolist(), out):
+            dst[branches] = [keys.setdefault(k, len(keys)) for k in zip(row, tq)]
         return out
 
     def arrays(self) -> Tuple[np.ndarray, np.ndarray]:
