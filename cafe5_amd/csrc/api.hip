@@ -23,6 +23,7 @@ hipError_t launch_build(int algo, const double* d_lam, const double* d_t, const 
                         int first_slot, int N, int Np, long long slot_elems, double* mt64, float* mt32,
                         float* lf32, hipStream_t stream, const unsigned char* copies, int top, int* band);
 hipError_t launch_fill_zero(void* p, long long bytes, hipStream_t stream);
+hipError_t launch_matrix_rows(const double* M, int N, int Np, double* out, hipStream_t stream);
 size_t recon_table_doubles(int n_prog, int Lp);
 hipError_t launch_block_max(const ReconNode* nodes, int n_prog, const double* mt64, int Np, long long slot_elems,
                             int Lp, double* tab, hipStream_t st);
@@ -227,7 +228,7 @@ struct cafe_gpu_ctx {
     // matrix pool
     int N = 0, Np = 0, capacity = 0;
     long long slot_elems = 0;
-    DevBuf mt64, mt32, lf32, keys;
+    DevBuf mt64, mt32, lf32, keys, get_rows;
     DevBuf band32;         // per slot and 16-row tile of mt32: its nonzero k-tiles (band_entry)
     DevBuf mt16h, mt16l;   // split-FP16 halves of mt32 (BATCHED16; made by its evaluations)
     std::vector<char> built;   // per slot: 0 no, 1 every copy, 2 FP64 and the FP32 copies a plan read
@@ -803,7 +804,7 @@ int cafe_gpu_destroy(cafe_gpu_ctx* ctx)
     if (!ctx) return CAFE_GPU_OK;
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    DevBuf* bufs[] = {&ctx->lg, &ctx->mt64, &ctx->mt32, &ctx->lf32, &ctx->keys, &ctx->d_ops,
+    DevBuf* bufs[] = {&ctx->lg, &ctx->mt64, &ctx->mt32, &ctx->lf32, &ctx->keys, &ctx->get_rows, &ctx->d_ops,
                       &ctx->d_kids, &ctx->d_steps, &ctx->d_steps_lane, &ctx->d_steps_hot, &ctx->d_counts, &ctx->d_perm, &ctx->d_err64,
                       &ctx->d_err32, &ctx->mt64e, &ctx->mt32e, &ctx->mt16h, &ctx->mt16l, &ctx->band32};
     for (DevBuf* b : bufs) b->release();
@@ -905,14 +906,11 @@ int cafe_gpu_matrix_get(cafe_gpu_ctx* ctx, int slot, double* out)
     if (!out) return fail(CAFE_GPU_EINVAL, "null output");
     if (slot < 0 || slot >= ctx->capacity || !ctx->built[slot])
         return fail(CAFE_GPU_ENOTFOUND, "matrix slot %d is not built", slot);
-    const int N = ctx->N, Np = ctx->Np;
-    std::vector<double> cm((size_t)N * Np);
-    if (int rc = fetch(ctx, {{cm.data(), ctx->mt64.as<double>() + (long long)slot * ctx->slot_elems,
-                              sizeof(double) * cm.size()}}))
-        return rc;
-    for (int s = 0; s < N; ++s)
-        for (int c = 0; c < N; ++c) out[(size_t)s * N + c] = cm[(size_t)c * Np + s];
-    return CAFE_GPU_OK;
+    const size_t bytes = sizeof(double) * (size_t)ctx->N * ctx->N;
+    HIP_OR_FAIL(ctx->get_rows.ensure(bytes));
+    HIP_OR_FAIL(launch_matrix_rows(ctx->mt64.as<double>() + (long long)slot * ctx->slot_elems, ctx->N, ctx->Np,
+                                   ctx->get_rows.as<double>(), ctx->stream));
+    return fetch(ctx, {{out, ctx->get_rows.p, bytes}});
 }
 
 int cafe_gpu_set_tree(cafe_gpu_ctx* ctx, int n_nodes, const int* parent, const int* leaf_col)

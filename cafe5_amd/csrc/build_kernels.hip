@@ -287,8 +287,13 @@ __global__ __launch_bounds__(64) void k_build_recurrence(const double* __restric
 // (s, c).  chooseln uses the host's glibc log-gamma table so the log-binomials
 // are the reference's values; terms are exp(t) * pow(coeff, j), added in
 // ascending j with separately rounded products and sums.
+//
+// Bound by FP64 vector instructions: min(s, c) + 1 terms per entry.  The powers
+// depend on the key and j only, so a block computes them once into LDS (a power
+// costs several times an exponential: 22 matrices of 201 sizes take 152 us, 309
+// with one per term), beside the part of the log-gamma table it reads.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double chooseln_dev(const double* __restrict__ lg, int n, int r)
+__device__ __forceinline__ double chooseln_dev(const double* lg, int n, int r)
 {
     if (r == 0) return 0.0;
     if (n <= 0 || r <= 0) return -__builtin_huge_val();
@@ -314,10 +319,18 @@ __global__ __launch_bounds__(256) void k_build_closed_form(const double* __restr
     if (band && mt32 && (use & kCopyRow) && c == 0 && blockIdx.x == 0)
         for (int t = threadIdx.x; t < band_stride; t += blockDim.x)
             band[(long long)(first_slot + key) * band_stride + t] = band_entry(0, band_stride);
-    if (s >= N) return;
     const double lt = lam_q[key] * t_q[key];
     const double alpha = lt / (1 + lt);
     const double coeff = 1 - 2 * alpha;
+    extern __shared__ double s_closed[];
+    double* s_pow = s_closed;        // [c + 1]: coeff^j
+    double* s_lg = s_closed + N;     // [2 N + 2]: log-gamma (sizes n + 1 <= s + c < 2 N)
+    if (!degenerate_key(alpha, coeff)) {
+        for (int j = threadIdx.x; j <= c; j += blockDim.x) s_pow[j] = pow(coeff, (double)j);
+        for (int j = threadIdx.x; j < 2 * N + 2; j += blockDim.x) s_lg[j] = lg[j];
+    }
+    __syncthreads();
+    if (s >= N) return;
     double v;
     if (s == 0) {
         v = (c == 0) ? 1.0 : 0.0;
@@ -328,10 +341,10 @@ __global__ __launch_bounds__(256) void k_build_closed_form(const double* __restr
         const int m = c < s ? c : s;
         double acc = 0.0;
         for (int j = 0; j <= m; ++j) {
-            const double t = __dadd_rn(__dadd_rn(chooseln_dev(lg, s, j),
-                                                 chooseln_dev(lg, s + c - 1 - j, s - 1)),
+            const double t = __dadd_rn(__dadd_rn(chooseln_dev(s_lg, s, j),
+                                                 chooseln_dev(s_lg, s + c - 1 - j, s - 1)),
                                        __dmul_rn((double)(s + c - 2 * j), log_alpha));
-            const double p = __dmul_rn(exp(t), pow(coeff, (double)j));
+            const double p = __dmul_rn(exp(t), s_pow[j]);
             acc = __dadd_rn(acc, p);
         }
         v = acc > 1.0 ? 1.0 : (acc < 0.0 ? 0.0 : acc);
@@ -396,6 +409,21 @@ __global__ __launch_bounds__(256) void k_fold_err32(const float* __restrict__ lf
     }
 }
 
+// One matrix out of its c-major slot, row-major without padding: 32 x 32 tiles
+// through LDS, so that both sides move whole lines (the host's strided copy of
+// 201 x 201 entries took longer than the transfer).
+__global__ __launch_bounds__(256) void k_matrix_rows(const double* __restrict__ M, int N, int Np, double* __restrict__ out)
+{
+    __shared__ double tile[32][33];
+    const int s0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
+    const int x = threadIdx.x & 31, y = threadIdx.x >> 5;
+    for (int k = y; k < 32; k += 8)
+        if (s0 + x < N && c0 + k < N) tile[k][x] = M[(long long)(c0 + k) * Np + s0 + x];
+    __syncthreads();
+    for (int k = y; k < 32; k += 8)
+        if (s0 + k < N && c0 + x < N) out[(long long)(s0 + k) * N + c0 + x] = tile[x][k];
+}
+
 // Zero-fill (used instead of hipMemsetAsync so the calls can be captured).
 __global__ void k_fill_zero_u32(uint32_t* __restrict__ p, long long n)
 {
@@ -426,7 +454,7 @@ hipError_t launch_build(int algo, const double* d_lam, const double* d_t, const 
         for (int k0 = 0; k0 < n; k0 += 65535) {
             const int nk = n - k0 < 65535 ? n - k0 : 65535;
             dim3 grid((N + 255) / 256, N, nk);
-            hipLaunchKernelGGL(k_build_closed_form, grid, dim3(256), 0, stream, d_lam + k0, d_t + k0,
+            hipLaunchKernelGGL(k_build_closed_form, grid, dim3(256), sizeof(double) * (3 * (size_t)N + 2), stream, d_lam + k0, d_t + k0,
                                d_lg, first_slot + k0, N, Np, slot_elems, mt64, mt32, lf32,
                                copies ? copies + k0 : nullptr, top, band, band_stride);
         }
@@ -467,6 +495,13 @@ hipError_t launch_fold(const double* mt64, const float* lf32, double* out64, flo
             hipLaunchKernelGGL(k_fold_err32, dim3(Np, nk), dim3(256), 0, stream, lf32, out32, err32, n_dev, n_rows,
                                N, Np, slot_elems, first_slot + k0);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_matrix_rows(const double* M, int N, int Np, double* out, hipStream_t stream)
+{
+    const int n = (N + 31) / 32;
+    hipLaunchKernelGGL(k_matrix_rows, dim3(n, n), dim3(256), 0, stream, M, N, Np, out);
     return hipGetLastError();
 }
 

@@ -163,7 +163,7 @@ class Engine:
         self._check(self.lib.cafe_gpu_matrix_build(self.ctx, len(lq), _dp(lq), _dp(tq), first_slot, algo))
 
     def matrix_get(self, slot: int) -> np.ndarray:
-        out = np.zeros((self.N, self.N))
+        out = np.empty((self.N, self.N))
         self._check(self.lib.cafe_gpu_matrix_get(self.ctx, slot, _dp(out)))
         return out
 
