@@ -2001,7 +2001,10 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
     // recomputes by their vectors' length) and st waits for all of them
     // before the next stage: a recompute is a latency-bound chain on a few
     // tiles, and beside a main pass it would slow that pass down.
-    const int S = concurrent ? std::min((int)ctx->side.size(), n_cls) : 0;
+    // (a single class still takes two streams when the FP64 pool is to be built
+    // beside its main pass: 2,000 families 221 -> 193 us a step)
+    const int S = concurrent ? std::min((int)ctx->side.size(), std::max(n_cls, late_build ? 2 : 0)) : 0;
+    const int light = n_cls == 1 ? S - 1 : pp.light_stream;
     if (late_build && S <= 1)
         if (int rc = (*late_build)(st)) return rc;
     using Launch = std::function<int(int, hipStream_t)>;
@@ -2023,7 +2026,7 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
             if (int rc = launch(ci, ctx->side[k])) return rc;
         }
         if (idx == 0 && late_build)
-            if (int rc = (*late_build)(ctx->side[pp.light_stream % S])) return rc;
+            if (int rc = (*late_build)(ctx->side[light % S])) return rc;
         for (int k = 0; k < S; ++k) {
             HIP_OR_FAIL(hipEventRecord(ev[1 + k], ctx->side[k]));
             HIP_OR_FAIL(hipStreamWaitEvent(st, ev[1 + k], 0));
