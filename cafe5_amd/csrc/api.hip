@@ -35,6 +35,9 @@ hipError_t launch_fold(const double* mt64, const float* lf32, double* out64, flo
                        const float* err32, int n_dev, int n_rows, int N, int Np, long long slot_elems,
                        int first_slot, int n, hipStream_t stream);
 hipError_t f64_dispatch(const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st, int* per_cu);
+int f64_level_stride(int nt);
+hipError_t launch_f64_levels(int nt, int max_tiles, const int* op_steps, const int* level_ops, int n_levels,
+                             const PruneParams& p, hipStream_t st);
 hipError_t launch_prune_mfma(const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st);
 hipError_t mfma_occupancy(const MfmaShape& s, int* per_cu);
 hipError_t f16_dispatch(const MfmaShape& s, int grid, const PruneParams& p, hipStream_t st, int* per_cu);
@@ -247,6 +250,10 @@ struct cafe_gpu_ctx {
     int n_slots_lane = 0;
     DevBuf d_steps_hot;      // and with the vector the next op reads kept in registers (per-lane kernel)
     int n_slots_hot = 0;
+    // and sorted by level (children's ops first), interior steps naming their
+    // child's op: the recompute of short lists
+    DevBuf d_steps_level, d_op_steps;
+    std::vector<int> level_ops;   // first op of every level, and the end
 
     // families
     int F = 0, n_leaves = 0;
@@ -805,7 +812,7 @@ int cafe_gpu_destroy(cafe_gpu_ctx* ctx)
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     DevBuf* bufs[] = {&ctx->lg, &ctx->mt64, &ctx->mt32, &ctx->lf32, &ctx->keys, &ctx->get_rows, &ctx->d_ops,
-                      &ctx->d_kids, &ctx->d_steps, &ctx->d_steps_lane, &ctx->d_steps_hot, &ctx->d_counts, &ctx->d_perm, &ctx->d_err64,
+                      &ctx->d_kids, &ctx->d_steps, &ctx->d_steps_lane, &ctx->d_steps_hot, &ctx->d_steps_level, &ctx->d_op_steps, &ctx->d_counts, &ctx->d_perm, &ctx->d_err64,
                       &ctx->d_err32, &ctx->mt64e, &ctx->mt32e, &ctx->mt16h, &ctx->mt16l, &ctx->band32};
     for (DevBuf* b : bufs) b->release();
     ctx->eager.release_all();
@@ -997,6 +1004,34 @@ int cafe_gpu_set_tree(cafe_gpu_ctx* ctx, int n_nodes, const int* parent, const i
     HIP_OR_FAIL(ctx->d_steps_hot.ensure(sizeof(StepDev) * hsteps.size()));
     HIP_OR_FAIL(hipMemcpy(ctx->d_steps_hot.p, hsteps.data(), sizeof(StepDev) * hsteps.size(),
                           hipMemcpyHostToDevice));
+    // level by level: an op's level is one past its interior children's
+    std::vector<int> level(n_nodes, 0), by_level(pl.ops.size()), op_of(n_nodes, -1);
+    for (const OpDev& op : pl.ops)   // (children before parents)
+        for (int c : kids[op.node])
+            if (lc[c] < 0) level[op.node] = std::max(level[op.node], level[c] + 1);
+    std::iota(by_level.begin(), by_level.end(), 0);
+    std::stable_sort(by_level.begin(), by_level.end(),
+                     [&](int a, int b) { return level[pl.ops[a].node] < level[pl.ops[b].node]; });
+    std::vector<StepDev> vsteps;
+    std::vector<int> op_steps;
+    ctx->level_ops.clear();
+    for (int i = 0; i < (int)by_level.size(); ++i) {
+        const OpDev& op = pl.ops[by_level[i]];
+        if (i == 0 || level[op.node] != level[pl.ops[by_level[i - 1]].node]) ctx->level_ops.push_back(i);
+        op_of[op.node] = i;
+        op_steps.push_back((int)vsteps.size());
+        for (int k = 0; k < op.n_child; ++k) {
+            const int c = pl.out_kids[op.child_begin + k].node;
+            vsteps.push_back(StepDev{c, lc[c], lc[c] >= 0 ? -1 : op_of[c],
+                                     (k == 0 ? kStepFirst : 0) | (k + 1 == op.n_child ? kStepLast : 0) |
+                                         (op.node == root ? kStepRoot : 0)});
+        }
+    }
+    ctx->level_ops.push_back((int)by_level.size());
+    HIP_OR_FAIL(ctx->d_steps_level.ensure(sizeof(StepDev) * vsteps.size()));
+    HIP_OR_FAIL(hipMemcpy(ctx->d_steps_level.p, vsteps.data(), sizeof(StepDev) * vsteps.size(), hipMemcpyHostToDevice));
+    HIP_OR_FAIL(ctx->d_op_steps.ensure(sizeof(int) * op_steps.size()));
+    HIP_OR_FAIL(hipMemcpy(ctx->d_op_steps.p, op_steps.data(), sizeof(int) * op_steps.size(), hipMemcpyHostToDevice));
     return CAFE_GPU_OK;
 }
 
@@ -1124,7 +1159,8 @@ struct KernelClass {
     // byte offsets of its global scratch in the main pass and the FP64
     // recompute: disjoint, since one class's recompute can run beside another
     // class's main pass
-    size_t off_main = 0, off_r64 = 0;
+    size_t off_main = 0, off_r64 = 0, off_level = 0;
+    int level_tiles = 0;   // most tiles its recompute takes level by level (0: none)
     int stream = 0;      // side stream of its launches
     // subtree patterns: its buckets run their programs over units' columns,
     // made level by level before the main pass (tiles, their count's place)
@@ -1326,6 +1362,11 @@ size_t f16_scratch_bytes(const MfmaShape& s, int n_slots, int slot_tiles, int gr
 // level of units is a launch more (2,000 families of 12 taxa at B = 100, three
 // levels: 305 -> 285 us a step).
 constexpr long long kPatternWork = 1024;
+// Recompute lists of vectors past LDS run level by level up to this many tiles
+// (256 families), with their vectors in at most kLevelBytes: shorter vectors'
+// chains are short (0.1 ms at 101 rows, 0.4 at 201) beside a launch per level.
+constexpr int kLevelTiles = 16;
+constexpr size_t kLevelBytes = (size_t)256 << 20;
 // Columns of one evaluation, at most.
 constexpr size_t kPatternBytes = (size_t)8 << 30;
 
@@ -1841,9 +1882,18 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
         if (!kc.f64) {
             kc.off_r64 = r64_sz;
             r64_sz += align256(f64_scratch_bytes(kc.r64, ctx->n_slots, kc.nt, pp.grid(kc.r64, kc.r16)));
+            if (!kc.r64.lds) {
+                const size_t tile = sizeof(double) * kTile * ctx->ops.size() * f64_level_stride(kc.nt);
+                kc.level_tiles = (int)std::min<size_t>(std::min(kLevelTiles, kc.r16), kLevelBytes / tile);
+                kc.off_level = r64_sz;
+                r64_sz += align256(tile * kc.level_tiles);
+            }
         }
     }
-    for (auto& kc : pp.classes) kc.off_r64 += main_sz;
+    for (auto& kc : pp.classes) {
+        kc.off_r64 += main_sz;
+        kc.off_level += main_sz;
+    }
     HIP_OR_FAIL(b.scratch.ensure(std::max<size_t>(main_sz + r64_sz, 256)));
 
     PruneParams& p = pp.base;
@@ -1989,6 +2039,15 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
         q.slot_tiles = kc.nt;
         q.scratch = scratch + kc.off_r64;
         q.near_floor = fbc + fam_off + 1;
+        // short lists level by level (which of the two works is decided on the device)
+        if (kc.level_tiles > 0) {
+            PruneParams a = q;
+            a.steps = ctx->d_steps_level.as<StepDev>();
+            a.scratch = scratch + kc.off_level;
+            HIP_OR_FAIL(launch_f64_levels(kc.nt, kc.level_tiles, ctx->d_op_steps.as<int>(), ctx->level_ops.data(),
+                                          (int)ctx->level_ops.size() - 1, a, s));
+            q.skip_tiles = kc.level_tiles;
+        }
         HIP_OR_FAIL(f64_dispatch(kc.r64, pp.grid(kc.r64, kc.r16), q, s, nullptr));
         return CAFE_GPU_OK;
     };

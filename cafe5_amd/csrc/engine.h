@@ -189,6 +189,7 @@ struct PruneParams {
     int n_slots;
     int slot_tiles;           // MFMA: 16-row tiles per stored partial vector
     int zero;                 // always 0 (an offset the compiler cannot fold)
+    int skip_tiles;           // FP64: a list of at most this many tiles is another launch's work
     int* near_floor;          // FP64: counts the families with values below kFp64Floor (null: not counted)
     // nonzero band of the FP32 row-major pool: per slot and 16-row tile t,
     // band[slot * band_stride + t] = lo | hi << 16, the k-tiles [lo, hi)

@@ -95,6 +95,7 @@ __global__ __launch_bounds__((64 * F64Waves<NTW, FB>::v)) void k_prune_f64(Prune
     // each XCD (workgroup b runs on b % 8) takes one contiguous range of the
     // list, whose neighbours share their matrices in its L2
     const int n_tiles = *as_const(p.n_tiles_dev);
+    if (n_tiles <= p.skip_tiles) return;   // launch_f64_levels'
     const int groups = (gridDim.x % 8 == 0) ? 8 : 1;
     const int per_group = gridDim.x / groups;
     const int grp = blockIdx.x % groups;
@@ -427,6 +428,158 @@ __global__ __launch_bounds__((64 * F64Waves<NTW, FB>::v)) void k_prune_f64(Prune
         }
         __syncthreads();   // every wave is done with this tile's LDS and vectors
     }
+}
+
+// ---------------------------------------------------------------------------
+// Short recompute lists of long vectors, level by level: a launch takes the ops
+// of one level of the tree (their children's vectors are complete), a wave 64
+// rows of one op for one family.  A contraction is its row's chain of fused
+// multiply-adds in ascending order -- the matrix instruction's sums, bit for
+// bit -- over the child's vector in LDS; vectors are in global memory.
+//
+// A few families are a chain of steps, and one CU's share of the memory system
+// bounds it: at 501 rows a step's matrix is 2 MB that no cache holds, 45 us at
+// what one CU can have in flight (59 on the matrix cores, sixteen families at
+// once whether they are there or not).  Spread over rows and branches, four
+// families of 100 taxa at B = 500 take 0.43 ms, against 4.4 one per workgroup
+// and 5.7 on the matrix cores.
+// ---------------------------------------------------------------------------
+constexpr int kLevelK = 32;   // columns per load group, two groups in flight
+
+__global__ __launch_bounds__(64) void k_f64_level(PruneParams p, const int* __restrict__ op_steps, int op0, int n_level,
+                                                  int n_ops, int max_tiles, int stride)
+{
+    const int n_tiles = *as_const(p.n_tiles_dev);
+    if (n_tiles > max_tiles) return;   // k_prune_f64's
+    extern __shared__ double s_vec[];   // [stride] a child's vector
+    const int lane = threadIdx.x, Np = p.Np;
+    const int chunks = (stride + 63) / 64;
+    double* V = (double*)p.scratch;     // [family of the list][op][stride]
+    const int n_items = n_tiles * kTile * n_level * chunks;
+    for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
+        const int op = op0 + item / chunks % n_level, fi = item / chunks / n_level;
+        const TileDesc td = ld_const(p.tiles, fi / kTile);
+        const int nf = td.nf < 0 ? -td.nf : td.nf;
+        if (fi % kTile >= nf) continue;
+        const BucketDev bk = ld_const(p.buckets, td.bucket);
+        const int ff = td.fam0 + fi % kTile;
+        const int fam = td.nf < 0 ? p.fam_list[ff] : bk.fam_begin + ff;
+        const int* nslot = p.node_slot + (long long)td.point * p.n_nodes;
+        double* Vf = V + (long long)fi * n_ops * stride;
+        const int row = item % chunks * 64 + lane;
+        double acc = 1.0;
+        bool root = false;
+        for (int st = op_steps[op];;) {
+            const StepDev sd = ld_const(p.steps, __builtin_amdgcn_readfirstlane(st++));
+            root = (sd.ctl & kStepRoot) != 0;
+            const int len = root ? bk.R : bk.L;   // (root rows are sizes 1..R)
+            const int r = row < len ? row : len - 1;
+            const long long base = (long long)nslot[sd.node] * p.slot_elems + (root ? 1 : 0) + r;
+            double x = 0.0;
+            if (sd.leaf_col >= 0) {
+                x = p.leaf64[base + (long long)p.counts_T[(long long)sd.leaf_col * p.F + fam] * Np];
+            } else {
+                const double* M = p.mt64 + base;
+                const int groups = (bk.L + kLevelK - 1) / kLevelK;   // (the vector's entries past the bound are 0)
+                double a[2][kLevelK];
+                auto load = [&](double (&m)[kLevelK], int gr) {
+                    const double* C = M + (long long)kLevelK * (gr < groups ? gr : groups - 1) * Np;
+#pragma unroll
+                    for (int k = 0; k < kLevelK; ++k) m[k] = C[(long long)k * Np];
+                };
+                auto sum = [&](const double (&m)[kLevelK], int gr) {
+                    const double* v = s_vec + kLevelK * gr;
+#pragma unroll
+                    for (int k = 0; k < kLevelK; ++k) x = fma(m[k], v[k], x);
+                };
+                load(a[0], 0);
+                const double* v = Vf + (long long)sd.in_slot * stride;
+                __syncthreads();
+                for (int k = lane; k < stride; k += 64) s_vec[k] = v[k];
+                __syncthreads();
+                for (int gr = 0; gr < groups; gr += 2) {
+                    load(a[1], gr + 1);
+                    sum(a[0], gr);
+                    if (gr + 1 >= groups) break;
+                    load(a[0], gr + 2);
+                    sum(a[1], gr + 1);
+                }
+            }
+            acc = sd.ctl & kStepFirst ? x : acc * x;
+            if (sd.ctl & kStepLast) break;
+        }
+        if (row < stride) Vf[(long long)op * stride + row] = row < (root ? bk.R : bk.L) ? acc : 0.0;
+    }
+}
+
+// The root's maximum of each family of the list, as k_prune_f64 takes it.
+__global__ __launch_bounds__(64) void k_f64_root(PruneParams p, int n_ops, int max_tiles, int stride)
+{
+    const int n_tiles = *as_const(p.n_tiles_dev);
+    if (n_tiles > max_tiles) return;
+    const int lane = threadIdx.x;
+    auto over_wave = [&](double v) {
+        for (int d = 1; d < 64; d <<= 1) {
+            const double o = __shfl_xor(v, d);
+            v = o > v ? o : v;
+        }
+        return v;
+    };
+    for (int fi = blockIdx.x; fi < n_tiles * kTile; fi += gridDim.x) {
+        const TileDesc td = ld_const(p.tiles, fi / kTile);
+        const int nf = td.nf < 0 ? -td.nf : td.nf;
+        if (fi % kTile >= nf) continue;
+        const BucketDev bk = ld_const(p.buckets, td.bucket);
+        const int ff = td.fam0 + fi % kTile;
+        const int dst = p.perm[td.nf < 0 ? p.fam_list[ff] : bk.fam_begin + ff];
+        const double* x = (const double*)p.scratch + ((long long)fi * n_ops + n_ops - 1) * stride;
+        const double* pr = p.prior64 + bk.prior_off;
+        const double inf = __builtin_huge_val();
+        double best = -inf, xmax = 0.0, val = -inf;
+        for (int j = lane; j < bk.R; j += 64) {
+            const double q = x[j] * pr[j];
+            best = q > best ? q : best;
+            xmax = x[j] > xmax ? x[j] : xmax;
+        }
+        best = over_wave(best);
+        xmax = over_wave(xmax);
+        if (p.model == 0) {
+            const bool every = !(best >= kFp64Floor && best < inf);
+            for (int j = lane; j < bk.R; j += 64)
+                if (every || x[j] * pr[j] >= best * kNearBest) {
+                    const double k = log(x[j]) + log(pr[j]);
+                    val = k > val ? k : val;
+                }
+            val = over_wave(val);
+        } else {
+            val = best;
+        }
+        if (lane == 0) {
+            const double k0 = p.model == 0 ? log(x[0]) + log(pr[0]) : x[0] * pr[0];
+            p.out_val[(long long)td.point * p.F + dst] = k0 != k0 ? k0 : val;
+            p.out_flag[(long long)td.point * p.F + dst] = xmax == 0.0 ? kFlagZeroSum : 0;
+            if (p.near_floor && (xmax < kFp64Floor || best < kFp64Floor)) atomicAdd(p.near_floor, 1);
+        }
+    }
+}
+
+// Entries of a vector of nt tiles, in whole load groups.
+int f64_level_stride(int nt) { return (nt * kTile + kLevelK - 1) / kLevelK * kLevelK; }
+
+// A list of at most max_tiles tiles (p.n_tiles_dev; a longer one is left to
+// k_prune_f64) over the program p.steps, whose interior steps name their
+// child's op in in_slot: op_steps[op] is an op's first step, level l's ops are
+// [level_ops[l], level_ops[l + 1]), the root's op the last.  p.scratch holds
+// kTile max_tiles n_ops vectors.
+hipError_t launch_f64_levels(int nt, int max_tiles, const int* op_steps, const int* level_ops, int n_levels,
+                             const PruneParams& p, hipStream_t st)
+{
+    const int stride = f64_level_stride(nt), n_ops = level_ops[n_levels];
+    for (int l = 0; l < n_levels; ++l)
+        hipLaunchKernelGGL(k_f64_level, dim3(2048), dim3(64), sizeof(double) * stride, st, p, op_steps, level_ops[l],
+                           level_ops[l + 1] - level_ops[l], n_ops, max_tiles, stride);
+    hipLaunchKernelGGL(k_f64_root, dim3(kTile * max_tiles), dim3(64), 0, st, p, n_ops, max_tiles, stride);
+    return hipGetLastError();
 }
 
 // One instance per shape; with per_cu set, reports how many workgroups of it
