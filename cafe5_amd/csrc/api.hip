@@ -1227,6 +1227,14 @@ MfmaShape mfma_shape(int nt)
     return s;
 }
 
+// FP32 launch shape of a plan with few families, whose time is the chain of
+// steps of the tiles each CU holds: one row tile per wave, as many waves as the
+// vector has tiles.  A score of 8,000 families of 34 taxa at B = 100 379 -> 312
+// us, 5,000 at 150 417 -> 381, 2,000 at 200 429 -> 366, 1,000 of 60 taxa at 120 983
+// -> 561; from about 32 families per CU on the wider shapes' fewer loads win
+// (200,000 gamma families: 0.94 ms against 1.25).
+MfmaShape mfma_shape_few(int nt) { return {1, nt <= 4 ? 4 : nt <= 8 ? 8 : 16, false, 0}; }
+
 // FP32 launch shape with 32-family tiles (two blocks of 16 per MFMA operand)
 // for vectors of up to 32 tiles (kMaxTilesFb2): two output tiles per wave
 // over 4, 8 or 16 waves (the products and factors of both blocks are held per
@@ -1324,7 +1332,8 @@ void place_partials(MfmaShape& s, int n_slots, int slot_tiles, int n_leaves, int
     if (s.fb > 1)   // two workgroups per CU, or one of 8 waves
         s.lds = s.w <= 8 && meta + frag + 4096 <= (s.w >= 8 ? 144 : 76) * 1024;
     else
-        s.lds = s.w <= 4 && meta + frag + 4096 <= 64 * 1024 && (meta + frag) / s.w <= 20 * 1024;
+        s.lds = (s.w <= 4 && meta + frag + 4096 <= 64 * 1024 && (meta + frag) / s.w <= 20 * 1024) ||
+                (s.w > 4 && s.ntw == 1 && meta + frag + 4096 <= 76 * 1024);   // (latency shapes)
     s.shm = meta + (s.lds ? frag : 0);
 }
 
@@ -1610,12 +1619,15 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     int n_mfma_keys = 0;
     for (const auto& kr : key_rows)
         if (lane_rows_of(kr.first) == 0) ++n_mfma_keys;
+    long long mfma_fams = 0;     // of all of them
     std::map<int, long long> key_fams;
     std::map<int, int> key_nt;   // and the tiles of its largest vector
     for (auto& bc : bucket_class) {
         key_fams[bc.first] += (long long)ctx->buckets[bc.second].count * n_points;
         key_nt[bc.first] = std::max(key_nt[bc.first], nt_of(ctx->buckets[bc.second]));
     }
+    for (const auto& kf : key_fams)
+        if (lane_rows_of(kf.first) == 0) mfma_fams += kf.second;
     // the plan's size classes, for the tuning entries measured in a plan
     unsigned long long plan_classes = 0;
     for (const auto& kr : key_rows)
@@ -1724,7 +1736,9 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
             if (int rc = f64_occupancy(kc.s64)) return rc;
             continue;
         }
-        kc.s32 = kc.fb == 2 ? mfma_shape_fb2(kc.nt) : mfma_shape(kc.nt);
+        kc.s32 = kc.fb == 2 ? mfma_shape_fb2(kc.nt)
+               : kc.nt >= 2 && kc.nt <= 16 && mfma_fams < 32LL * ctx->n_cu ? mfma_shape_few(kc.nt)
+                                                                         : mfma_shape(kc.nt);
         kc.r64 = f64_shape(kc.nt, 1, ctx->n_slots, ctx->n_leaves, ctx->n_cu);
         place_partials(kc.s32, kc.n_slots, kc.slot_tiles, kc.n_cols, kc.max_pat);
         HIP_OR_FAIL(mfma_occupancy(kc.s32, &kc.s32.per_cu));
