@@ -582,7 +582,7 @@ int find_patterns(cafe_gpu_ctx* ctx)
     }
     std::vector<int> row(n, -1);   // a unit node's row of the extended count table
     int n_rows = nl;
-    std::vector<std::vector<int>> rows;   // [n_rows - nl][F]
+    std::vector<int> rows;   // [n_rows - nl][F]
     std::vector<StepDev> steps, steps_reuse;
     std::vector<ColDev> cols;
     std::vector<int> reps, table;
@@ -694,9 +694,9 @@ int find_patterns(cafe_gpu_ctx* ctx)
             if (!unit[u]) continue;
             if (row[u] < 0) {
                 row[u] = n_rows++;
-                rows.emplace_back(F, 0);
+                rows.resize((size_t)(n_rows - nl) * F, 0);
             }
-            std::copy(ids[u].begin(), ids[u].end(), rows[row[u] - nl].begin() + bk.fam_begin);
+            std::copy(ids[u].begin(), ids[u].end(), rows.begin() + (size_t)(row[u] - nl) * F + bk.fam_begin);
             PatternUnit un;
             unit_of[u] = (int)P.units.size();
             un.prog = program(u, true);
@@ -717,8 +717,7 @@ int find_patterns(cafe_gpu_ctx* ctx)
     if (!P.units.empty()) {
         HIP_OR_FAIL(P.ext.ensure(sizeof(int) * (size_t)n_rows * F));
         HIP_OR_FAIL(hipMemcpy(P.ext.p, ctx->d_counts.p, sizeof(int) * (size_t)nl * F, hipMemcpyDeviceToDevice));
-        for (int r = nl; r < n_rows; ++r)
-            HIP_OR_FAIL(hipMemcpy(P.ext.as<int>() + (size_t)r * F, rows[r - nl].data(), sizeof(int) * F, hipMemcpyHostToDevice));
+        HIP_OR_FAIL(hipMemcpy(P.ext.as<int>() + (size_t)nl * F, rows.data(), sizeof(int) * rows.size(), hipMemcpyHostToDevice));
         auto put = [&](DevBuf& b, const void* v, size_t bytes) -> int {
             HIP_OR_FAIL(b.ensure(bytes));
             HIP_OR_FAIL(hipMemcpy(b.p, v, bytes, hipMemcpyHostToDevice));
