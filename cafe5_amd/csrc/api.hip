@@ -178,7 +178,7 @@ struct EvalBufs {
 // A program over pattern columns: its steps and columns in Patterns' buffers.
 struct PatternProg {
     int step0 = 0, n_steps = 0, col0 = 0, n_cols = 0, n_pat = 0;
-    int n_slots = 0, n_slots_reuse = 0;   // of its steps and steps_reuse
+    int n_slots = 0, n_slots_reuse = 0, n_slots_hot = 0;   // of its three step lists
 };
 struct PatternUnit {
     PatternProg prog;
@@ -195,7 +195,7 @@ struct Patterns {
     std::vector<PatternProg> main;      // per bucket
     std::vector<int> first_unit;        // per bucket (and the end)
     DevBuf ext;                         // count table with the units' pattern rows after the leaves'
-    DevBuf steps, steps_reuse;          // programs (steps_reuse: outputs in their children's slots)
+    DevBuf steps, steps_reuse, steps_hot;   // programs (outputs in their children's slots; and hot)
     DevBuf cols, reps;
     void clear()
     {
@@ -206,7 +206,7 @@ struct Patterns {
     }
     void release_all()
     {
-        for (DevBuf* b : {&ext, &steps, &steps_reuse, &cols, &reps}) b->release();
+        for (DevBuf* b : {&ext, &steps, &steps_reuse, &steps_hot, &cols, &reps}) b->release();
     }
 };
 
@@ -519,6 +519,13 @@ constexpr int kPatternShare = 2;
 // and 1.70 ms dividing by 2, by 6 and never; 5,000 families 0.75, 0.78, 0.76).
 constexpr int kPatternNest = 3;
 
+// Entries of a pattern column of a bucket: whole row tiles, and the rows the
+// per-lane kernel gathers.
+int column_entries(const BucketHost& bk)
+{
+    return round_up(std::max({bk.B + 1, bk.R + 1, lane_rows_for(std::max(bk.B, bk.R) + 1)}), kTile);
+}
+
 // Pattern ids of the pairs (a[f], b[f]), a < na and b < nb, numbered in order
 // of appearance; 0 where there are more than `limit`.
 int pair_patterns(const std::vector<int>& a, int na, const std::vector<int>& b, int nb, int limit, std::vector<int>& id,
@@ -583,13 +590,13 @@ int find_patterns(cafe_gpu_ctx* ctx)
     std::vector<int> row(n, -1);   // a unit node's row of the extended count table
     int n_rows = nl;
     std::vector<int> rows;   // [n_rows - nl][F]
-    std::vector<StepDev> steps, steps_reuse;
+    std::vector<StepDev> steps[3];   // in order, with reuse, hot
     std::vector<ColDev> cols;
     std::vector<int> reps, table;
     P.main.resize(ctx->buckets.size());
     for (int bi = 0; bi < (int)ctx->buckets.size(); ++bi) {
         const BucketHost& bk = ctx->buckets[bi];
-        const int xs = std::max(round_up(bk.B + 1, kTile), round_up(bk.R + 1, kTile));
+        const int xs = column_entries(bk);
         P.first_unit.push_back((int)P.units.size());
         std::vector<std::vector<int>> ids(n);
         std::vector<int> count(n, 0);   // patterns of a node (0: not a candidate)
@@ -663,12 +670,13 @@ int find_patterns(cafe_gpu_ctx* ctx)
                 cols.push_back(ColDev{leaf[c], 0});
             }
             pr.n_cols = (int)cols.size() - pr.col0;
-            pr.step0 = (int)steps.size();
-            for (const bool reuse : {false, true}) {
-                Planner pl(kids, code, reuse);
+            pr.step0 = (int)steps[0].size();
+            int* n_slots[3] = {&pr.n_slots, &pr.n_slots_reuse, &pr.n_slots_hot};
+            for (int v = 0; v < 3; ++v) {
+                Planner pl(kids, code, v > 0, v == 2);
                 pl.compute_need(top);
-                pl.emit(top);
-                (reuse ? pr.n_slots_reuse : pr.n_slots) = pl.max_slot + 1;
+                pl.emit(top, v < 2);
+                *n_slots[v] = std::max(1, pl.max_slot + 1);
                 std::vector<StepDev> st = flatten_steps(pl.ops, pl.out_kids);
                 for (StepDev& s : st) {
                     if (is_unit) s.ctl &= ~kStepRoot;
@@ -682,8 +690,7 @@ int find_patterns(cafe_gpu_ctx* ctx)
                                          kStepFirst | kStepLast | kStepOut |
                                              (ctx->parent_h[top] == root ? kStepRoot : 0)});
                 pr.n_steps = (int)st.size();
-                auto& all = reuse ? steps_reuse : steps;
-                all.insert(all.end(), st.begin(), st.end());
+                steps[v].insert(steps[v].end(), st.begin(), st.end());
             }
             for (int c : pats) code[c] = -1;
             for (int c : leaves) code[c] = -1;
@@ -723,8 +730,9 @@ int find_patterns(cafe_gpu_ctx* ctx)
             HIP_OR_FAIL(hipMemcpy(b.p, v, bytes, hipMemcpyHostToDevice));
             return CAFE_GPU_OK;
         };
-        if (int rc = put(P.steps, steps.data(), sizeof(StepDev) * steps.size())) return rc;
-        if (int rc = put(P.steps_reuse, steps_reuse.data(), sizeof(StepDev) * steps_reuse.size())) return rc;
+        if (int rc = put(P.steps, steps[0].data(), sizeof(StepDev) * steps[0].size())) return rc;
+        if (int rc = put(P.steps_reuse, steps[1].data(), sizeof(StepDev) * steps[1].size())) return rc;
+        if (int rc = put(P.steps_hot, steps[2].data(), sizeof(StepDev) * steps[2].size())) return rc;
         if (int rc = put(P.cols, cols.data(), sizeof(ColDev) * cols.size())) return rc;
         if (int rc = put(P.reps, reps.data(), sizeof(int) * reps.size())) return rc;
     }
@@ -1165,7 +1173,7 @@ struct KernelClass {
     // made level by level before the main pass (tiles, their count's place)
     bool pat = false;
     int max_pat = 0, n_cols = 0;            // most pattern and leaf columns of a program
-    int n_slots = 0, n_slots_lane = 0;      // most partial vectors of a program (in order, with reuse)
+    int n_slots = 0, n_slots_lane = 0, n_slots_hot = 0;   // most partial vectors of a program (in order, reuse, hot)
     struct Level {
         int begin, n, count_at;
     };
@@ -1645,14 +1653,14 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
         for (const auto& kr : key_rows) {
             const int key = kr.first;
             const bool f64 = path == CAFE_GPU_PATH_PLAIN64 || path == CAFE_GPU_PATH_BATCHED64 || key > kMfmaMaxTiles;
-            if (lane_rows_of(key) > 0 || (f64 && ctx->n_leaves > 512)) continue;
+            if (f64 && ctx->n_leaves > 512) continue;   // (counts not staged)
             long long fams = 0;
             size_t bytes = 0;
             for (auto& bc : bucket_class) {
                 if (bc.first != key || pat.first_unit[bc.second] == pat.first_unit[bc.second + 1]) continue;
                 fams += (long long)ctx->buckets[bc.second].count * n_points;
                 for (int u = pat.first_unit[bc.second]; u < pat.first_unit[bc.second + 1]; ++u)
-                    bytes += 8 * (size_t)pat.units[u].n * max_point * kTile * key_nt[key];
+                    bytes += 8 * (size_t)pat.units[u].n * max_point * column_entries(ctx->buckets[bc.second]);
             }
             if (fams < kPatternWork || pat_bytes + bytes > kPatternBytes) continue;
             key_pat[key] = true;
@@ -1672,12 +1680,14 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
             kc.n_cols = kc.pat ? 0 : ctx->n_leaves;
             kc.n_slots = kc.pat ? 0 : ctx->n_slots;
             kc.n_slots_lane = kc.pat ? 0 : ctx->n_slots_lane;
+            kc.n_slots_hot = kc.pat ? 0 : ctx->n_slots_hot;
             if (kc.pat) {
                 auto add = [&](const PatternProg& pr) {
                     kc.max_pat = std::max(kc.max_pat, pr.n_pat);
                     kc.n_cols = std::max(kc.n_cols, pr.n_cols);
                     kc.n_slots = std::max(kc.n_slots, pr.n_slots);
                     kc.n_slots_lane = std::max(kc.n_slots_lane, pr.n_slots_reuse);
+                    kc.n_slots_hot = std::max(kc.n_slots_hot, pr.n_slots_hot);
                 };
                 for (auto& o : bucket_class) {
                     if (o.first != bc.first) continue;
@@ -1703,9 +1713,9 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
                 }
             }
             if (kc.lane_rows > 0) {
-                kc.lane_slots = ctx->n_slots_hot + 1;   // the stored slots and the hot array
+                kc.lane_slots = kc.n_slots_hot + 1;   // the stored slots and the hot array
                 const PruneParams none{};
-                HIP_OR_FAIL(lane_dispatch(kc.lane_rows, kc.lane_slots, 0, lane_shm(ctx->n_leaves), none, nullptr,
+                HIP_OR_FAIL(lane_dispatch(kc.lane_rows, kc.lane_slots, 0, lane_shm(kc.n_cols), none, nullptr,
                                           &kc.lane_per_cu));
                 if (kc.lane_per_cu == 0) kc.lane_rows = 0;   // no instance fits: matrix-core kernel
             }
@@ -1824,7 +1834,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
         }
         for (auto& kc : pp.classes) {
             if (!kc.pat) continue;
-            const int tw = kTile * kc.fb;
+            const int tw = kc.lane_rows > 0 ? 64 : kTile * kc.fb;
             std::vector<std::vector<TileDesc>> level;
             for (auto& bc : bucket_class) {
                 if (key_nt[bc.first] != kc.nt || !key_pat.count(bc.first)) continue;
@@ -1832,9 +1842,8 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
                     const PatternUnit& pu = pat.units[u];
                     UnitDev& ud = units[u];
                     ud.n = pu.n;
-                    // (a column covers the bucket's own rows)
                     const BucketHost& bk = ctx->buckets[bc.second];
-                    ud.xs = std::max(round_up(bk.B + 1, kTile), round_up(bk.R + 1, kTile));
+                    ud.xs = column_entries(bk);
                     long long& top = kc.f64 ? n64 : n32;
                     ud.x0 = top;
                     top += (long long)pu.n * max_point * ud.xs;
@@ -2003,14 +2012,12 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
         q.slot_tiles = kc.slot_tiles;
         q.scratch = scratch + kc.off_main;
         q.n_slots = kc.n_slots;
-        if (kc.lane_rows > 0) {   // BATCHED32 / BATCHED16: small vectors, one family per lane
+        const bool lane = kc.lane_rows > 0;   // BATCHED32 / BATCHED16: small vectors, one family per lane
+        if (lane) {
             q.steps = ctx->d_steps_hot.as<StepDev>();
-            q.n_slots = ctx->n_slots_hot;
-            HIP_OR_FAIL(lane_dispatch(kc.lane_rows, kc.lane_slots, pp.grid_lane(kc.lane_per_cu, n, kc.lane_grid_mult),
-                                      lane_shm(ctx->n_leaves), q, s, nullptr));
-            return CAFE_GPU_OK;
+            q.n_slots = kc.n_slots_hot;
         }
-        const bool f16 = !kc.f64 && pp.path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles;
+        const bool f16 = !kc.f64 && !lane && pp.path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles;
         if (f16) {
             q.steps = ctx->d_steps_lane.as<StepDev>();
             q.n_slots = kc.n_slots_lane;
@@ -2018,6 +2025,10 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
         if (kc.f64) q.slot_tiles = kc.nt;
         auto launch = [&](const PruneParams& a, int tiles) -> int {
             if (kc.f64) HIP_OR_FAIL(f64_dispatch(kc.s64, pp.grid(kc.s64, tiles), a, s, nullptr));
+            else if (lane)
+                HIP_OR_FAIL(lane_dispatch(kc.lane_rows, kc.lane_slots,
+                                          pp.grid_lane(kc.lane_per_cu, tiles, kc.lane_grid_mult), lane_shm(kc.n_cols), a,
+                                          s, nullptr));
             else if (f16) HIP_OR_FAIL(f16_dispatch(kc.s16, pp.grid(kc.s16, tiles), a, s, nullptr));
             else HIP_OR_FAIL(launch_prune_mfma(kc.s32, pp.grid(kc.s32, tiles), a, s));
             return CAFE_GPU_OK;
@@ -2026,7 +2037,7 @@ int enqueue_prune(cafe_gpu_ctx* ctx, EvalBufs& b, const PrunePlan& pp, hipStream
             q.units = b.units.as<UnitDev>();
             q.max_pat = kc.max_pat;
             q.n_leaves = kc.n_cols;
-            q.steps = (f16 ? ctx->pat.steps_reuse : ctx->pat.steps).as<StepDev>();
+            q.steps = (lane ? ctx->pat.steps_hot : f16 ? ctx->pat.steps_reuse : ctx->pat.steps).as<StepDev>();
             q.counts_T = ctx->pat.ext.as<int>();
             for (const auto& l : kc.levels) {
                 PruneParams a = q;

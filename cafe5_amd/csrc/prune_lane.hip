@@ -29,6 +29,11 @@
 // output may take the slot of one of its children (the children are all read
 // before the output is written, by the same lane).
 //
+// Shared subtrees (PruneParams::units) turn most interior children into gathers:
+// a unit's column and its exponent and bound, loaded like a leaf's column.  The
+// 64-point grid over 17,400 families of bound 20 among 20,000 takes 3.35 -> 2.83
+// ms a step.
+//
 // Numerics follow the single-wave matrix-core kernel exactly: stored vectors
 // are renormalised to a maximum just below 2^vec_exp, the exponent is carried
 // in an integer, and a bound on what FP32 flushing to zero could have dropped
@@ -109,7 +114,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LaneWaves<LR
     const int lane = threadIdx.x;
     const int Np = p.Np;
     const int a_exp = p.vec_exp;
-    const int n_steps = p.n_steps;
     const long long slot_elems = p.slot_elems;
     // FP32 leaf factors: up to n_dev flushed terms (one without an error model)
     const double leaf_cert = (p.n_dev > 1 ? p.n_dev : 1) * kTau32 * kTwoPowMinusMatExp;
@@ -118,7 +122,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LaneWaves<LR
     // LR matrix entries and products that may flush, and the stored vector's
     // own entries
     const double cint = kTau32 * (LR * kTwoPowMinusMatExp * (1.0 + two_m_a) + two_m_a);
-    extern __shared__ int s_cnt[];   // [leaf][64]: the tile's leaf counts, lane l's in column l
+    extern __shared__ int s_cnt[];   // [column][64]: the tile's leaf counts and patterns, lane l's in column l
 
     const int n_tiles = *as_const(p.n_tiles_dev);
     const int groups = (gridDim.x % 8 == 0) ? 8 : 1;   // XCD-aware static split (see k_prune_mfma)
@@ -134,7 +138,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LaneWaves<LR
         const int fi = valid ? lane : 0;
         const int fs = td.nf < 0 ? p.fam_list[td.fam0 + fi] : bk.fam_begin + td.fam0 + fi;
         const int dst = p.perm[fs];   // the caller's index of this lane's family
-        for (int l = 0; l < p.n_leaves; ++l) s_cnt[l * 64 + lane] = p.counts_T[(long long)l * p.F + fs];
+        const StepDev* __restrict__ steps = p.steps + (p.units ? bk.step0 : 0);
+        const int n_steps = p.units ? bk.n_steps : p.n_steps;
+        const int n_cols = p.units ? bk.n_cols : p.n_leaves;
+        for (int l = 0; l < n_cols; ++l) {
+            const int row = p.units ? as_const((const int*)(p.cols + bk.col0 + l))[0] : l;
+            s_cnt[l * 64 + lane] = p.counts_T[(long long)row * p.F + fs];
+        }
         const __attribute__((address_space(4))) int* nslot = as_const(p.node_slot + (long long)td.point * p.n_nodes);
 
         constexpr int H = NS - 1;   // the hot array; stored slots 0 .. NS-2
@@ -163,7 +173,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LaneWaves<LR
             bool root = false;
             int out = 0;
             for (;;) {
-                const StepDev sd = ld_const(p.steps, st++);
+                const StepDev sd = ld_const(steps, st++);
                 root = (sd.ctl & kStepRoot) != 0;
                 out = sd.ctl & kStepSlotMask;
                 // the node's first child sets the product (1 x factor, exactly),
@@ -178,10 +188,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LaneWaves<LR
                 if (sd.leaf_col >= 0) {
                     // leaf: column `count` of the (error-model folded) matrix
                     const int cnt = s_cnt[sd.leaf_col * 64 + lane];
-                    const float* __restrict__ col = p.leaf32 + base + (long long)cnt * Np;
-                    e_sum -= kMatExp;
-                    log2S += kMatExp;
-                    cert += leaf_cert;
+                    const float* __restrict__ col;
+                    if (sd.ctl & kStepPattern) {   // column `pattern` of a unit: an interior child's terms
+                        const UnitDev u = ld_const(p.units, sd.in_slot);
+                        const long long c = (long long)td.point * u.n + cnt;
+                        col = p.x32 + u.x0 + c * u.xs;
+                        e_sum += p.xm_e[u.m0 + c];
+                        cert += p.xm_c[u.m0 + c];
+                        log2S += kMatExp + a_exp;
+                    } else {
+                        col = p.leaf32 + base + (long long)cnt * Np;
+                        e_sum -= kMatExp;
+                        log2S += kMatExp;
+                        cert += leaf_cert;
+                    }
                         // 16-byte loads: a column starts 128-byte aligned (Np is a
                     // multiple of 32) and holds Np >= 4 ceil(LR / 4) entries
                     // (Np >= 32 always; 33-row classes have N >= 22, Np >= 64)
@@ -290,7 +310,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LaneWaves<LR
             sc[H] = cnew;
             if (out != kHotSlot) put<NS - 1>(sv, se, sc, out, sv[H], se[H], sc[H]);
         }
-        {
+        if (p.units && bk.out >= 0) {   // the branch's factor (its one step's) as a column
+            const UnitDev u = ld_const(p.units, bk.out);
+            const long long c = (long long)td.point * u.n + td.fam0 - bk.list0 + lane;
+            if (valid) {
+                float* X = p.x32 + u.x0 + c * u.xs;
+#pragma unroll
+                for (int i = 0; i < LR; ++i) X[i] = acc[i];
+                p.xm_e[u.m0 + c] = e_sum;
+                p.xm_c[u.m0 + c] = cert;
+            }
+        } else {
             // root: best x_j * prior_j over root sizes j + 1, j = 0..R-1
             const __attribute__((address_space(4))) double* pr = as_const(p.prior64 + bk.prior_off);
             RootBest rb{-__builtin_huge_val(), 0.0, -1, 0.0};

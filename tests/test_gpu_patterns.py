@@ -130,3 +130,20 @@ def test_patterns_follow_the_table(eng):
     eng.matrix_build(*keys.arrays())
     r = eng.evaluate(slots, _prior(48), native.PATH_BATCHED64)
     assert np.array_equal(r["lnl"][0], first)
+
+
+@pytest.mark.parametrize("path", native.REDUCED_PATHS)
+@pytest.mark.parametrize("B,R,F,error", [(20, 20, 1100, False), (9, 14, 600, False), (20, 12, 1025, True),
+                                         (32, 32, 1300, False), (24, 30, 777, True)])
+def test_one_family_per_lane(eng, path, B, R, F, error):
+    # the per-lane kernel's sizes: columns of 21 and 33 rows
+    err = None
+    if error:
+        err = np.tile([0.04, 0.92, 0.04], (B + 1, 1))
+        err[0] = (0.0, 0.96, 0.04)
+    for tree in (_odd_tree(), wl.yule_tree(30, 4)):
+        counts = np.minimum(_counts(tree, F, B, 3 * B + F), B - 1)
+        got = _lnl(eng, tree, counts, B, R, path, err)
+        _same(path, got, _pieces(eng, tree, counts, B, R, path, err))
+        plain = _lnl(eng, tree, counts, B, R, native.PATH_PLAIN64, err)
+        _same(path, got, plain)
