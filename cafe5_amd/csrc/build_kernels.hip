@@ -410,8 +410,9 @@ __global__ __launch_bounds__(256) void k_fold_err32(const float* __restrict__ lf
 }
 
 // One matrix out of its c-major slot, row-major without padding: 32 x 32 tiles
-// through LDS, so that both sides move whole lines (the host's strided copy of
-// 201 x 201 entries took longer than the transfer).
+// through LDS, so that both sides move whole lines (matrices past the staging
+// buffer; a host's strided copy of 401 x 401 entries takes longer than the
+// transfer).
 __global__ __launch_bounds__(256) void k_matrix_rows(const double* __restrict__ M, int N, int Np, double* __restrict__ out)
 {
     __shared__ double tile[32][33];

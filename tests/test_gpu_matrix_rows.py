@@ -1,5 +1,5 @@
-"""Matrices as the host gets them, at sizes around the 32 x 32 tiles of the
-copy and the 256 rows of the closed form's blocks: every entry of both builds
+"""Matrices as the host gets them, turned on the host (small) and on the device, at
+sizes around its 32 x 32 tiles and the 256 rows of the closed form's blocks: every entry of both builds
 against the oracle's term-by-term matrix (FP64 sums of non-negative terms: both
 within 2e-12 of it, relative), the saturated and the zero key included."""
 import numpy as np
@@ -19,7 +19,7 @@ def eng():
 
 
 @pytest.mark.parametrize("algo", [native.BUILD_CLOSED_FORM, native.BUILD_RECURRENCE])
-@pytest.mark.parametrize("N", [2, 31, 32, 33, 64, 65, 257])
+@pytest.mark.parametrize("N", [2, 33, 64, 200, 256, 257, 288, 289])
 def test_entries(eng, algo, N):
     lam, t = [0.002, 0.01, 0.0, 0.5], [30.0, 7.0, 10.0, 9.0]
     eng.matrix_reset(N, 4)
