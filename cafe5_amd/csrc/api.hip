@@ -62,7 +62,7 @@ constexpr int kSideStreams = 4;
 
 // Fixed device scratch of the entry points that allocate nothing
 // (cafe_gpu_reconstruct_noalloc): a reconstruction's program, family list,
-// state rows, error flags and per-family L, C and product rows.  Every device
+// state rows, error flag, block maxima and per-family L rows.  Every device
 // the library runs on holds its own copy for the life of the process.  In host
 // code `scratch` names a host-side stand-in, never the device memory: its
 // device address comes from hipGetSymbolAddress, once per device (see
@@ -240,7 +240,7 @@ struct cafe_gpu_ctx {
     int n_nodes = 0, tree_leaves = 0, n_slots = 0, max_children = 2;
     std::vector<int> parent_h, leaf_col_h;   // the tree as set
     DevBuf d_recon;                          // reconstruction: program, families, prior, states, flags
-    DevBuf d_recon_scratch;                  // reconstruction: per-family L, C and product rows
+    DevBuf d_recon_scratch;                  // reconstruction: per-family L rows
     char* fixed_scratch = nullptr;           // this device's copy of `scratch` (device address)
     std::vector<OpDev> ops;
     std::vector<ChildDev> kids;
