@@ -184,6 +184,7 @@ struct PatternUnit {
     PatternProg prog;
     int bucket;
     int n;         // patterns
+    int xs;        // entries per column
     int list0;     // their representatives' place in `reps`
     int level;     // 1 + the largest level of a unit it reads (0: none)
 };
@@ -519,11 +520,23 @@ constexpr int kPatternShare = 2;
 // and 1.70 ms dividing by 2, by 6 and never; 5,000 families 0.75, 0.78, 0.76).
 constexpr int kPatternNest = 3;
 
-// Entries of a pattern column of a bucket: whole row tiles, and the rows the
-// per-lane kernel gathers.
-int column_entries(const BucketHost& bk)
+// 16-row tiles of a bucket's vectors and root rows (sizes 0..R).
+int tiles_of(const BucketHost& bk)
 {
-    return round_up(std::max({bk.B + 1, bk.R + 1, lane_rows_for(std::max(bk.B, bk.R) + 1)}), kTile);
+    return std::max(round_up(bk.B + 1, kTile), round_up(bk.R + 1, kTile)) / kTile;
+}
+
+// Entries of a pattern column of a bucket: whole row tiles, and the rows the
+// per-lane kernel writes and gathers.  That kernel's instance covers every
+// bucket of the size class (33 rows for bounds 20 and 28 side by side, where
+// the first alone takes 21), so the class's largest vector decides.
+int column_entries(const std::vector<BucketHost>& buckets, int bi)
+{
+    const BucketHost& bk = buckets[bi];
+    int rows = 0;   // of the class
+    for (const BucketHost& o : buckets)
+        if (tiles_of(o) == tiles_of(bk)) rows = std::max(rows, std::max(o.B, o.R) + 1);
+    return round_up(std::max({bk.B + 1, bk.R + 1, lane_rows_for(rows)}), kTile);
 }
 
 // Pattern ids of the pairs (a[f], b[f]), a < na and b < nb, numbered in order
@@ -596,7 +609,7 @@ int find_patterns(cafe_gpu_ctx* ctx)
     P.main.resize(ctx->buckets.size());
     for (int bi = 0; bi < (int)ctx->buckets.size(); ++bi) {
         const BucketHost& bk = ctx->buckets[bi];
-        const int xs = column_entries(bk);
+        const int xs = column_entries(ctx->buckets, bi);
         P.first_unit.push_back((int)P.units.size());
         std::vector<std::vector<int>> ids(n);
         std::vector<int> count(n, 0);   // patterns of a node (0: not a candidate)
@@ -709,6 +722,7 @@ int find_patterns(cafe_gpu_ctx* ctx)
             un.prog = program(u, true);
             un.bucket = bi;
             un.n = count[u];
+            un.xs = xs;
             un.list0 = (int)reps.size();
             un.level = level[u];
             reps.resize(reps.size() + un.n, -1);
@@ -1593,9 +1607,6 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     for (auto& bk : ctx->buckets)
         maxLR = std::max(maxLR, std::max(round_up(bk.B + 1, kTile), round_up(bk.R + 1, kTile)));
     pp.maxLR = maxLR;
-    auto nt_of = [](const BucketHost& bk) {   // root rows run 0..R
-        return std::max(round_up(bk.B + 1, kTile), round_up(bk.R + 1, kTile)) / kTile;
-    };
     std::vector<std::pair<int, int>> bucket_class;   // (class key, bucket)
     for (int bi = 0; bi < (int)ctx->buckets.size(); ++bi) {
         const BucketHost& bk = ctx->buckets[bi];
@@ -1606,7 +1617,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
             return fail(CAFE_GPU_EINVAL, "bucket B=%d R=%d exceeds the sizes this path supports", bk.B, bk.R);
         // PLAIN64: one class per power of two of 4-tile blocks (the FP64
         // kernel takes vectors of any length)
-        int key = nt_of(bk);
+        int key = tiles_of(bk);
         if (path == CAFE_GPU_PATH_PLAIN64) {
             int pow2 = 4;
             while (pow2 < key) pow2 <<= 1;
@@ -1643,7 +1654,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     std::map<int, int> key_nt;   // and the tiles of its largest vector
     for (auto& bc : bucket_class) {
         key_fams[bc.first] += (long long)ctx->buckets[bc.second].count * n_points;
-        key_nt[bc.first] = std::max(key_nt[bc.first], nt_of(ctx->buckets[bc.second]));
+        key_nt[bc.first] = std::max(key_nt[bc.first], tiles_of(ctx->buckets[bc.second]));
     }
     for (const auto& kf : key_fams)
         if (lane_rows_of(kf.first) == 0) mfma_fams += kf.second;
@@ -1672,7 +1683,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
                 if (bc.first != key || pat.first_unit[bc.second] == pat.first_unit[bc.second + 1]) continue;
                 fams += (long long)ctx->buckets[bc.second].count * n_points;
                 for (int u = pat.first_unit[bc.second]; u < pat.first_unit[bc.second + 1]; ++u)
-                    bytes += 8 * (size_t)pat.units[u].n * max_point * column_entries(ctx->buckets[bc.second]);
+                    bytes += 8 * (size_t)pat.units[u].n * max_point * pat.units[u].xs;
             }
             if (fams < kPatternWork || pat_bytes + bytes > kPatternBytes) continue;
             key_pat[key] = true;
@@ -1736,7 +1747,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
         }
         KernelClass& kc = pp.classes.back();
         const int ci = (int)pp.classes.size() - 1;
-        kc.nt = std::max(kc.nt, nt_of(bk));
+        kc.nt = std::max(kc.nt, tiles_of(bk));
         kc.slot_tiles = std::max(kc.slot_tiles, round_up(bk.B + 1, kTile) / kTile);
         const int tw = kc.lane_rows > 0 ? 64 : kTile * kc.fb;   // families per tile
         for (int pi = 0; pi < n_points; ++pi) {
@@ -1854,8 +1865,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
                     const PatternUnit& pu = pat.units[u];
                     UnitDev& ud = units[u];
                     ud.n = pu.n;
-                    const BucketHost& bk = ctx->buckets[bc.second];
-                    ud.xs = column_entries(bk);
+                    ud.xs = pu.xs;
                     long long& top = kc.f64 ? n64 : n32;
                     ud.x0 = top;
                     top += (long long)pu.n * max_point * ud.xs;
