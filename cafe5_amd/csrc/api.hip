@@ -12,6 +12,7 @@
 #include <map>
 #include <mutex>
 #include <numeric>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -1171,6 +1172,7 @@ namespace {
 // Kernel size class: buckets whose vectors have the same number of 16-row
 // tiles.
 struct KernelClass {
+    int key;             // of its buckets (plan_prune)
     int nt;              // 16-row tiles of the class's largest vector
     int slot_tiles;      // 16-row tiles of its largest stored (non-root) vector
     MfmaShape s32, s64;  // launch shapes of the FP32 and FP64 MFMA kernels
@@ -1595,9 +1597,10 @@ int upload_eval_inputs(cafe_gpu_ctx* ctx, EvalBufs& b, const cafe_gpu_eval_desc*
 
 // Builds and uploads the tile list for `n_points` parameter points (heaviest
 // classes and buckets first, grouped by kernel size class) and sizes the
-// scratch.
+// scratch.  `whole` are the keys of the classes that do not run over subtree
+// patterns although they could.
 int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points, const int* point_ids,
-               double* root_out, int root_stride, PrunePlan& pp)
+               double* root_out, int root_stride, PrunePlan& pp, const std::set<int>& whole = {})
 {
     pp = PrunePlan();
     pp.path = path;
@@ -1677,6 +1680,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
             const int key = kr.first;
             const bool f64 = path == CAFE_GPU_PATH_PLAIN64 || path == CAFE_GPU_PATH_BATCHED64 || key > kMfmaMaxTiles;
             if (f64 && ctx->n_leaves > 512) continue;   // (counts not staged)
+            if (whole.count(key)) continue;
             long long fams = 0;
             size_t bytes = 0;
             for (auto& bc : bucket_class) {
@@ -1696,6 +1700,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
         const BucketHost& bk = ctx->buckets[bc.second];
         if (pp.classes.empty() || bc.first != prev_key) {
             KernelClass kc{};
+            kc.key = bc.first;
             kc.begin = kc.end = (int)tiles.size();
             kc.fams = key_fams[bc.first];
             kc.seg_begin = kc.seg_end = (int)segs.size();
@@ -1761,6 +1766,13 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
         kc.seg_end = (int)segs.size();
     }
     const int n_cls = (int)pp.classes.size();
+    // a shape over patterns that does not fit is no error: its class leaves them below
+    auto fit = [](const KernelClass& kc, hipError_t e, MfmaShape& sh) {
+        if (e == hipSuccess || !kc.pat) return e;
+        (void)hipGetLastError();
+        sh.per_cu = 0;
+        return hipSuccess;
+    };
     for (auto& kc : pp.classes) {
         if (kc.f64) {
             pp.has_f64 = true;
@@ -1773,7 +1785,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
                                                                          : mfma_shape(kc.nt);
         kc.r64 = f64_shape(kc.nt, 1, ctx->n_slots, ctx->n_leaves, ctx->n_cu);
         place_partials(kc.s32, kc.n_slots, kc.slot_tiles, kc.n_cols, kc.max_pat);
-        HIP_OR_FAIL(mfma_occupancy(kc.s32, &kc.s32.per_cu));
+        HIP_OR_FAIL(fit(kc, mfma_occupancy(kc.s32, &kc.s32.per_cu), kc.s32));
         if (int rc = f64_occupancy(kc.r64)) return rc;
         if (path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles) {
             // the program whose outputs reuse a child's slot (the store's
@@ -1781,11 +1793,11 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
             kc.s16 = mfma_shape(kc.nt);
             place_partials16(kc.s16, kc.n_slots_lane, kc.slot_tiles, kc.n_cols, kc.max_pat);
             const PruneParams none{};
-            HIP_OR_FAIL(f16_dispatch(kc.s16, 0, none, nullptr, &kc.s16.per_cu));
+            HIP_OR_FAIL(fit(kc, f16_dispatch(kc.s16, 0, none, nullptr, &kc.s16.per_cu), kc.s16));
             if (kc.s16.per_cu == 0 && kc.s16.lds) {   // LDS does not fit: global scratch
                 kc.s16.lds = false;
                 kc.s16.shm = f16_meta_only(kc.s16, kc.n_slots_lane, kc.n_cols, kc.max_pat);
-                HIP_OR_FAIL(f16_dispatch(kc.s16, 0, none, nullptr, &kc.s16.per_cu));
+                HIP_OR_FAIL(fit(kc, f16_dispatch(kc.s16, 0, none, nullptr, &kc.s16.per_cu), kc.s16));
             }
         }
     }
@@ -1794,6 +1806,18 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
     for (auto& kc : pp.classes)
         if (!kc.plain)
             if (int rc = apply_tuning(ctx, path, kc, plan_classes)) return rc;
+    // A pattern column takes two to four times a leaf's LDS (exponent and bound
+    // beside the offset): a tree of many two-leaf clades can be too wide for a
+    // CU that way (from about 640 taxa with 32-family tiles) and still fit with
+    // its leaves.
+    for (auto& kc : pp.classes) {
+        if (!kc.pat || kc.lane_rows > 0) continue;
+        const bool f16 = !kc.f64 && path == CAFE_GPU_PATH_BATCHED16 && kc.nt <= kF16MaxTiles;
+        if ((kc.f64 ? kc.s64 : f16 ? kc.s16 : kc.s32).per_cu > 0) continue;
+        std::set<int> out = whole;
+        out.insert(kc.key);
+        return plan_prune(ctx, b, path, model, n_points, point_ids, root_out, root_stride, pp, out);
+    }
     // Main-pass classes to side streams, longest first onto the least loaded
     // stream.  Estimated cost: contraction work (tiles x nt^2, plus a per-tile
     // overhead) and a floor for the serial chain of one large tile; a
@@ -1860,7 +1884,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
             const int tw = kc.lane_rows > 0 ? 64 : kTile * kc.fb;
             std::vector<std::vector<TileDesc>> level;
             for (auto& bc : bucket_class) {
-                if (key_nt[bc.first] != kc.nt || !key_pat.count(bc.first)) continue;
+                if (bc.first != kc.key) continue;
                 for (int u = pat.first_unit[bc.second]; u < pat.first_unit[bc.second + 1]; ++u) {
                     const PatternUnit& pu = pat.units[u];
                     UnitDev& ud = units[u];

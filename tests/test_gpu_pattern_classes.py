@@ -52,3 +52,41 @@ def test_two_bounds_of_one_class(eng, path, small, large):
     for i in range(0, F, 600):   # 300 families a bucket
         part = _lnl(eng, tree, counts[i:i + 600], B[i:i + 600], path)
         assert np.all(reduced_ok(got[i:i + 600], part)), i
+
+
+def _comb(n):
+    """A spine of n / 2 two-leaf clades (n leaves)."""
+    h = n // 2
+    parent = np.empty(n + h + h - 1, dtype=np.int32)
+    leaf = np.full(len(parent), -1, dtype=np.int32)
+    leaf[:n] = np.arange(n)
+    parent[:n] = n + np.arange(n) // 2
+    spine = n + h + np.arange(h - 1)   # spine[i] joins clade i + 1 and what is before it
+    parent[n] = spine[0]
+    parent[n + 1:n + h] = spine
+    parent[spine[:-1]] = spine[1:]
+    parent[spine[-1]] = -1
+    length = np.where(leaf >= 0, 6.0, 1.0)
+    length[spine[-1]] = 0.0
+    return wl.Tree(parent, leaf, length, [f"n{i}" for i in range(len(parent))])
+
+
+def wide_table(F, n):
+    """Families whose two-leaf clades have few patterns and larger clades many."""
+    rng = np.random.default_rng(n)
+    base = 1 + rng.integers(0, 12, F)
+    return (base[:, None] + np.where(rng.random((F, n)) < 0.08, rng.choice([-1, 1], (F, n)), 0)).astype(np.int32)
+
+
+@pytest.mark.parametrize("n", [640, 700])
+def test_wide_trees(eng, n):
+    # with 32-family tiles the two-leaf clades' columns would take 160 KB of
+    # LDS and more, the leaves half of it; 512 and more leaves share nothing
+    # on the FP64 path
+    tree = _comb(n)
+    counts = wide_table(8300, n)
+    B = np.full(len(counts), 40, dtype=np.int32)
+    got = _lnl(eng, tree, counts, B, native.PATH_BATCHED32)
+    want = _lnl(eng, tree, counts, B, native.PATH_PLAIN64)
+    assert np.isfinite(want).all()
+    assert np.all(reduced_ok(got, want)), np.argwhere(~reduced_ok(got, want))[:5]
