@@ -11,6 +11,7 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <new>
 #include <numeric>
 #include <set>
 #include <string>
@@ -761,7 +762,13 @@ void make_patterns(cafe_gpu_ctx* ctx)
     Patterns& P = ctx->pat;
     if (P.made) return;
     P.clear();
-    if (find_patterns(ctx) != CAFE_GPU_OK) {
+    int rc;
+    try {
+        rc = find_patterns(ctx);
+    } catch (const std::bad_alloc&) {
+        rc = CAFE_GPU_ENOMEM;
+    }
+    if (rc != CAFE_GPU_OK) {
         (void)hipGetLastError();
         P.clear();
         P.release_all();
@@ -1599,8 +1606,8 @@ int upload_eval_inputs(cafe_gpu_ctx* ctx, EvalBufs& b, const cafe_gpu_eval_desc*
 // classes and buckets first, grouped by kernel size class) and sizes the
 // scratch.  `whole` are the keys of the classes that do not run over subtree
 // patterns although they could.
-int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points, const int* point_ids,
-               double* root_out, int root_stride, PrunePlan& pp, const std::set<int>& whole = {})
+int plan_over(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points, const int* point_ids,
+              double* root_out, int root_stride, PrunePlan& pp, const std::set<int>& whole)
 {
     pp = PrunePlan();
     pp.path = path;
@@ -1816,7 +1823,7 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
         if ((kc.f64 ? kc.s64 : f16 ? kc.s16 : kc.s32).per_cu > 0) continue;
         std::set<int> out = whole;
         out.insert(kc.key);
-        return plan_prune(ctx, b, path, model, n_points, point_ids, root_out, root_stride, pp, out);
+        return plan_over(ctx, b, path, model, n_points, point_ids, root_out, root_stride, pp, out);
     }
     // Main-pass classes to side streams, longest first onto the least loaded
     // stream.  Estimated cost: contraction work (tiles x nt^2, plus a per-tile
@@ -2021,6 +2028,29 @@ int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points
         p.xm_e = (int*)(p.xm_c + n_meta);
     }
     return CAFE_GPU_OK;
+}
+
+// The columns are what an evaluation can do without: where the device has no
+// room for them (or for the rest beside them), every class runs its whole
+// program.
+int plan_prune(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points, const int* point_ids,
+               double* root_out, int root_stride, PrunePlan& pp)
+{
+    const size_t block = b.block.size(), views = b.views.size();
+    std::set<int> whole;
+    for (;;) {
+        const int rc = plan_over(ctx, b, path, model, n_points, point_ids, root_out, root_stride, pp, whole);
+        const size_t n = whole.size();
+        for (const auto& kc : pp.classes)
+            if (kc.pat) whole.insert(kc.key);
+        if (rc != CAFE_GPU_ENOMEM || whole.size() == n) return rc;
+        (void)hipGetLastError();
+        b.cols_x.release();
+        b.cols_meta.release();
+        b.block.resize(block);   // (the tables put before)
+        b.views.resize(views);
+        b.bucket_h.resize(ctx->buckets.size());
+    }
 }
 
 // Enqueues the pruning sequence: the main path per size class, then
