@@ -145,6 +145,10 @@ struct PinnedBuf {
 
 struct BucketHost {
     int B, R, count, fam_begin, max_count;
+    bool operator==(const BucketHost& o) const
+    {
+        return B == o.B && R == o.R && count == o.count && fam_begin == o.fam_begin && max_count == o.max_count;
+    }
 };
 
 // A table of an evaluation's input block.
@@ -190,8 +194,9 @@ struct PatternUnit {
     int list0;     // their representatives' place in `reps`
     int level;     // 1 + the largest level of a unit it reads (0: none)
 };
-// The subtree patterns of the families under the tree (UnitDev), made once per
-// tree and families.
+// The subtree patterns of the families under the tree (UnitDev), made by the
+// first evaluation that can use them and kept until another tree or other
+// families are set.
 struct Patterns {
     bool made = false;
     std::vector<PatternUnit> units;     // per bucket contiguous
@@ -580,7 +585,12 @@ int pair_patterns(const std::vector<int>& a, int na, const std::vector<int>& b, 
 }
 
 // Finds the units of every bucket, their programs and those of the buckets,
-// and uploads them (once per tree and families).
+// and uploads them.  A pass over every node's ids on the host: 5 ms for 10,000
+// families of 34 taxa, 20 for 50,000, 300 for 200,000 of 100 taxa -- about ten
+// evaluations' gain -- so it is left to the first evaluation that can share
+// (root vectors and reconstructions do not), and its result is kept while the
+// same tree and counts are set again, as a model that sets both for every score
+// does.
 int find_patterns(cafe_gpu_ctx* ctx)
 {
     Patterns& P = ctx->pat;
@@ -1010,7 +1020,8 @@ int cafe_gpu_set_tree(cafe_gpu_ctx* ctx, int n_nodes, const int* parent, const i
         return fail(CAFE_GPU_EINVAL, "tree needs %d live partial vectors (max %d)", pl.max_slot + 1, kMaxSlots);
     HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));   // nothing reads what is replaced here
     ctx->input_gen++;
-    ctx->pat.clear();
+    if (n_nodes != ctx->n_nodes || !std::equal(parent, parent + n_nodes, ctx->parent_h.begin()) || lc != ctx->leaf_col_h)
+        ctx->pat.clear();
     ctx->n_nodes = n_nodes;
     ctx->tree_leaves = n_leaves;
     ctx->parent_h.assign(parent, parent + n_nodes);
@@ -1098,21 +1109,22 @@ int cafe_gpu_set_families(cafe_gpu_ctx* ctx, int F, int n_leaves, const int* cou
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
         return fb[a] != fb[b] ? fb[a] < fb[b] : fr[a] < fr[b];
     });
-    ctx->buckets.clear();
+    std::vector<BucketHost> buckets;
     for (int k = 0; k < F; ++k) {
         const int f = order[k];
-        if (ctx->buckets.empty() || ctx->buckets.back().B != fb[f] || ctx->buckets.back().R != fr[f])
-            ctx->buckets.push_back(BucketHost{fb[f], fr[f], 0, k, 0});
-        auto& b = ctx->buckets.back();
+        if (buckets.empty() || buckets.back().B != fb[f] || buckets.back().R != fr[f])
+            buckets.push_back(BucketHost{fb[f], fr[f], 0, k, 0});
+        auto& b = buckets.back();
         b.count++;
         b.max_count = std::max(b.max_count, top[f]);
     }
     HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
     ctx->input_gen++;
-    ctx->pat.clear();
     std::vector<int> cT((size_t)n_leaves * F);
     for (int k = 0; k < F; ++k)
         for (int i = 0; i < n_leaves; ++i) cT[(size_t)i * F + k] = counts[(size_t)order[k] * n_leaves + i];
+    // (the patterns are of the sorted counts and the sizes; the caller's order may change)
+    if (cT != ctx->counts_T || buckets != ctx->buckets) ctx->pat.clear();
     HIP_OR_FAIL(ctx->d_counts.ensure(sizeof(int) * cT.size()));
     HIP_OR_FAIL(ctx->d_perm.ensure(sizeof(int) * F));
     HIP_OR_FAIL(hipMemcpy(ctx->d_counts.p, cT.data(), sizeof(int) * cT.size(), hipMemcpyHostToDevice));
@@ -1121,8 +1133,8 @@ int cafe_gpu_set_families(cafe_gpu_ctx* ctx, int F, int n_leaves, const int* cou
     ctx->fam_max = top;
     ctx->F = F;
     ctx->n_leaves = n_leaves;
+    ctx->buckets.swap(buckets);
     ctx->counts_T.swap(cT);
-    if (ctx->tree_leaves == n_leaves) make_patterns(ctx);
     return CAFE_GPU_OK;
 }
 
@@ -1675,19 +1687,26 @@ int plan_over(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points,
     // the classes that run over subtree patterns: those with units, enough
     // family-likelihoods, on a kernel that reads columns, with their columns
     // within the memory set aside
-    make_patterns(ctx);
+    auto can_share = [&](int key) {
+        const bool f64 = path == CAFE_GPU_PATH_PLAIN64 || path == CAFE_GPU_PATH_BATCHED64 || key > kMfmaMaxTiles;
+        return !root_out && !(f64 && ctx->n_leaves > 512) && !whole.count(key);   // (past 512 the counts are not staged)
+    };
+    std::map<int, long long> key_work;   // of the buckets that are searched
+    for (auto& bc : bucket_class)
+        if (ctx->buckets[bc.second].count >= kPatternFamilies)
+            key_work[bc.first] += (long long)ctx->buckets[bc.second].count * n_points;
+    for (const auto& kw : key_work)
+        if (can_share(kw.first) && kw.second >= kPatternWork) make_patterns(ctx);
     const Patterns& pat = ctx->pat;
     const int nb = (int)ctx->buckets.size();
     int max_point = 0;
     for (int i = 0; i < n_points; ++i) max_point = std::max(max_point, point_ids[i] + 1);
     std::map<int, bool> key_pat;
     size_t pat_bytes = 0;
-    if (!pat.units.empty() && !root_out)
+    if (!pat.units.empty())
         for (const auto& kr : key_rows) {
             const int key = kr.first;
-            const bool f64 = path == CAFE_GPU_PATH_PLAIN64 || path == CAFE_GPU_PATH_BATCHED64 || key > kMfmaMaxTiles;
-            if (f64 && ctx->n_leaves > 512) continue;   // (counts not staged)
-            if (whole.count(key)) continue;
+            if (!can_share(key)) continue;
             long long fams = 0;
             size_t bytes = 0;
             for (auto& bc : bucket_class) {
