@@ -852,7 +852,8 @@ int cafe_gpu_destroy(cafe_gpu_ctx* ctx)
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     DevBuf* bufs[] = {&ctx->lg, &ctx->mt64, &ctx->mt32, &ctx->lf32, &ctx->keys, &ctx->get_rows, &ctx->d_ops,
                       &ctx->d_kids, &ctx->d_steps, &ctx->d_steps_lane, &ctx->d_steps_hot, &ctx->d_steps_level, &ctx->d_op_steps, &ctx->d_counts, &ctx->d_perm, &ctx->d_err64,
-                      &ctx->d_err32, &ctx->mt64e, &ctx->mt32e, &ctx->mt16h, &ctx->mt16l, &ctx->band32};
+                      &ctx->d_err32, &ctx->mt64e, &ctx->mt32e, &ctx->mt16h, &ctx->mt16l, &ctx->band32, &ctx->d_recon,
+                      &ctx->d_recon_scratch};
     for (DevBuf* b : bufs) b->release();
     ctx->eager.release_all();
     ctx->pat.release_all();
