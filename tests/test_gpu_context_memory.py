@@ -4,14 +4,13 @@ import numpy as np
 import pytest
 
 from cafe5_amd import native, workloads as wl
+from device_memory import free_bytes
 from oracle_lib import Oracle
 
 pytestmark = pytest.mark.gpu
 
 
 def test_closed_after_a_reconstruction():
-    import torch
-
     tree = wl.yule_tree(34, 3)
     F, B = 4000, 200
     counts = wl.simulate_families(tree, 1 + np.arange(F) % 9, np.full(tree.n_nodes, 0.003), 2, cap=B)
@@ -27,5 +26,5 @@ def test_closed_after_a_reconstruction():
         eng.matrix_build(*keys.arrays())
         eng.reconstruct(slots, prior, B, B)
         eng.close()
-        free.append(torch.cuda.mem_get_info(0)[0])
+        free.append(free_bytes())
     assert free[0] - free[2] < 32 << 20, free   # a context's rows: 200 MB

@@ -6,17 +6,15 @@ import pytest
 
 from bars import reduced_ok
 from cafe5_amd import native, workloads as wl
+from device_memory import MB, Filled, free_bytes
 from oracle_lib import Oracle
 
 pytestmark = pytest.mark.gpu
-MB = 1 << 20
 LEFT = 128 * MB
 
 
 @pytest.mark.parametrize("path", [native.PATH_PLAIN64, native.PATH_BATCHED32])
 def test_no_room_for_columns(path):
-    import torch
-
     tree = wl.yule_tree(14, 3)
     F, B, P = 6000, 100, 96
     rng = np.random.default_rng(1)
@@ -35,31 +33,17 @@ def test_no_room_for_columns(path):
         e.timings()   # (built)
         return e
 
-    def free():
-        torch.cuda.empty_cache()
-        return torch.cuda.mem_get_info(0)[0]
-
     eng = ready()
-    before = free()
+    before = free_bytes()
     want = eng.evaluate(slots, prior, path)["lnl"].copy()
-    assert before - free() > LEFT + 128 * MB   # most of it columns
+    assert before - free_bytes() > LEFT + 128 * MB   # most of it columns
     eng.close()
     eng = ready()
-    hold = []   # everything but LEFT, in blocks
-    for size in (64 << 30, 8 << 30, 1 << 30, 16 * MB):
-        try:
-            while True:
-                hold.append(torch.empty(size, dtype=torch.uint8, device="cuda:0"))
-        except torch.cuda.OutOfMemoryError:
-            pass
-    assert len(hold) > LEFT // (16 * MB)
-    del hold[-(LEFT // (16 * MB)):]
-    free()
+    rest = Filled(LEFT)
     try:
         got = eng.evaluate(slots, prior, path)["lnl"]
     finally:
-        hold.clear()
-        free()
+        rest.release()
         eng.close()
     if path == native.PATH_PLAIN64:
         assert np.array_equal(got, want)

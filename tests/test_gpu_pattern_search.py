@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from cafe5_amd import native, workloads as wl
+from device_memory import free_bytes
 from oracle_lib import Oracle
 
 pytestmark = pytest.mark.gpu
@@ -22,11 +23,6 @@ def _table():
 
 
 def test_nothing_is_searched_where_nothing_is_shared():
-    import torch
-
-    def free():
-        return torch.cuda.mem_get_info(0)[0]
-
     tree, counts, keys, slots = _table()
     warm = native.Engine(0)   # (kernels loaded)
     warm.set_tree(tree)
@@ -40,15 +36,15 @@ def test_nothing_is_searched_where_nothing_is_shared():
     eng.matrix_reset(B + 1, len(keys.keys))
     eng.matrix_build(*keys.arrays())
     eng.timings()
-    f0 = free()
+    f0 = free_bytes()
     eng.set_families(counts, B, R)
-    f1 = free()
+    f1 = free_bytes()
     # the counts and their order; the search's tables hold the counts again
     # and a row per shared node
     assert f0 - f1 < 1.4 * counts.nbytes, f0 - f1
     eng.root_vectors(slots, prior, native.PATH_PLAIN64)
     # vectors, values and lists of every family: 8 R and about 60 bytes
-    assert f1 - free() < F * (8 * R + 60) + counts.nbytes // 2, f1 - free()
+    assert f1 - free_bytes() < F * (8 * R + 60) + counts.nbytes // 2, f1 - free_bytes()
     warm.close()
     eng.close()
 
