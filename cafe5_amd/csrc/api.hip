@@ -162,7 +162,7 @@ struct EvalBufs {
     DevBuf fb_tiles, fb_count, val, flag, lnl, cat, post, fail, total, scratch, root, fam_list, cols_x, cols_meta;
     // the inputs: put() together on the host, then one block (commit_inputs)
     DevBuf inputs;
-    DevView node_slot, prior64, prior32, catp, buckets, tiles, ntiles, segs, class_off, units;
+    DevView node_slot, prior64, catp, buckets, tiles, ntiles, segs, class_off, units;
     std::vector<char> block;
     std::vector<std::pair<DevView*, size_t>> views;
     std::vector<BucketDev> bucket_h;   // the bucket table (plan_prune adds the programs and units)
@@ -251,8 +251,7 @@ struct cafe_gpu_ctx {
     DevBuf d_recon_scratch;                  // reconstruction: per-family L rows
     char* fixed_scratch = nullptr;           // this device's copy of `scratch` (device address)
     std::vector<OpDev> ops;
-    std::vector<ChildDev> kids;
-    DevBuf d_ops, d_kids, d_steps;
+    DevBuf d_steps;
     int n_steps = 0;
     DevBuf d_steps_lane;     // the same steps with output-reusing slots (split-FP16 kernel)
     int n_slots_lane = 0;
@@ -850,8 +849,8 @@ int cafe_gpu_destroy(cafe_gpu_ctx* ctx)
     if (!ctx) return CAFE_GPU_OK;
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    DevBuf* bufs[] = {&ctx->lg, &ctx->mt64, &ctx->mt32, &ctx->lf32, &ctx->keys, &ctx->get_rows, &ctx->d_ops,
-                      &ctx->d_kids, &ctx->d_steps, &ctx->d_steps_lane, &ctx->d_steps_hot, &ctx->d_steps_level, &ctx->d_op_steps, &ctx->d_counts, &ctx->d_perm, &ctx->d_err64,
+    DevBuf* bufs[] = {&ctx->lg, &ctx->mt64, &ctx->mt32, &ctx->lf32, &ctx->keys, &ctx->get_rows,
+                      &ctx->d_steps, &ctx->d_steps_lane, &ctx->d_steps_hot, &ctx->d_steps_level, &ctx->d_op_steps, &ctx->d_counts, &ctx->d_perm, &ctx->d_err64,
                       &ctx->d_err32, &ctx->mt64e, &ctx->mt32e, &ctx->mt16h, &ctx->mt16l, &ctx->band32, &ctx->d_recon,
                       &ctx->d_recon_scratch};
     for (DevBuf* b : bufs) b->release();
@@ -1031,14 +1030,8 @@ int cafe_gpu_set_tree(cafe_gpu_ctx* ctx, int n_nodes, const int* parent, const i
     for (auto& k : kids) ctx->max_children = std::max(ctx->max_children, (int)k.size());
     ctx->n_slots = pl.max_slot + 1;
     ctx->ops = pl.ops;
-    ctx->kids = pl.out_kids;
-    HIP_OR_FAIL(ctx->d_ops.ensure(sizeof(OpDev) * ctx->ops.size()));
-    HIP_OR_FAIL(ctx->d_kids.ensure(sizeof(ChildDev) * ctx->kids.size()));
-    HIP_OR_FAIL(hipMemcpy(ctx->d_ops.p, ctx->ops.data(), sizeof(OpDev) * ctx->ops.size(), hipMemcpyHostToDevice));
-    HIP_OR_FAIL(hipMemcpy(ctx->d_kids.p, ctx->kids.data(), sizeof(ChildDev) * ctx->kids.size(),
-                          hipMemcpyHostToDevice));
-    // the same program as a flat list of child steps
-    const std::vector<StepDev> steps = flatten_steps(ctx->ops, ctx->kids);
+    // the program as a flat list of child steps
+    const std::vector<StepDev> steps = flatten_steps(pl.ops, pl.out_kids);
     ctx->n_steps = (int)steps.size();
     HIP_OR_FAIL(ctx->d_steps.ensure(sizeof(StepDev) * steps.size()));
     HIP_OR_FAIL(hipMemcpy(ctx->d_steps.p, steps.data(), sizeof(StepDev) * steps.size(), hipMemcpyHostToDevice));
@@ -1578,7 +1571,6 @@ int upload_eval_inputs(cafe_gpu_ctx* ctx, EvalBufs& b, const cafe_gpu_eval_desc*
     }
     const int nb = (int)ctx->buckets.size();
     std::vector<double> pr64((size_t)nb * d->prior_stride, 0.0);
-    std::vector<float> pr32(pr64.size());
     std::vector<BucketDev>& bd = b.bucket_h;
     bd.assign(nb, BucketDev{});
     for (int i = 0; i < nb; ++i) {
@@ -1594,14 +1586,12 @@ int upload_eval_inputs(cafe_gpu_ctx* ctx, EvalBufs& b, const cafe_gpu_eval_desc*
         bd[i].prior_off = i * d->prior_stride;
         bd[i].out = -1;
     }
-    for (size_t i = 0; i < pr64.size(); ++i) pr32[i] = (float)pr64[i];
     std::vector<double> cp(K, 1.0);
     if (d->cat_probs) cp.assign(d->cat_probs, d->cat_probs + K);
     b.block.clear();
     b.views.clear();
     b.put(b.node_slot, slot.data(), sizeof(int) * ns);
     b.put(b.prior64, pr64.data(), sizeof(double) * pr64.size());
-    b.put(b.prior32, pr32.data(), sizeof(float) * pr32.size());
     b.put(b.catp, cp.data(), sizeof(double) * K);
     const size_t PF = (size_t)P * ctx->F;
     HIP_OR_FAIL(b.val.ensure(sizeof(double) * PF));
@@ -1993,9 +1983,6 @@ int plan_over(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points,
 
     PruneParams& p = pp.base;
     p.buckets = b.buckets.as<BucketDev>();
-    p.ops = ctx->d_ops.as<OpDev>();
-    p.n_ops = (int)ctx->ops.size();
-    p.kids = ctx->d_kids.as<ChildDev>();
     p.steps = ctx->d_steps.as<StepDev>();
     p.n_steps = ctx->n_steps;
     p.n_leaves = ctx->n_leaves;
@@ -2015,7 +2002,6 @@ int plan_over(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points,
     p.cm32 = ctx->lf32.as<float>();
     p.n_dev = ctx->n_dev;
     p.prior64 = b.prior64.as<double>();
-    p.prior32 = b.prior32.as<float>();
     p.model = model;
     p.out_val = b.val.as<double>();
     p.out_flag = b.flag.as<int>();

@@ -65,7 +65,7 @@ struct BucketDev {
     int Rp;            // root rows 0..R (size 0 unused) rounded up to 16
     int fam_begin;     // first family (bucket-sorted order)
     int count;
-    int prior_off;     // offset of this bucket's prior in the prior tables
+    int prior_off;     // offset of this bucket's prior in the prior table
     // its program where the launch uses subtree patterns (PruneParams::units)
     int step0, n_steps;   // steps [step0, step0 + n_steps)
     int col0, n_cols;     // columns [col0, col0 + n_cols) its leaf steps read
@@ -143,10 +143,7 @@ struct PruneParams {
     const int* n_tiles_dev;   // number of tiles (device-resident count)
     // model
     const BucketDev* buckets;
-    const OpDev* ops;
-    int n_ops;
-    const ChildDev* kids;
-    const StepDev* steps;     // the same program as child steps
+    const StepDev* steps;     // the evaluation program as child steps
     int n_steps;
     int n_leaves;
     int n_nodes;
@@ -168,7 +165,6 @@ struct PruneParams {
     int n_dev;                // error-model deviations (0: none); folded into leaf64/leaf32
     // root prior per bucket: prior[bucket.prior_off + j]
     const double* prior64;
-    const float* prior32;
     int model;                // CAFE_GPU_MODEL_*
     // outputs [point][F] in the caller's family order
     double* out_val;
