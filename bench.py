@@ -13,7 +13,7 @@ Workload (one "step" = one pass of the hot path over the whole batch):
 
 The headline path is BATCHED32 (FP32 MFMA contractions, per-family rescaling,
 FP64 recompute of families the flush bound cannot certify).  The plain FP64
-drop-in (per-family matrix-vector products) and the batched FP64 MFMA path are
+drop-in and the batched FP64 path (the same kernel in other size classes) are
 timed on the same inputs, the FP32 results are compared with FP64 ones, and the
 compiled reference (oracle/_ref, or the oracle port) is timed on a bounded
 sample on the host cores.
@@ -119,11 +119,11 @@ def time_plan(plan: native.Plan, steps: int, warmup: int, profile_steps: int):
 
 
 def read_traffic(nt: int, kernel: str):
-    """HBM bytes per launch of the FP32 main-pass kernel of the nt-tile size
-    class, from the committed rocprofv3 counter summary (FETCH_SIZE and
-    WRITE_SIZE of that kernel, each scaled by what the counter reads for a
-    device copy of known size); None when the summary does not cover it or
-    was taken on another kernel (name prefix `kernel`)."""
+    """HBM bytes of one FP32 main pass of the nt-tile size class (its launches
+    over shared subtrees and the families' together), from the committed
+    rocprofv3 counter summary (FETCH_SIZE and WRITE_SIZE, each scaled by what
+    the counter reads for a device copy of known size); None when the summary
+    does not cover it or was taken on another kernel (name prefix `kernel`)."""
     path = os.path.join(ROOT, "profiles", "prune_fp32_uneven34_traffic.json")
     if not os.path.exists(path):
         return None
@@ -393,7 +393,7 @@ def _accuracy(runs, test_path, ref_path):
             "max_rel_dlnL_total": float(np.max(tr)),
             "nonfinite_families_match": bool(np.array_equal(np.isfinite(a), fin)),
             "families_recomputed_fp64": int(runs[test_path]["recomputed"][0]),
-            "families_recomputed_plain64": int(runs[test_path]["recomputed"][1])}
+            "families_near_subnormal": int(runs[test_path]["recomputed"][1])}
 
 
 def _class_roofline(run, flops, peak, unit_desc):
@@ -408,10 +408,9 @@ def _class_roofline(run, flops, peak, unit_desc):
                       f"launch of the {int(nt_cls[dom])}-tile size class ({int(tiles_cls[dom])} tiles of "
                       f"{int(dl[5])} families, {int(dl[4])} workgroups)",
             "algorithmic_flops_per_launch": flops, "avg_ms": ms, "flops_per_family_likelihood": unit_desc,
-            "executed": "the FP32 matrix-core kernel multiplies only the k-tiles inside each step's nonzero band "
-                        "(matrix blocks that are exactly 0 in FP32 are skipped), so it executes fewer matrix-core "
-                        "flops than the dense algorithmic count above; the counters under profiles/ give the "
-                        "executed rate"}
+            "executed": "the count above is dense and every family's; equal subtrees of families are computed once "
+                        "and the FP32 matrix-core kernel skips matrix blocks that are exactly 0, so fewer flops are "
+                        "executed (the counters under profiles/ give executed rates)"}
 
 
 def _ref_cpu_base(w, B, R, err, node_lambda_classes, n_sample, threads, gamma=None):
@@ -853,7 +852,7 @@ def main():
         "nonfinite_families_match": same_fin,
         "nonfinite_family_likelihoods": int((~fin).sum()),
         "fp32_families_recomputed_batched64": int(rc64),
-        "families_recomputed_plain64_near_subnormal": int(rcplain),
+        "families_near_subnormal": int(rcplain),
         "batched64_max_rel_dlnL": float(d64.max()) if d64.size else 0.0,
     }
     # the bars the reduced path is held to (the metric's |dlnL| <= 1e-6 is
@@ -886,14 +885,14 @@ def main():
     dl = launch_cls[dom]
     lane_dom = int(dl[0]) == 1
     if lane_dom:
-        dom_kernel = f"void k_prune_lane<{int(dl[1])}, "
+        dom_kernel = f"k_prune_lane<{int(dl[1])}, "
         dom_desc = (f"k_prune_lane<{int(dl[1])},*> (one family per lane, FP32 vector FMAs, no MFMA) main-pass "
                     f"launch of the {dom_nt}-tile size class (buckets B={dom_buckets}, {int(tiles_cls[dom])} tiles "
                     f"of 64 families)")
     else:
-        dom_kernel = f"void k_prune_mfma<float, {int(dl[1])}, {int(dl[2])}, true, {'true' if dl[3] else 'false'}>"
-        dom_desc = (f"k_prune_mfma<float,{int(dl[1])},{int(dl[2])},true,*> main-pass launch of the {dom_nt}-tile "
-                    f"size class (buckets B={dom_buckets}, {int(tiles_cls[dom])} tiles of 16 families)")
+        dom_kernel = (f"k_prune_mfma<{int(dl[1])}, {int(dl[2])}, {'true' if dl[3] else 'false'}, {int(dl[5]) // 16}>")
+        dom_desc = (f"{dom_kernel} main-pass launch of the {dom_nt}-tile size class (buckets B={dom_buckets}, "
+                    f"{int(tiles_cls[dom])} tiles of {int(dl[5])} families)")
     traffic = read_traffic(dom_nt, dom_kernel)
     build_bytes = len(lam_q) * N * N * (8 + 4 + 4)
     roofline = {"bound": "valu" if lane_dom else "mfma", "achieved": achieved / 1e12 if achieved else None,

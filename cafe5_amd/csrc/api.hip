@@ -513,8 +513,11 @@ std::vector<StepDev> flatten_steps(const std::vector<OpDev>& ops, const std::vec
     return steps;
 }
 
-// Buckets of fewer families are not searched for patterns (a few tiles wait for
-// one chain of steps, which more launches only lengthen).
+// Buckets of fewer families are not searched for patterns: at one point a few
+// tiles wait for one chain of steps, which more launches only lengthen.  (Grids
+// of many points would gain little by a lower limit, families of one small bucket
+// having few patterns in common: 483 families at each of 64 points kept 74 to
+// 100% of their contractions at a limit of 16.)
 constexpr int kPatternFamilies = 512;
 // A node is a candidate while its patterns are at most half of the families:
 // one step of 50,000 gamma families 1.49 ms, against 1.52 at a quarter and 1.62
@@ -584,12 +587,12 @@ int pair_patterns(const std::vector<int>& a, int na, const std::vector<int>& b, 
 }
 
 // Finds the units of every bucket, their programs and those of the buckets,
-// and uploads them.  A pass over every node's ids on the host: 5 ms for 10,000
-// families of 34 taxa, 20 for 50,000, 300 for 200,000 of 100 taxa -- about ten
-// evaluations' gain -- so it is left to the first evaluation that can share
-// (root vectors and reconstructions do not), and its result is kept while the
-// same tree and counts are set again, as a model that sets both for every score
-// does.
+// and uploads them.  A pass over every node's ids on the host: 0.8 ms for 10,000
+// families of 34 taxa, 3.9 for 50,000, 87 for 200,000 of 100 taxa (several times
+// that on a slower host) -- what two evaluations and more gain by it -- so it is
+// left to the first evaluation that can share (root vectors and reconstructions
+// do not), and its result is kept while the same tree and counts are set again,
+// as a model that sets both for every score does.
 int find_patterns(cafe_gpu_ctx* ctx)
 {
     Patterns& P = ctx->pat;
@@ -1279,8 +1282,13 @@ MfmaShape mfma_shape(int nt)
 // steps of the tiles each CU holds: one row tile per wave, as many waves as the
 // vector has tiles.  A score of 8,000 families of 34 taxa at B = 100 379 -> 312
 // us, 5,000 at 150 417 -> 381, 2,000 at 200 429 -> 366, 1,000 of 60 taxa at 120 983
-// -> 561; from about 32 families per CU on the wider shapes' fewer loads win
-// (200,000 gamma families: 0.94 ms against 1.25).
+// -> 561.  More families fill the chip and the wider shapes' fewer loads win; the
+// line, 32 families per CU, lies between the sizes where that happens (one step
+// over shared subtrees, this shape against the 32-family tiles taken from there
+// on): 34 taxa at B = 100 8,191 families 161 us against 204, 12,000 202 against 221,
+// 32,000 296 against 290; at 150 5,000 families 254 against 335, 8,000 291 against
+// 310 (275 on 16-family tiles), 12,000 341 against 323; 60 taxa at 120 8,000 246
+// against 292, 16,000 295 against 324; 200,000 gamma families 1.25 ms against 0.94.
 MfmaShape mfma_shape_few(int nt) { return {1, nt <= 4 ? 4 : nt <= 8 ? 8 : 16, false, 0}; }
 
 // FP32 launch shape with 32-family tiles (two blocks of 16 per MFMA operand)
@@ -1839,8 +1847,10 @@ int plan_over(cafe_gpu_ctx* ctx, EvalBufs& b, int path, int model, int n_points,
     // stream.  Estimated cost: contraction work (tiles x nt^2, plus a per-tile
     // overhead) and a floor for the serial chain of one large tile; a
     // per-lane class counts a quarter (it runs unpadded at the full vector
-    // rate beside the matrix-core classes: measured 3.480 -> 3.459 ms per
-    // step on the uneven-size workload against the full count, 3.52 at half).
+    // rate beside the matrix-core classes).  On the uneven-size workload that
+    // was 3.46 ms per step against 3.48 at the full count and 3.52 at half
+    // while every class ran whole programs; over shared subtrees, which
+    // shorten the per-lane classes most, it is 2.75 against 2.66 and 2.69.
     {
         std::vector<double> cost(n_cls);
         std::vector<int> order(n_cls);

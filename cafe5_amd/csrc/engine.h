@@ -117,7 +117,7 @@ struct StepDev {
     int node;       // child node (branch matrix node_slot[point][node])
     int leaf_col;   // >= 0: leaf column; -1: interior child
     int in_slot;    // interior: slot holding its partial vector
-    int ctl;        // out_slot | kStepFirst | kStepLast | kStepRoot
+    int ctl;        // out_slot | kStepFirst | kStepLast | kStepRoot | kStepPattern | kStepOut
 };
 enum : int {
     kStepFirst = 1 << 8,   // first child of its op: the product starts at 1
@@ -236,7 +236,7 @@ struct MfmaShape {
     size_t shm;
     int per_cu;          // workgroups resident on one CU (registers and LDS)
     int grid_mult = 0;   // workgroups per resident slot (0: the planner's default)
-    int fb = 1;          // blocks of 16 families per tile (4: FP64 only)
+    int fb = 1;          // blocks of 16 families per tile (1 or 2)
     bool staged = true;      // FP64: a tile's leaf counts in LDS
 };
 

@@ -40,8 +40,9 @@ constexpr double kTau32 = 1.1754943508222875e-38;
 constexpr double kTwoPowMinusMatExp = 1.0 / (double)(1 << kMatExp);
 // an FP32 likelihood is accepted when the flush bound is below this fraction
 constexpr double kCertEta = 1e-9;
-// below this, FP64 values may lose bits to subnormals; such families are
-// recomputed in the reference's summation order (PLAIN64)
+// below this, FP64 values may lose bits to subnormals: a reduced path's family
+// is recomputed in FP64, and the FP64 kernel counts its own (near_floor; its sums
+// are in the reference's order, so there is nothing to recompute)
 constexpr double kFp64Floor = 1e-290;
 
 // 1/mant rounded up (mant in [0.5, 1)): the FP32 reciprocal is within one

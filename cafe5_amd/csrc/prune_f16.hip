@@ -107,7 +107,7 @@ __device__ __forceinline__ RootBest16 root_combine16(RootBest16 r)
 }
 
 // ---------------------------------------------------------------------------
-// The kernel: the structure of k_prune_mfma<float, ...> (child steps walked
+// The kernel: the structure of k_prune_mfma (child steps walked
 // with the next step's operands prefetched into the other half of a
 // ping-pong buffer; wave wv computes the contiguous run [wv n / W,
 // (wv + 1) n / W) of the n output tiles, and an interior step multiplies the

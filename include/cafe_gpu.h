@@ -285,7 +285,8 @@ int cafe_gpu_plan_destroy(cafe_gpu_plan *plan);
  * to plans with exactly those classes, and is preferred there to an entry
  * without the list, which applies to any plan.  An entry whose
  * shape does not exist or does not fit the class is ignored, and the class
- * keeps its built-in shape. */
+ * keeps its built-in shape (BATCHED64 entries of three and four tiles per wave
+ * are such: its kernel has one and two). */
 /* Replaces the table with the entries of a cache file; *n_loaded (may be
  * NULL) receives their number. */
 int cafe_gpu_tuning_load(cafe_gpu_ctx *ctx, const char *path, int *n_loaded);
